@@ -24,67 +24,30 @@ uint16_t bf16_bits(float f) {  // round to nearest even (finite inputs)
   return (uint16_t)(u >> 16);
 }
 
+// Workspace for a batch of `rows`.  The chain kernel writes all of the transposed workspace that the
+// weight kernel reads, so nothing is kept in it from one batch to the next.
 int ensure_rows(fp_surrogate* s, int rows) {
-  if (rows <= s->rows) return FP_OK;
-  const size_t r = (size_t)rows;
-  HIP_TRY(s->Xb.alloc(r * fp::kFeat));
-  HIP_TRY(s->Tb.alloc(r * 3));
-  HIP_TRY(s->Z1.alloc(r * fp::kHid));
-  HIP_TRY(s->Z2.alloc(r * fp::kHid));
-  HIP_TRY(s->Z3.alloc(r * fp::kHid));
-  HIP_TRY(s->H1.alloc(r * fp::kHid));
-  HIP_TRY(s->H2.alloc(r * fp::kHid));
-  HIP_TRY(s->H3.alloc(r * fp::kHid));
-  HIP_TRY(s->Y.alloc(r * 3));
-  HIP_TRY(s->dY.alloc(r * 3));
-  HIP_TRY(s->dH.alloc(r * fp::kHid));
-  HIP_TRY(s->dZ.alloc(r * fp::kHid));
-  HIP_TRY(s->partial.alloc((r * 3 + fp::kBlock - 1) / fp::kBlock));
-  s->rows = rows;
+  s->pitch = (rows + fp::kTrainTile - 1) / fp::kTrainTile * fp::kTrainTile;
+  HIP_TRY(s->wb.reserve(fp::kParams));
+  HIP_TRY(s->wbt.reserve(2 * fp::kHid * fp::kHid));
+  HIP_TRY(s->part.reserve((size_t)fp::train_slices(s->pitch) * fp::kParams));
+  HIP_TRY(s->loss_part.reserve((size_t)fp::train_groups(s->pitch)));
+  HIP_TRY(s->tr.reserve((size_t)s->pitch * fp::kTrRows));
   return FP_OK;
 }
 
 }  // namespace
 
-int surrogate_fwd_bwd(fp_surrogate* s, int B, int loss_slot) {
+// Forward, error and backward of the batch and its weight-gradient slices; the update kernel then
+// leaves the gradient in s->g, the loss in *loss and, with adam.p set, the updated parameters.
+int surrogate_step(fp_surrogate* s, const __bf16* X, const float* T, uint64_t count, uint64_t seed, int rows, float* Y,
+                   float* loss, const fp::AdamArgs& adam) {
   using namespace fp;
-  hipStream_t st = s->stream;
-  const float* P = s->p.p;
-  float* G = s->g.p;
-  const __bf16* W = s->wb.p;
-  HIP_TRY(launch_to_bf16(P, s->wb.p, kParams, st));
-  // forward: Z_l [B][128] = H_{l-1} W_l^T (+ b_l), H_l = bf16(gelu(Z_l))
-  HIP_TRY(launch_gemm_bf16(B, kHid, kFeat, s->Xb.p, kFeat, 1, W + kOffW1, 1, kFeat, s->Z1.p, kHid, 1, false, st));
-  HIP_TRY(launch_bias_act(s->Z1.p, P + kOffB1, s->H1.p, B, kHid, true, st));
-  HIP_TRY(launch_gemm_bf16(B, kHid, kHid, s->H1.p, kHid, 1, W + kOffW2, 1, kHid, s->Z2.p, kHid, 1, false, st));
-  HIP_TRY(launch_bias_act(s->Z2.p, P + kOffB2, s->H2.p, B, kHid, true, st));
-  HIP_TRY(launch_gemm_bf16(B, kHid, kHid, s->H2.p, kHid, 1, W + kOffW3, 1, kHid, s->Z3.p, kHid, 1, false, st));
-  HIP_TRY(launch_bias_act(s->Z3.p, P + kOffB3, s->H3.p, B, kHid, true, st));
-  HIP_TRY(launch_gemm_bf16(B, kOut, kHid, s->H3.p, kHid, 1, W + kOffW4, 1, kHid, s->Y.p, kOut, 1, false, st));
-  HIP_TRY(launch_mse(s->Y.p, P + kOffB4, s->Tb.p, B, s->dY.p, s->partial.p, st));
-  const int np = (int)((3L * B + kBlock - 1) / kBlock);
-  HIP_TRY(launch_sum(s->partial.p, np, 1.0f / (3.0f * (float)B), s->loss.p + loss_slot, st));
-  // backward
-  // layer 4: dW4 [3][128] = dY^T H3, db4 = sum dY, dH3 [B][128] = dY W4
-  HIP_TRY(launch_gemm_bf16(kOut, kHid, B, s->dY.p, 1, kOut, s->H3.p, kHid, 1, G + kOffW4, kHid, 1, false, st));
-  HIP_TRY(launch_colsum(s->dY.p, B, kOut, G + kOffB4, st));
-  HIP_TRY(launch_gemm_bf16(B, kHid, kOut, s->dY.p, kOut, 1, W + kOffW4, kHid, 1, s->dH.p, kHid, 1, false, st));
-  // layers 3, 2, 1: dZ = bf16(dH * gelu'(Z)), dW = dZ^T H_prev, db = sum dZ, dH_prev = dZ W
-  struct L {
-    const float* Z;
-    const __bf16* Hprev;
-    int kin, offW, offB;
-  } layers[3] = {{s->Z3.p, s->H2.p, kHid, kOffW3, kOffB3},
-                 {s->Z2.p, s->H1.p, kHid, kOffW2, kOffB2},
-                 {s->Z1.p, s->Xb.p, kFeat, kOffW1, kOffB1}};
-  for (int l = 0; l < 3; ++l) {
-    const L& q = layers[l];
-    HIP_TRY(launch_gelu_bwd(s->dH.p, q.Z, s->dZ.p, (long)B * kHid, kHid, st));
-    HIP_TRY(launch_gemm_bf16(kHid, q.kin, B, s->dZ.p, 1, kHid, q.Hprev, q.kin, 1, G + q.offW, q.kin, 1, false, st));
-    HIP_TRY(launch_colsum(s->dZ.p, B, kHid, G + q.offB, st));
-    if (l < 2)
-      HIP_TRY(launch_gemm_bf16(B, kHid, kHid, s->dZ.p, kHid, 1, W + q.offW, kHid, 1, s->dH.p, kHid, 1, false, st));
-  }
+  TrainBatch b{X, T, count, seed, rows, s->pitch, s->p.p, s->wb.p, s->wbt.p, s->tr.p, Y, s->loss_part.p};
+  HIP_TRY(launch_train_chain(b, s->stream));
+  HIP_TRY(launch_train_weights(s->tr.p, s->pitch, s->part.p, s->stream));
+  HIP_TRY(launch_train_update(s->part.p, train_slices(s->pitch), s->g.p, s->loss_part.p, train_groups(s->pitch),
+                              1.0f / (3.0f * (float)rows), loss, adam, s->wb.p, s->wbt.p, s->stream));
   return FP_OK;
 }
 
@@ -178,7 +141,6 @@ int fp_surrogate_new(const fp_surrogate_config* cfg, uint64_t seed, const float*
   HIP_TRY(s->v.alloc(fp::kParams));
   HIP_TRY(hipMemset(s->m.p, 0, sizeof(float) * fp::kParams));
   HIP_TRY(hipMemset(s->v.p, 0, sizeof(float) * fp::kParams));
-  HIP_TRY(s->wb.alloc(fp::kParams));
   HIP_TRY(s->loss.alloc(1));
   *out = s.release();
   return FP_OK;
@@ -213,11 +175,15 @@ int fp_surrogate_grad(fp_surrogate* s, const float* X, const float* T, uint64_t 
   if (rows == 0 || rows > (1u << 20)) return fail(FP_EINVAL, "rows must be in [1, 2^20]");
   const int B = (int)rows;
   if (int e = fph::ensure_rows(s, B)) return e;
-  fph::DBuf<float> xf;
-  HIP_TRY(xf.upload(X, rows * fp::kFeat));
-  HIP_TRY(hipMemcpy(s->Tb.p, T, sizeof(float) * 3 * rows, hipMemcpyHostToDevice));
-  HIP_TRY(fp::launch_to_bf16(xf.p, s->Xb.p, (long)rows * fp::kFeat, s->stream));
-  if (int e = fph::surrogate_fwd_bwd(s, B, 0)) return e;
+  HIP_TRY(s->Xf.reserve(rows * fp::kFeat));
+  HIP_TRY(s->Xb.reserve(rows * fp::kFeat));
+  HIP_TRY(s->Tb.reserve(rows * fp::kOut));
+  HIP_TRY(s->Y.reserve(rows * fp::kOut));
+  HIP_TRY(hipMemcpy(s->Xf.p, X, sizeof(float) * fp::kFeat * rows, hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpy(s->Tb.p, T, sizeof(float) * fp::kOut * rows, hipMemcpyHostToDevice));
+  HIP_TRY(fp::launch_to_bf16(s->Xf.p, s->Xb.p, (long)rows * fp::kFeat, s->stream));
+  HIP_TRY(fp::launch_train_weights_bf16(s->p.p, s->wb.p, s->wbt.p, s->stream));
+  if (int e = fph::surrogate_step(s, s->Xb.p, s->Tb.p, 0, 0, B, s->Y.p, s->loss.p, fp::AdamArgs{})) return e;
   HIP_TRY(hipStreamSynchronize(s->stream));
   if (loss) HIP_TRY(hipMemcpy(loss, s->loss.p, sizeof(float), hipMemcpyDeviceToHost));
   if (grad) HIP_TRY(hipMemcpy(grad, s->g.p, sizeof(float) * fp::kParams, hipMemcpyDeviceToHost));
@@ -276,23 +242,19 @@ int fp_surrogate_train(fp_surrogate* s, uint64_t steps, uint32_t batch, float lr
   if (!(lr > 0.0f)) return fail(FP_EINVAL, "bad learning rate");
   const int B = (int)batch;
   if (int e = fph::ensure_rows(s, B)) return e;
-  fph::DBuf<float> lossv;
-  HIP_TRY(lossv.alloc(steps ? steps : 1));
+  HIP_TRY(s->lossv.reserve(steps ? steps : 1));
+  HIP_TRY(fp::launch_train_weights_bf16(s->p.p, s->wb.p, s->wbt.p, s->stream));
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (uint64_t k = 0; k < steps; ++k) {
     uint64_t h = seed ^ (0x51ed27ull * (k + 1));
-    HIP_TRY(fp::launch_gather_batch(s->X.p, s->T.p, s->count, fph::splitmix(h), B, s->Xb.p, s->Tb.p, s->stream));
-    // loss of this batch goes to lossv[k]
-    std::swap(s->loss.p, lossv.p);
-    const int e = fph::surrogate_fwd_bwd(s, B, (int)k);
-    std::swap(s->loss.p, lossv.p);
-    if (e) return e;
     ++s->adam_t;
     const float c1 = 1.0f - std::pow(b1, (float)s->adam_t), c2 = 1.0f - std::pow(b2, (float)s->adam_t);
-    HIP_TRY(fp::launch_adam(s->p.p, s->g.p, s->m.p, s->v.p, fp::kParams, lr, b1, b2, eps, c1, c2, s->stream));
+    const fp::AdamArgs adam{s->p.p, s->m.p, s->v.p, lr, b1, b2, eps, c1, c2};
+    if (int e = fph::surrogate_step(s, s->X.p, s->T.p, s->count, fph::splitmix(h), B, nullptr, s->lossv.p + k, adam))
+      return e;
   }
   HIP_TRY(hipStreamSynchronize(s->stream));
-  if (losses && steps) HIP_TRY(hipMemcpy(losses, lossv.p, steps * sizeof(float), hipMemcpyDeviceToHost));
+  if (losses && steps) HIP_TRY(hipMemcpy(losses, s->lossv.p, steps * sizeof(float), hipMemcpyDeviceToHost));
   return FP_OK;
 }
 

@@ -92,24 +92,44 @@ hipError_t launch_sur_samples(const StepArgs& a, const CsrView& t, const uint32_
                               uint32_t n, Pos3 next, const SlotEnt* slots, FeatParams fp, float out_scale, bool struts,
                               __bf16* X, float* T, hipStream_t s);
 
-// Training kernels
-// C(m, n) = sum_k A(m, k) B(k, n) (+ C when accumulate), bf16 operands at arbitrary strides, f32 C.
-hipError_t launch_gemm_bf16(int M, int N, int K, const __bf16* A, long sam, long sak, const __bf16* B, long sbk,
-                            long sbn, float* C, long scm, long scn, bool accumulate, hipStream_t s);
-// Z (f32 [rows][n]) += bias; H = bf16(gelu(Z)) (act) or bf16(Z)
-hipError_t launch_bias_act(float* Z, const float* bias, __bf16* H, int rows, int n, bool act, hipStream_t s);
-// dZ = bf16(dH * gelu'(Z))
-hipError_t launch_gelu_bwd(const float* dH, const float* Z, __bf16* dZ, long count, int n, hipStream_t s);
-// db[j] = sum_r dZ[r][j]
-hipError_t launch_colsum(const __bf16* dZ, int rows, int n, float* db, hipStream_t s);
-// Y (f32 [rows][3], pre-bias) += b4; dY = bf16(2 (Y - T) / (3 rows)); per-block squared-error sums
-hipError_t launch_mse(float* Y, const float* b4, const float* T, int rows, __bf16* dY, float* partial, hipStream_t s);
-hipError_t launch_sum(const float* partial, int n, float scale, float* out, hipStream_t s);
-hipError_t launch_adam(float* p, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
-                       float c1, float c2, hipStream_t s);
+// Training (surrogate_train.hip).  One optimiser step is three launches: the chain kernel takes
+// every batch row through the network and back, the weight kernel forms the weight gradients over
+// slices of the batch, the update kernel sums the slices and applies Adam.
+constexpr int kTrainTile = 128;    // workspace rows are padded to this
+constexpr int kTrainSlices = 64;   // most batch slices of the weight gradients
+// Transposed workspace, [row of the operand][batch row], each operand row `pitch` bf16 long: the
+// batch's features (80 rows, 72..79 zero), the hidden activations, what the backward pass sends to
+// each layer's sums, and the output error (16 rows, 3..15 zero).
+constexpr int kTrX = 0, kTrH1 = 80, kTrH2 = kTrH1 + kHid, kTrH3 = kTrH2 + kHid, kTrZ1 = kTrH3 + kHid,
+              kTrZ2 = kTrZ1 + kHid, kTrZ3 = kTrZ2 + kHid, kTrY = kTrZ3 + kHid, kTrRows = kTrY + 16;
+struct TrainBatch {
+  const __bf16* X;  // bf16 rows of 72 and f32 targets of 3
+  const float* T;
+  uint64_t count, seed;  // rows drawn from `count` by a hash of (seed, j); count 0: batch row j is row j
+  int rows, pitch;       // batch rows, and the workspace's row length (a multiple of kTrainTile)
+  const float* P;        // f32 parameters (biases)
+  const __bf16* wb;      // bf16 parameters, and the transposes [in][out] of W2 and W3
+  const __bf16* wbt;
+  __bf16* tr;            // transposed workspace (kTrRows * pitch)
+  float* Y;              // outputs [rows][3], or nullptr
+  float* loss_part;      // squared-error sum of each workgroup
+};
+struct AdamArgs {
+  float *p, *m, *v;  // nullptr p: gradient only
+  float lr, b1, b2, eps, c1, c2;
+};
+inline int train_waves(int pitch) { return pitch <= 64 * 256 ? 4 : 8; }
+inline int train_groups(int pitch) { return pitch / (16 * train_waves(pitch)); }
+inline int train_slices(int pitch) { return pitch / 256 < 1 ? 1 : pitch / 256 > kTrainSlices ? kTrainSlices : pitch / 256; }
+hipError_t launch_train_chain(const TrainBatch& b, hipStream_t s);
+// Weight and bias gradients of each of train_slices(pitch) batch slices: part[slice][kParams].
+hipError_t launch_train_weights(const __bf16* tr, int pitch, float* part, hipStream_t s);
+// g = sum of the slices, *loss = scale * sum of the n_loss partial losses, then Adam and the bf16 copies
+// (a.p != nullptr) of the updated parameters.
+hipError_t launch_train_update(const float* part, int slices, float* g, const float* loss_part, int n_loss,
+                               float scale, float* loss, const AdamArgs& a, __bf16* wb, __bf16* wbt, hipStream_t s);
+// The bf16 copies of the parameters.
+hipError_t launch_train_weights_bf16(const float* p, __bf16* wb, __bf16* wbt, hipStream_t s);
 hipError_t launch_to_bf16(const float* in, __bf16* out, long n, hipStream_t s);
-// rows idx[j] of X (bf16 [.][72]) and T (f32 [.][3]) -> Xb, Tb; idx from a hash of (seed, j) mod count
-hipError_t launch_gather_batch(const __bf16* X, const float* T, uint64_t count, uint64_t seed, int batch, __bf16* Xb,
-                               float* Tb, hipStream_t s);
 
 }  // namespace fp

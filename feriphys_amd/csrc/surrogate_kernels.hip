@@ -1,45 +1,13 @@
 // gfx950 kernels of the learned large-step surrogate: per-vertex features, the fused bf16 MFMA
-// inference kernel, the big-step update, step diagnostics, training-sample generation and the
-// training kernels (bf16 MFMA GEMM, GELU forward/backward, MSE, Adam).
-//
-// MFMA used throughout: v_mfma_f32_16x16x32_bf16.  Operand layout (lane l of a wave, s = 0..7):
-// A[16 x 32]: row l%16, k = (l/16)*8 + s;  B[32 x 16]: column l%16, k = (l/16)*8 + s;
-// C[16 x 16] (4 f32 per lane): rows (l/16)*4 + r, column l%16.
-#include "surrogate.hpp"
+// inference kernel, the big-step update, step diagnostics and training-sample generation (the
+// training kernels are in surrogate_train.hip).
+#include "surrogate_device.hpp"
 
 #pragma clang fp contract(fast)
 
 namespace fp {
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// The network's activation, a GELU without transcendentals: x s(x) with the normal CDF replaced by
-// a C1 piecewise quadratic,
-//   s(x) = clamp(0.5 + x (a - b min(|x|, x*)), 0, 1),  a = 1 / x*,  b = 1 / (2 x*^2),
-// which reaches 1 (and 0) with zero slope at |x| = x*, so act(x) is exactly x for x >= x* and 0 for
-// x <= -x*; x* = 2.46298 minimises max |act(x) - x Phi(x)| (0.0197).  Four VALU operations per
-// element (the two clamps ride on a multiply and an FMA): the activation is what the inference
-// kernel spends most of its vector instructions on.
-constexpr float kXs = 2.4629791631638027f, kA = 0.4060123670374283f, kB = 0.08242302109366773f;
-constexpr float kIXs = (float)(1.0 / 2.4629791631638027), kBX = (float)(0.08242302109366773 * 2.4629791631638027);
-__device__ __forceinline__ float gelu(float x) {
-  const float t = __builtin_amdgcn_fmed3f(fabsf(x) * kIXs, 0.0f, 1.0f);  // min(|x|, x*) / x*
-  const float s = __builtin_amdgcn_fmed3f(fmaf(x, fmaf(-kBX, t, kA), 0.5f), 0.0f, 1.0f);
-  return x * s;
-}
-__device__ __forceinline__ float gelu_grad(float x) {
-  const float t = __builtin_amdgcn_fmed3f(fabsf(x) * kIXs, 0.0f, 1.0f);
-  const float s = __builtin_amdgcn_fmed3f(fmaf(x, fmaf(-kBX, t, kA), 0.5f), 0.0f, 1.0f);
-  const float ds = fabsf(x) < kXs ? fmaf(-2.0f * kB, fabsf(x), kA) : 0.0f;  // s'(x) = a - 2 b |x|
-  return fmaf(x, ds, s);
-}
 
 __device__ __forceinline__ void store_state(const SoA& o, uint32_t i, f3 x, f3 v) {
   o.x[i] = x.x; o.y[i] = x.y; o.z[i] = x.z;
@@ -66,12 +34,6 @@ __device__ __forceinline__ void slot_feat(const SoA& S, f3 p, f3 v, uint32_t sel
   slot_feat_from(p, v, ld3(S.x, S.y, S.z, nb), ld3(S.vx, S.vy, S.vz, nb), has ? e.rest : 1.0f, has, fp, f);
 }
 
-__device__ __forceinline__ uint64_t mix64(uint64_t z) {
-  z += 0x9e3779b97f4a7c15ull;
-  z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
-  z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
-  return z ^ (z >> 31);
-}
 __device__ __forceinline__ float unit_open(uint64_t h) { return ((float)(h >> 40) + 0.5f) * (1.0f / 16777216.0f); }
 
 // ---------------------------------------------------------------------------------------------
@@ -401,148 +363,9 @@ __global__ void __launch_bounds__(kBlock) sur_samples_kernel(StepArgs A, CsrView
   for (int c = 0; c < 3; ++c) Tg[3 * (size_t)j + c] = ok ? t[c] : 0.0f;
 }
 
-// ---------------------------------------------------------------------------------------------
-// Training GEMM: 64 x 64 C tile per 256-thread workgroup (4 waves of 32 x 32 = 2 x 2 MFMA tiles),
-// K in steps of 32 through LDS.  Operands are read at arbitrary strides (the transposes of the
-// backward pass), staged as As[m][k] and Bs[n][k] so every MFMA operand is one 16-byte LDS read.
-__global__ void __launch_bounds__(256) gemm_bf16_kernel(int M, int N, int K, const __bf16* __restrict__ A, long sam,
-                                                        long sak, const __bf16* __restrict__ B, long sbk, long sbn,
-                                                        float* __restrict__ C, long scm, long scn, int accumulate) {
-  __shared__ __attribute__((aligned(16))) __bf16 As[64][40];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[64][40];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  f32x4 acc[2][2];
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const __bf16 zero = (__bf16)0.0f;
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    for (int e = 0; e < 8; ++e) {
-      const int idx = tid + e * 256;
-      int mm, kk;
-      if (sak == 1) { mm = idx >> 5; kk = idx & 31; } else { kk = idx >> 6; mm = idx & 63; }
-      const int gm = m0 + mm, gk = k0 + kk;
-      As[mm][kk] = (gm < M && gk < K) ? A[(long)gm * sam + (long)gk * sak] : zero;
-      int nn;
-      if (sbk == 1) { nn = idx >> 5; kk = idx & 31; } else { kk = idx >> 6; nn = idx & 63; }
-      const int gn = n0 + nn, gk2 = k0 + kk;
-      Bs[nn][kk] = (gn < N && gk2 < K) ? B[(long)gk2 * sbk + (long)gn * sbn] : zero;
-    }
-    __syncthreads();
-    bf16x8 a[2], b[2];
-    for (int i = 0; i < 2; ++i) a[i] = *reinterpret_cast<const bf16x8*>(&As[wm + 16 * i + col][g * 8]);
-    for (int j = 0; j < 2; ++j) b[j] = *reinterpret_cast<const bf16x8*>(&Bs[wn + 16 * j + col][g * 8]);
-    for (int i = 0; i < 2; ++i)
-      for (int j = 0; j < 2; ++j) acc[i][j] = mfma(a[i], b[j], acc[i][j]);
-    __syncthreads();
-  }
-  for (int i = 0; i < 2; ++i)
-    for (int j = 0; j < 2; ++j)
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm + 16 * i + 4 * g + r, nn = n0 + wn + 16 * j + col;
-        if (m < M && nn < N) {
-          float* c = C + (long)m * scm + (long)nn * scn;
-          *c = accumulate ? *c + acc[i][j][r] : acc[i][j][r];
-        }
-      }
-}
-
-__global__ void __launch_bounds__(kBlock) bias_act_kernel(float* __restrict__ Z, const float* __restrict__ bias,
-                                                           __bf16* __restrict__ H, long count, int n, int act) {
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= count) return;
-  const float z = Z[i] + bias[i % n];
-  Z[i] = z;
-  H[i] = (__bf16)(act ? gelu(z) : z);
-}
-
-__global__ void __launch_bounds__(kBlock) gelu_bwd_kernel(const float* __restrict__ dH, const float* __restrict__ Z,
-                                                           __bf16* __restrict__ dZ, long count) {
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (i >= count) return;
-  dZ[i] = (__bf16)(dH[i] * gelu_grad(Z[i]));
-}
-
-__global__ void __launch_bounds__(kBlock) colsum_kernel(const __bf16* __restrict__ dZ, int rows, int n,
-                                                         float* __restrict__ db) {
-  __shared__ float s[kBlock];
-  const int j = blockIdx.x;
-  float acc = 0.0f;
-  for (int r = threadIdx.x; r < rows; r += kBlock) acc += (float)dZ[(long)r * n + j];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) db[j] = s[0];
-}
-
-__global__ void __launch_bounds__(kBlock) mse_kernel(float* __restrict__ Y, const float* __restrict__ b4,
-                                                      const float* __restrict__ T, int rows, __bf16* __restrict__ dY,
-                                                      float* __restrict__ partial) {
-  __shared__ float s[kBlock];
-  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  float e2 = 0.0f;
-  if (i < 3L * rows) {
-    const float y = Y[i] + b4[i % 3];
-    Y[i] = y;
-    const float d = y - T[i];
-    e2 = d * d;
-    dY[i] = (__bf16)(2.0f * d / (3.0f * (float)rows));
-  }
-  s[threadIdx.x] = e2;
-  __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[blockIdx.x] = s[0];
-}
-
-__global__ void __launch_bounds__(kBlock) sum_kernel(const float* __restrict__ partial, int n, float scale,
-                                                      float* __restrict__ out) {
-  __shared__ float s[kBlock];
-  float acc = 0.0f;
-  for (int i = threadIdx.x; i < n; i += kBlock) acc += partial[i];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = s[0] * scale;
-}
-
-__global__ void __launch_bounds__(kBlock) adam_kernel(float* __restrict__ p, const float* __restrict__ g,
-                                                       float* __restrict__ m, float* __restrict__ v, int n, float lr,
-                                                       float b1, float b2, float eps, float c1, float c2) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
 __global__ void __launch_bounds__(kBlock) to_bf16_kernel(const float* __restrict__ in, __bf16* __restrict__ out, long n) {
   const long i = (long)blockIdx.x * kBlock + threadIdx.x;
   if (i < n) out[i] = (__bf16)in[i];
-}
-
-__global__ void __launch_bounds__(kBlock) gather_batch_kernel(const __bf16* __restrict__ X, const float* __restrict__ T,
-                                                               uint64_t count, uint64_t seed, int batch,
-                                                               __bf16* __restrict__ Xb, float* __restrict__ Tb) {
-  const int j = blockIdx.x * kBlock + threadIdx.x;
-  if (j >= batch) return;
-  const uint64_t r = mix64(seed ^ mix64((uint64_t)j)) % count;
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(X + r * kFeat);
-  uint32_t* dst = reinterpret_cast<uint32_t*>(Xb + (uint64_t)j * kFeat);
-  for (int k = 0; k < kFeat / 2; ++k) dst[k] = src[k];
-  for (int c = 0; c < 3; ++c) Tb[3 * (uint64_t)j + c] = T[3 * r + c];
 }
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -617,62 +440,9 @@ hipError_t launch_sur_samples(const StepArgs& a, const CsrView& t, const uint32_
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_bf16(int M, int N, int K, const __bf16* A, long sam, long sak, const __bf16* B, long sbk,
-                            long sbn, float* C, long scm, long scn, bool accumulate, hipStream_t s) {
-  if (M <= 0 || N <= 0) return hipSuccess;
-  hipLaunchKernelGGL(gemm_bf16_kernel, dim3((N + 63) / 64, (M + 63) / 64), dim3(256), 0, s, M, N, K, A, sam, sak, B,
-                     sbk, sbn, C, scm, scn, accumulate ? 1 : 0);
-  return hipGetLastError();
-}
-
-hipError_t launch_bias_act(float* Z, const float* bias, __bf16* H, int rows, int n, bool act, hipStream_t s) {
-  const long count = (long)rows * n;
-  if (count == 0) return hipSuccess;
-  hipLaunchKernelGGL(bias_act_kernel, dim3(blocks_for(count)), dim3(kBlock), 0, s, Z, bias, H, count, n, act ? 1 : 0);
-  return hipGetLastError();
-}
-
-hipError_t launch_gelu_bwd(const float* dH, const float* Z, __bf16* dZ, long count, int n, hipStream_t s) {
-  (void)n;
-  if (count == 0) return hipSuccess;
-  hipLaunchKernelGGL(gelu_bwd_kernel, dim3(blocks_for(count)), dim3(kBlock), 0, s, dH, Z, dZ, count);
-  return hipGetLastError();
-}
-
-hipError_t launch_colsum(const __bf16* dZ, int rows, int n, float* db, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(colsum_kernel, dim3(n), dim3(kBlock), 0, s, dZ, rows, n, db);
-  return hipGetLastError();
-}
-
-hipError_t launch_mse(float* Y, const float* b4, const float* T, int rows, __bf16* dY, float* partial, hipStream_t s) {
-  if (rows == 0) return hipSuccess;
-  hipLaunchKernelGGL(mse_kernel, dim3(blocks_for(3L * rows)), dim3(kBlock), 0, s, Y, b4, T, rows, dY, partial);
-  return hipGetLastError();
-}
-
-hipError_t launch_sum(const float* partial, int n, float scale, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(kBlock), 0, s, partial, n, scale, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_adam(float* p, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
-                       float c1, float c2, hipStream_t s) {
-  hipLaunchKernelGGL(adam_kernel, dim3(blocks_for(n)), dim3(kBlock), 0, s, p, g, m, v, n, lr, b1, b2, eps, c1, c2);
-  return hipGetLastError();
-}
-
 hipError_t launch_to_bf16(const float* in, __bf16* out, long n, hipStream_t s) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks_for(n)), dim3(kBlock), 0, s, in, out, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_gather_batch(const __bf16* X, const float* T, uint64_t count, uint64_t seed, int batch, __bf16* Xb,
-                               float* Tb, hipStream_t s) {
-  if (batch == 0 || count == 0) return hipSuccess;
-  hipLaunchKernelGGL(gather_batch_kernel, dim3(blocks_for(batch)), dim3(kBlock), 0, s, X, T, count, seed, batch, Xb,
-                     Tb);
   return hipGetLastError();
 }
 

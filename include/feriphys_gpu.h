@@ -273,7 +273,7 @@ void fp_sim_free(fp_sim* sim);
  * the explicit integrators of state.rs.  A per-vertex network (72 features -> 3 x 128 GELU -> 3;
  * bf16 weights and activations, f32 accumulation on the matrix cores) stands in for the strut
  * forces over a step of H = ratio * dt.  Its GELU is x * clamp(0.5 + x (a - b min(|x|, x*)), 0, 1),
- * a C1 piecewise quadratic for the normal CDF (surrogate_kernels.hip; within 0.0197 of x Phi(x)).
+ * a C1 piecewise quadratic for the normal CDF (surrogate_device.hpp; within 0.0197 of x Phi(x)).
  * The step:
  *     a  = (gravity + face forces [+ strut forces when base_struts]) / m + out_scale * net(f)
  *     v' = v + H a,   x' = x + H v'
