@@ -32,33 +32,73 @@ FP_HD float rcp_rn(float x) {
   return 1.0f / x;
 }
 
-// sqrt(x), correctly rounded.  On gfx950 for x in [2^-96, FLT_MAX]: the hardware square root
-// (within 1 ulp) and the choice among it and its two neighbours by the sign of the exact
-// residuals x - s' s (the compiler's own correctly rounded sequence without its rescaling of tiny
-// inputs and its zero/infinity fix-up, which that range does not need); checked on every such
-// input against the full sequence (fp_selftest_exact_math).  Other inputs take the full sequence.
+// sqrt(x), correctly rounded.  On gfx950 for x in [2^-96, FLT_MAX]: the hardware reciprocal square
+// root r, g = x r (within 2 ulp) and one Newton step g + (x - g g) r / 2 with the exact residual, one
+// transcendental and four other operations (choosing among the hardware square root and its two
+// neighbours by their residuals took eight); checked on every such input against the full sequence
+// (fp_selftest_exact_math).  Other inputs take the full sequence.
+#ifdef __HIP_DEVICE_COMPILE__
+FP_HD float sqrt_in_range(float x) {
+  const float r = __builtin_amdgcn_rsqf(x), g = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * r, g);
+}
+FP_HD float rcp_in_range(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+#endif
 FP_HD float sqrt_rn(float x) {
 #ifdef __HIP_DEVICE_COMPILE__
-  if (x >= 0x1p-96f && x <= 3.40282347e38f) {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float dn = __uint_as_float(__float_as_uint(s) - 1u), up = __uint_as_float(__float_as_uint(s) + 1u);
-    const float rdn = __builtin_fmaf(-dn, s, x), rup = __builtin_fmaf(-up, s, x);
-    const float t = rdn <= 0.0f ? dn : s;
-    return rup > 0.0f ? up : t;
-  }
+  if (x >= 0x1p-96f && x <= 3.40282347e38f) return sqrt_in_range(x);
 #endif
   return __builtin_sqrtf(x);
+}
+
+// sqrt(x) and 1 / sqrt(x), each correctly rounded (the reciprocal of the rounded root): one range
+// test for both.
+FP_HD void sqrt_rcp_rn(float x, float& root, float& inv) {
+#ifdef __HIP_DEVICE_COMPILE__
+  if (x >= 0x1p-96f && x <= 0x1p96f) {
+    root = sqrt_in_range(x);
+    inv = rcp_in_range(root);
+    return;
+  }
+#endif
+  root = __builtin_sqrtf(x);
+  inv = 1.0f / root;
+}
+
+// a / b, correctly rounded, given y = RN(1 / b): q = a y and one correction by the exact residual
+// a - b q.  For all 2^46 pairs of significands this equals the division (checked exhaustively on
+// gfx950), so it holds wherever nothing under- or overflows and a != 0: callers keep |a| and |b|
+// within [2^-60, 2^60].  Five operations where the compiler's division sequence takes about ten.
+FP_HD float div_by_rcp(float a, float b, float y) {
+  const float q = a * y;
+  return __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+}
+FP_HD bool div_range(float x) {
+  const float ax = __builtin_fabsf(x);
+  return ax >= 0x1p-60f && ax <= 0x1p60f;
+}
+FP_HD float div_rn(float a, float b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  if (div_range(a) && div_range(b)) return div_by_rcp(a, b, rcp_in_range(b));
+#endif
+  return a / b;
 }
 
 // x / PI (PI = std::f32::consts::PI = 0x40490fdb), correctly rounded: for x >= 2^-100 the product
 // with RN(1/PI) corrected once by the exact remainder fma(-q0, PI, x) (the same method as div3_rn;
 // below 2^-104 the remainder is no longer exact), otherwise (tiny, zero, negative, NaN) the
 // division itself.
-FP_HD float div_pi_rn(float x) {
+FP_HD float div_pi_in_range(float x) {
   const float pi = 3.14159274101257324f, inv_pi = 0.31830987334251404f;  // 0x40490fdb, RN(1/PI) = 0x3ea2f983
-  if (!(x >= 0x1p-100f)) return x / pi;
   const float q0 = x * inv_pi;
   return __builtin_fmaf(__builtin_fmaf(-q0, pi, x), inv_pi, q0);
+}
+FP_HD float div_pi_rn(float x) {
+  if (!(x >= 0x1p-100f)) return x / 3.14159274101257324f;
+  return div_pi_in_range(x);
 }
 
 }  // namespace fp

@@ -124,6 +124,41 @@ FP_HD float fdlibm_atan2f_ref(float y, float x) {
   return (z - pi_lo) - pi;
 }
 
+// atan(t) of t in [2^-29, 2^25) as fdlibm rounds it, without its branches (see fdlibm_atan2f): the
+// reduced argument's numerator and denominator by interval, and the rest from their quotient u.
+// A t is exact (A is 0, 1 or 2), so its difference with B is one fused operation.
+struct FdlReduced {
+  float num, den, hi, lo;
+};
+FP_HD FdlReduced fdl_reduce(float t) {
+  const uint32_t it = fdl_bits(t);
+  const bool c0 = it >= 0x3ee00000u, c1 = it >= 0x3f300000u, c2 = it >= 0x3f980000u, c3 = it >= 0x401c0000u;
+  const float A = c3 ? 0.0f : (c0 && !c1) ? 2.0f : 1.0f;
+  const float B = !c0 ? 0.0f : (c2 && !c3) ? 1.5f : 1.0f;
+  const float hi = !c0   ? 0.0f
+                   : !c1 ? fdl_from_bits(0x3eed6338u)
+                   : !c2 ? fdl_from_bits(0x3f490fdau)
+                   : !c3 ? fdl_from_bits(0x3f7b985eu)
+                         : fdl_from_bits(0x3fc90fdau);
+  const float lo = !c0   ? 0.0f
+                   : !c1 ? fdl_from_bits(0x31ac376au)
+                   : !c2 ? fdl_from_bits(0x33222169u)
+                   : !c3 ? fdl_from_bits(0x33140fb5u)
+                         : fdl_from_bits(0x33a22169u);
+  return FdlReduced{__builtin_fmaf(t, A, -B), A + t * B, hi, lo};
+}
+FP_HD float fdl_atan_from(const FdlReduced& q, float u) {
+  const float a0 = fdl_from_bits(0x3eaaaaabu), a1 = fdl_from_bits(0xbe4ccccdu), a2 = fdl_from_bits(0x3e124925u),
+              a3 = fdl_from_bits(0xbde38e38u), a4 = fdl_from_bits(0x3dba2e6eu), a5 = fdl_from_bits(0xbd9d8795u),
+              a6 = fdl_from_bits(0x3d886b35u), a7 = fdl_from_bits(0xbd6ef16bu), a8 = fdl_from_bits(0x3d4bda59u),
+              a9 = fdl_from_bits(0xbd15a221u), a10 = fdl_from_bits(0x3c8569d7u);
+  const float z = u * u;
+  const float w = z * z;
+  const float s1 = z * (a0 + w * (a2 + w * (a4 + w * (a6 + w * (a8 + w * a10)))));
+  const float s2 = w * (a1 + w * (a3 + w * (a5 + w * (a7 + w * a9))));
+  return q.hi - ((u * (s1 + s2) - q.lo) - u);
+}
+
 // fdlibm_atan2f_ref without data-dependent branches, for finite non-zero y and x (other inputs take
 // the reference path).  Why each fdlibm branch can go:
 //   x == 1 calls atanf(y) directly: the general path computes atanf(|y / 1|) and the same sign;
@@ -139,29 +174,8 @@ FP_HD float fdlibm_atan2f(float y, float x) {
   const float pi = fdl_from_bits(0x40490fdbu), pi_lo = fdl_from_bits(0xb3bbbd2eu);
   const float t = fdl_abs(y / x);
   const uint32_t it = fdl_bits(t);
-  const bool c0 = it >= 0x3ee00000u, c1 = it >= 0x3f300000u, c2 = it >= 0x3f980000u, c3 = it >= 0x401c0000u;
-  const float A = c3 ? 0.0f : (c0 && !c1) ? 2.0f : 1.0f;
-  const float B = !c0 ? 0.0f : (c2 && !c3) ? 1.5f : 1.0f;
-  const float hi = !c0   ? 0.0f
-                   : !c1 ? fdl_from_bits(0x3eed6338u)
-                   : !c2 ? fdl_from_bits(0x3f490fdau)
-                   : !c3 ? fdl_from_bits(0x3f7b985eu)
-                         : fdl_from_bits(0x3fc90fdau);
-  const float lo = !c0   ? 0.0f
-                   : !c1 ? fdl_from_bits(0x31ac376au)
-                   : !c2 ? fdl_from_bits(0x33222169u)
-                   : !c3 ? fdl_from_bits(0x33140fb5u)
-                         : fdl_from_bits(0x33a22169u);
-  const float u = (t * A - B) / (A + t * B);
-  const float a0 = fdl_from_bits(0x3eaaaaabu), a1 = fdl_from_bits(0xbe4ccccdu), a2 = fdl_from_bits(0x3e124925u),
-              a3 = fdl_from_bits(0xbde38e38u), a4 = fdl_from_bits(0x3dba2e6eu), a5 = fdl_from_bits(0xbd9d8795u),
-              a6 = fdl_from_bits(0x3d886b35u), a7 = fdl_from_bits(0xbd6ef16bu), a8 = fdl_from_bits(0x3d4bda59u),
-              a9 = fdl_from_bits(0xbd15a221u), a10 = fdl_from_bits(0x3c8569d7u);
-  const float z = u * u;
-  const float w = z * z;
-  const float s1 = z * (a0 + w * (a2 + w * (a4 + w * (a6 + w * (a8 + w * a10)))));
-  const float s2 = w * (a1 + w * (a3 + w * (a5 + w * (a7 + w * a9))));
-  float r = hi - ((u * (s1 + s2) - lo) - u);
+  const FdlReduced q0 = fdl_reduce(t);
+  float r = fdl_atan_from(q0, q0.num / q0.den);
   r = it < 0x31000000u ? t : r;                                // |t| < 2^-29: atan(t) = t
   r = it >= 0x4c000000u ? fdl_from_bits(0x3fc90fdbu) : r;      // t >= 2^25: atanhi[3] + atanlo[3]
   const bool yneg = fdl_bits(y) >> 31, xneg = fdl_bits(x) >> 31;

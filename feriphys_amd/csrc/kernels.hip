@@ -433,25 +433,33 @@ hipError_t launch_csr(const StepArgs& a, const CsrView& t, const BlockRange* blo
 }
 
 // Every finite f32 x (grid-stride over all bit patterns): the exact kernels' shortened forms
-// against the operations they stand for, bad[0] rcp_rn(x) vs 1 / x, bad[1] div_pi_rn(x) vs x / PI,
-// bad[2] div3_rn(x) vs x / 3, bad[3] the branch-free atan2 vs fdlibm's control flow at y = 1 and
-// y = -1.7, bad[4] sqrt_rn(x) vs the compiler's correctly rounded sqrt (NaN payloads aside).
+// against the operations they stand for, bad[0] rcp_rn(x) vs 1 / x and div_rn with x as divisor and
+// as dividend, bad[1] div_pi_rn(x) vs x / PI, bad[2] div3_rn(x) vs x / 3, bad[3] the branch-free
+// atan2 vs fdlibm's control flow at y = 1 and y = -1.7, and the corner weight's in-range form vs
+// the same, bad[4] sqrt_rn(x) and sqrt_rcp_rn(x) vs the compiler's correctly rounded sqrt and the
+// division (NaN payloads aside).
 __global__ void __launch_bounds__(kBlock) selftest_kernel(unsigned long long* __restrict__ bad) {
   unsigned long long b[5] = {0, 0, 0, 0, 0};
   auto bits = [](float f) { return __float_as_uint(f); };
+  auto differ = [&](float p, float q) { return bits(p) != bits(q) && !(__builtin_isnan(p) && __builtin_isnan(q)); };
+  const float pi = 3.14159274101257324f;
   for (uint64_t k = (uint64_t)blockIdx.x * kBlock + threadIdx.x; k < (1ull << 32); k += (uint64_t)gridDim.x * kBlock) {
     const float x = __uint_as_float((uint32_t)k);
     if (!__builtin_isfinite(x)) continue;
     b[0] += bits(rcp_rn(x)) != bits(1.0f / x);
-    b[1] += bits(div_pi_rn(x)) != bits(x / 3.14159274101257324f);
+    b[0] += differ(div_rn(1.7f, x), 1.7f / x) || differ(div_rn(x, -0.3f), x / -0.3f);
+    b[1] += bits(div_pi_rn(x)) != bits(x / pi);
     b[2] += bits(div3_rn(x)) != bits(x / 3.0f);
     const float ys[2] = {1.0f, -1.7f};
-    for (int j = 0; j < 2; ++j) {
-      const float a = fdlibm_atan2f(ys[j], x), r = fdlibm_atan2f_ref(ys[j], x);
-      b[3] += bits(a) != bits(r) && !(__builtin_isnan(a) && __builtin_isnan(r));
-    }
-    const float sq = sqrt_rn(x), sr = __builtin_sqrtf(x);
-    b[4] += bits(sq) != bits(sr) && !(__builtin_isnan(sq) && __builtin_isnan(sr));
+    for (int j = 0; j < 2; ++j) b[3] += differ(fdlibm_atan2f(ys[j], x), fdlibm_atan2f_ref(ys[j], x));
+    float w;
+    if (ExactMath::corner_in_range(1.0f, x, w)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
+    if (x >= 0.0f && ExactMath::corner_in_range(x, -0.37f, w))
+      b[3] += differ(w, fdlibm_atan2f_ref(__builtin_sqrtf(x), -0.37f) / pi);
+    const float sr = __builtin_sqrtf(x);
+    float root, inv;
+    sqrt_rcp_rn(x, root, inv);
+    b[4] += differ(sqrt_rn(x), sr) || differ(root, sr) || differ(inv, 1.0f / sr);
   }
   for (int q = 0; q < 5; ++q)
     if (b[q]) atomicAdd(&bad[q], b[q]);

@@ -100,8 +100,13 @@ __device__ __forceinline__ void strut_accumulate(f3& F, f3 p_self, f3 v_self, f3
   f3 d = sub(p_nbr, p_self);
   // |d| - rest cancels to the strain, so |d| is always formed exactly (unfused dot, IEEE sqrt):
   // one ulp of |d| is k * ulp(L), already ~5e-5 of a typical strut force.
-  float len = sqrt_rn(dot(d, d));
-  float inv = M::rcp(len);
+  float len, inv;
+  if constexpr (M::kExact) {
+    M::sqrt_rcp(dot(d, d), len, inv);
+  } else {
+    len = sqrt_rn(dot(d, d));
+    inv = M::rcp(len);
+  }
   f3 u = f3{d.x * inv, d.y * inv, d.z * inv};
   float s = k * (len - rest);
   F = add(F, f3{s * u.x, s * u.y, s * u.z});
@@ -112,7 +117,7 @@ __device__ __forceinline__ void strut_accumulate(f3& F, f3 p_self, f3 v_self, f3
 // Drag + lift on one face (springy_mesh.rs:631-646); the weighted share for corner `corner` is
 // (angle / PI) * this (:647-652).
 template <class M>
-__device__ __forceinline__ f3 face_force(f3 p0, f3 p1, f3 p2, f3 u0, f3 u1, f3 u2, const StepParams& P) {
+FP_HD f3 face_force(f3 p0, f3 p1, f3 p2, f3 u0, f3 u1, f3 u2, const StepParams& P) {
   // (v0 + v1 + v2) / 3.0 (springy_mesh.rs:634); div3_rn is that division, correctly rounded
   f3 avg;
   if constexpr (M::kExact)
@@ -122,9 +127,9 @@ __device__ __forceinline__ f3 face_force(f3 p0, f3 p1, f3 p2, f3 u0, f3 u1, f3 u
              ((u0.z + u1.z) + u2.z) * (1.0f / 3.0f)};
   f3 rv = sub(avg, P.wind);
   f3 cr = cross(sub(p1, p0), sub(p2, p0));
-  float cm = M::sqrt_(M::dot(cr, cr));
+  float cm, inv;
+  M::sqrt_rcp(M::dot(cr, cr), cm, inv);
   float area = cm / 2.0f;
-  float inv = M::rcp(cm);
   f3 n = f3{cr.x * inv, cr.y * inv, cr.z * inv};
   float eff = area * fabsf(M::dot(n, rv));
   float sd = P.neg_drag * eff;
@@ -139,13 +144,15 @@ __device__ __forceinline__ f3 face_force(f3 p0, f3 p1, f3 p2, f3 u0, f3 u1, f3 u
 // Face::vertex_angle (springy_mesh.rs:163-172): angle between (p_b - p_a) and (p_c - p_a) at p_a,
 // called as (p2 - p0).angle(p1 - p0) for corner 0 etc.; returns angle / PI.
 template <class M>
-__device__ __forceinline__ float corner_weight(f3 pa, f3 pnext, f3 pprev) {
+FP_HD float corner_weight(f3 pa, f3 pnext, f3 pprev) {
   // vertex_angle(v0, v1, v2) = (p[v2] - p[v0]).angle(p[v1] - p[v0]); angle = atan2(|a x b|, a.b)
   f3 a = sub(pprev, pa);
   f3 b = sub(pnext, pa);
   f3 axb = cross(a, b);
-  float th = M::atan2_(M::sqrt_(M::dot(axb, axb)), M::dot(a, b));
-  return M::div_pi(th);  // Rad / Rad(PI), PI = std::f32::consts::PI
+  const float n2 = M::dot(axb, axb), d = M::dot(a, b);
+  float w;
+  if (M::corner_in_range(n2, d, w)) return w;
+  return M::div_pi(M::atan2_(M::sqrt_(n2), d));  // Rad / Rad(PI), PI = std::f32::consts::PI
 }
 
 // Forces of one torsional hinge (springy_mesh.rs:555-610, the reference's operation order): hinge
@@ -179,8 +186,8 @@ __device__ __forceinline__ void hinge_forces(f3 x0, f3 x1, f3 x2, f3 x3, f3 v2, 
 // with the force frozen over the step (its derivative entries are 0).  RK4 expands to the stage
 // values below; each line is the reference's vec_add/scale of that record component.
 template <class M>
-__device__ __forceinline__ void integrate(const StepParams& P, float m, f3 x, f3 v, f3 F, f3& xn, f3& vn) {
-  f3 a1 = f3{M::div(F.x, m), M::div(F.y, m), M::div(F.z, m)};
+FP_HD void integrate(const StepParams& P, float m, f3 x, f3 v, f3 F, f3& xn, f3& vn) {
+  const f3 a1 = M::div3(F, m);
   if (P.integration == FP_EULER) {  // S + S' * h  (state.rs:75-83)
     xn = f3{x.x + v.x * P.dt, x.y + v.y * P.dt, x.z + v.z * P.dt};
     vn = f3{v.x + a1.x * P.dt, v.y + a1.y * P.dt, v.z + a1.z * P.dt};
@@ -188,7 +195,7 @@ __device__ __forceinline__ void integrate(const StepParams& P, float m, f3 x, f3
   }
   // Stages 2-4 see the force record F + 0 (the force slot's derivative is 0), which differs from F
   // only for F = -0: then (F + 0) / m = +0 / m, otherwise it is a1.
-  const float z0 = M::div(0.0f, m);
+  const float z0 = m > 0.0f ? 0.0f : M::div(0.0f, m);
   f3 a2 = f3{F.x == 0.0f ? z0 : a1.x, F.y == 0.0f ? z0 : a1.y, F.z == 0.0f ? z0 : a1.z};
   const float hh = P.dt_half, h = P.dt, h6 = P.dt6, h3 = P.dt3;
   f3 v2 = f3{v.x + a1.x * hh, v.y + a1.y * hh, v.z + a1.z * hh};
