@@ -147,6 +147,16 @@ FP_HD FdlReduced fdl_reduce(float t) {
                          : fdl_from_bits(0x33a22169u);
   return FdlReduced{__builtin_fmaf(t, A, -B), A + t * B, hi, lo};
 }
+// The same by table: the interval bounds 7/16, 11/16, 19/16, 39/16 are sixteenths, so floor(16 t), at
+// most 39, names the interval; entry j holds (A, B, hi, lo).
+constexpr int kFdlEntries = 40;
+FP_HD void fdl_entry(int j, float q[4]) {
+  const int k = j >= 39 ? 4 : j >= 19 ? 3 : j >= 11 ? 2 : j >= 7 ? 1 : 0;
+  q[0] = k == 4 ? 0.0f : k == 1 ? 2.0f : 1.0f;
+  q[1] = k == 0 ? 0.0f : k == 3 ? 1.5f : 1.0f;
+  q[2] = fdl_from_bits(k == 0 ? 0u : k == 1 ? 0x3eed6338u : k == 2 ? 0x3f490fdau : k == 3 ? 0x3f7b985eu : 0x3fc90fdau);
+  q[3] = fdl_from_bits(k == 0 ? 0u : k == 1 ? 0x31ac376au : k == 2 ? 0x33222169u : k == 3 ? 0x33140fb5u : 0x33a22169u);
+}
 FP_HD float fdl_atan_from(const FdlReduced& q, float u) {
   const float a0 = fdl_from_bits(0x3eaaaaabu), a1 = fdl_from_bits(0xbe4ccccdu), a2 = fdl_from_bits(0x3e124925u),
               a3 = fdl_from_bits(0xbde38e38u), a4 = fdl_from_bits(0x3dba2e6eu), a5 = fdl_from_bits(0xbd9d8795u),

@@ -443,6 +443,9 @@ __global__ void __launch_bounds__(kBlock) selftest_kernel(unsigned long long* __
   auto bits = [](float f) { return __float_as_uint(f); };
   auto differ = [&](float p, float q) { return bits(p) != bits(q) && !(__builtin_isnan(p) && __builtin_isnan(q)); };
   const float pi = 3.14159274101257324f;
+  __shared__ alignas(16) float tab[kFdlEntries][4];
+  if (threadIdx.x < kFdlEntries) fdl_entry((int)threadIdx.x, tab[threadIdx.x]);
+  __syncthreads();
   for (uint64_t k = (uint64_t)blockIdx.x * kBlock + threadIdx.x; k < (1ull << 32); k += (uint64_t)gridDim.x * kBlock) {
     const float x = __uint_as_float((uint32_t)k);
     if (!__builtin_isfinite(x)) continue;
@@ -453,6 +456,7 @@ __global__ void __launch_bounds__(kBlock) selftest_kernel(unsigned long long* __
     const float ys[2] = {1.0f, -1.7f};
     for (int j = 0; j < 2; ++j) b[3] += differ(fdlibm_atan2f(ys[j], x), fdlibm_atan2f_ref(ys[j], x));
     float w;
+    if (ExactMath::corner_in_range(1.0f, x, w, tab)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
     if (ExactMath::corner_in_range(1.0f, x, w)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
     if (x >= 0.0f && ExactMath::corner_in_range(x, -0.37f, w))
       b[3] += differ(w, fdlibm_atan2f_ref(__builtin_sqrtf(x), -0.37f) / pi);

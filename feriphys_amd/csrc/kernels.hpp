@@ -120,9 +120,11 @@ struct TileRange {
 // Tile shapes compiled for the tiled grid kernel (rows x columns per 256-thread workgroup).  A
 // TR x TC tile touches (TR+1) x (TC+1) quads; 15x15 and 7x31 make that exactly 256, one quad (two
 // faces) per thread in the face phase.
-enum TileShape { TILE_15x15 = 0, TILE_7x31 = 1, TILE_16x16 = 2, N_TILE_SHAPES = 3 };
-constexpr int kTileRows[N_TILE_SHAPES] = {15, 7, 16};
-constexpr int kTileCols[N_TILE_SHAPES] = {15, 31, 16};
+// TILE_8x8 is not a caller's choice: the exact kernel takes it for simulations of few tiles (see
+// build_block_lists).
+enum TileShape { TILE_15x15 = 0, TILE_7x31 = 1, TILE_16x16 = 2, N_TILE_SHAPES = 3, TILE_8x8 = 3, N_LAUNCH_SHAPES = 4 };
+constexpr int kTileRows[N_LAUNCH_SHAPES] = {15, 7, 16, 8};
+constexpr int kTileCols[N_LAUNCH_SHAPES] = {15, 31, 16, 8};
 
 hipError_t launch_csr(const StepArgs& a, const CsrView& t, const BlockRange* blocks, uint32_t n_blocks, int mode,
                       bool exact, hipStream_t s);
@@ -150,9 +152,10 @@ hipError_t launch_torsion_gather(const StepArgs& a, const CsrView& t, const Bloc
                                  hipStream_t s);
 hipError_t launch_grid(const StepArgs& a, const ClothView* cloths, const BlockRange* blocks, uint32_t n_blocks,
                        int mode, bool exact, hipStream_t s);
-// LDS-tiled grid kernel over `n_tiles` tiles that all have tile shape `shape`.
+// LDS-tiled grid kernel over `n_tiles` tiles that all have launch shape `shape`: the exact step or
+// forces, or the surrogate's big step (fast arithmetic).
 hipError_t launch_grid_tiled(const StepArgs& a, const ClothView* cloths, const TileRange* tiles, uint32_t n_tiles,
-                             int shape, int mode, bool exact, hipStream_t s);
+                             int shape, int mode, hipStream_t s);
 // SpringyMesh::update_points on device: old state = a.in (+ force records, masses), new = `nw_rec`
 // (10-float Stateful records, indexed by global vertex id); the result is written in place into
 // a.in, the force records and the masses.

@@ -231,6 +231,10 @@ int upload_obstacles(ObstacleSet& s, const std::vector<fp::HostObstacle>& obstac
         }
       }
   }
+  for (int k = 0; k < 3; ++k) {
+    O.box_lo[k] = s.hit_box.lo[k];
+    O.box_hi[k] = s.hit_box.hi[k];
+  }
   return FP_OK;
 }
 

@@ -196,6 +196,16 @@ void cloth_tiles(uint32_t mesh, const fp::ClothDesc& d, int shape, std::vector<f
     for (uint32_t c = 0; c < d.cols; c += tc) out.push_back(fp::TileRange{mesh, r, c, (uint32_t)shape});
 }
 
+uint64_t tile_count(const fp::ClothDesc& d, int shape) {
+  const uint64_t tr = (uint64_t)fp::kTileRows[shape], tc = (uint64_t)fp::kTileCols[shape];
+  return ((d.rows + tr - 1) / tr) * ((d.cols + tc - 1) / tc);
+}
+// Most 8x8 tiles that the exact kernel takes in place of the requested shapes: three to a CU.  Up to
+// there a step is one tile's chain of dependent work and the twelve-wave form is the faster (5.1 us
+// against 9.0 up to 128 x 128 vertices, 256 tiles; 8.1 against 9.4 at 192 x 192, 576 tiles); at 256 x
+// 256, 1,024 tiles, both take 9.6, and beyond it the larger tiles' fewer operations win.
+constexpr uint64_t kSmallTiles = 768;
+
 // Runs of the tile list per XCD (see xcd_order).
 constexpr size_t kTilePieces = 8;
 
@@ -233,7 +243,11 @@ int build_block_lists(fp_sim* s) {
   if (sig == s->lists_sig) return FP_OK;
   std::vector<fp::BlockRange> g, c, cf, sb, sf;
   std::vector<fp::PatchRange> pl;
-  std::vector<fp::TileRange> by_shape[fp::N_TILE_SHAPES], all_tiles;
+  std::vector<fp::TileRange> by_shape[fp::N_LAUNCH_SHAPES], all_tiles;
+  uint64_t n_small = 0;  // 8x8 tiles of all the cloths
+  for (const auto& m : s->meshes)
+    if (m.host.cloth.valid && m.uniform_mass) n_small += tile_count(m.host.cloth, fp::TILE_8x8);
+  const bool small = s->math == FP_MATH_EXACT && n_small <= kSmallTiles;
   for (uint32_t mi = 0; mi < s->meshes.size(); ++mi) {
     MeshSlot& ms = s->meshes[mi];
     const bool grid_ok = ms.host.cloth.valid && ms.uniform_mass;
@@ -244,7 +258,8 @@ int build_block_lists(fp_sim* s) {
     ms.on_patch = false;
     if (ms.kernel == MK_GRID_TILED) {
       // the fast kernel has one quad per thread: 15x15 and 7x31 tiles (16x16 becomes 15x15)
-      ms.launch_shape = s->math == FP_MATH_FAST && ms.tile_shape == fp::TILE_16x16 ? fp::TILE_15x15 : ms.tile_shape;
+      ms.launch_shape = small ? fp::TILE_8x8
+                        : s->math == FP_MATH_FAST && ms.tile_shape == fp::TILE_16x16 ? fp::TILE_15x15 : ms.tile_shape;
       std::vector<fp::TileRange> mt;
       cloth_tiles(mi, ms.host.cloth, ms.launch_shape, mt);
       by_shape[ms.launch_shape].insert(by_shape[ms.launch_shape].end(), mt.begin(), mt.end());
@@ -287,7 +302,7 @@ int build_block_lists(fp_sim* s) {
   s->n_csr_blocks = (uint32_t)c.size();
   HIP_TRY(s->grid_blocks.upload(g.data(), g.size()));
   HIP_TRY(s->csr_blocks.upload(c.data(), c.size()));
-  for (int sh = 0; sh < fp::N_TILE_SHAPES; ++sh) {
+  for (int sh = 0; sh < fp::N_LAUNCH_SHAPES; ++sh) {
     std::vector<fp::TileRange> o = xcd_order(by_shape[sh], kTilePieces);
     s->n_tiles[sh] = (uint32_t)o.size();
     HIP_TRY(s->tiles[sh].upload(o.data(), o.size()));
@@ -315,14 +330,14 @@ int check_sim_mesh(const fp_sim* s, uint64_t mesh) {
 hipError_t tiled_launch(fp_sim* s, const fp::StepArgs& a, const fp::TileRange* tiles, uint32_t n, int shape, int mode) {
   if (s->math == FP_MATH_FAST && shape != fp::TILE_16x16)
     return fp::launch_grid_fast(a, s->cloths.p, tiles, n, shape, mode, s->obst.hit_box, s->stream);
-  return fp::launch_grid_tiled(a, s->cloths.p, tiles, n, shape, mode, s->math == FP_MATH_EXACT, s->stream);
+  return fp::launch_grid_tiled(a, s->cloths.p, tiles, n, shape, mode, s->stream);
 }
 
 int run_steps(fp_sim* s, uint64_t n) {
   for (uint64_t k = 0; k < n; ++k) {
     fp::StepArgs a = s->args(s->forces_dirty);
     bool exact = s->math == FP_MATH_EXACT;
-    for (int sh = 0; sh < fp::N_TILE_SHAPES; ++sh)
+    for (int sh = 0; sh < fp::N_LAUNCH_SHAPES; ++sh)
       HIP_TRY(tiled_launch(s, a, s->tiles[sh].p, s->n_tiles[sh], sh, fp::MODE_STEP));
     HIP_TRY(fp::launch_grid(a, s->cloths.p, s->grid_blocks.p, s->n_grid_blocks, fp::MODE_STEP, exact, s->stream));
     HIP_TRY(fp::launch_faces(a, s->csr(), s->csr_face_blocks.p, s->n_csr_face_blocks, exact, s->stream));

@@ -93,8 +93,8 @@ struct fp_sim {
   uint32_t n_grid_blocks = 0, n_csr_blocks = 0;
   // LDS-tiled grid kernel: per mesh its tiles (all of the mesh's tile shape), and per shape the
   // tiles of every tiled mesh in XCD-aware launch order
-  fph::DBuf<fp::TileRange> tiles[fp::N_TILE_SHAPES], mesh_tiles;
-  uint32_t n_tiles[fp::N_TILE_SHAPES] = {0, 0, 0};
+  fph::DBuf<fp::TileRange> tiles[fp::N_LAUNCH_SHAPES], mesh_tiles;
+  uint32_t n_tiles[fp::N_LAUNCH_SHAPES] = {};
   fph::DBuf<fp::ClothView> cloths;
   fph::DBuf<fp::StepParams> params;
   int32_t kernel = FP_KERNEL_AUTO, math = FP_MATH_EXACT;

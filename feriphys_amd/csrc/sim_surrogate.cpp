@@ -135,9 +135,8 @@ int sur_big_step(fp_sim* s, fp_surrogate_stats& st, float* mlp_ms) {
   if (mlp_ms) HIP_TRY(hipEventRecord(s->ev1, s->stream));
   HIP_TRY(fp::launch_sur_integrate(a, s->csr(), vb, nvb, S.da.p, S.work.p, !fused, s->stream));
   if (fused)
-    for (int sh = 0; sh < fp::N_TILE_SHAPES; ++sh)
-      HIP_TRY(fp::launch_grid_tiled(a, s->cloths.p, s->tiles[sh].p, s->n_tiles[sh], sh, fp::MODE_SURROGATE, false,
-                                    s->stream));
+    for (int sh = 0; sh < fp::N_LAUNCH_SHAPES; ++sh)
+      HIP_TRY(fp::launch_grid_tiled(a, s->cloths.p, s->tiles[sh].p, s->n_tiles[sh], sh, fp::MODE_SURROGATE, s->stream));
   HIP_TRY(fp::launch_sur_diag(a.in, a.out, S.slots.p, S.slot_k.p, S.big_params.p, s->mass.p, S.work.p, s->all_blocks.p,
                               nblk, S.diag.p, s->stream));
   std::vector<fp::DiagOut> d(nblk);

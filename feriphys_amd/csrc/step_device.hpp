@@ -83,6 +83,9 @@ struct ObsView {
   GridView grid[4];
   const uint32_t* always;  // ascending
   uint32_t n_always;
+  // with use_grid and no `always` faces: a box outside which no segment can hit a face (the union of
+  // the faces' boxes grown twice by the margin, unbounded along a thin face's dropped axis)
+  float box_lo[3], box_hi[3];
 };
 
 __device__ __forceinline__ f3 ld3(const float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ z,
@@ -144,14 +147,14 @@ FP_HD f3 face_force(f3 p0, f3 p1, f3 p2, f3 u0, f3 u1, f3 u2, const StepParams& 
 // Face::vertex_angle (springy_mesh.rs:163-172): angle between (p_b - p_a) and (p_c - p_a) at p_a,
 // called as (p2 - p0).angle(p1 - p0) for corner 0 etc.; returns angle / PI.
 template <class M>
-FP_HD float corner_weight(f3 pa, f3 pnext, f3 pprev) {
+FP_HD float corner_weight(f3 pa, f3 pnext, f3 pprev, const float (*tab)[4] = nullptr) {
   // vertex_angle(v0, v1, v2) = (p[v2] - p[v0]).angle(p[v1] - p[v0]); angle = atan2(|a x b|, a.b)
   f3 a = sub(pprev, pa);
   f3 b = sub(pnext, pa);
   f3 axb = cross(a, b);
   const float n2 = M::dot(axb, axb), d = M::dot(a, b);
   float w;
-  if (M::corner_in_range(n2, d, w)) return w;
+  if (M::corner_in_range(n2, d, w, tab)) return w;
   return M::div_pi(M::atan2_(M::sqrt_(n2), d));  // Rad / Rad(PI), PI = std::f32::consts::PI
 }
 
@@ -180,6 +183,22 @@ __device__ __forceinline__ void hinge_forces(f3 x0, f3 x1, f3 x2, f3 x3, f3 v2, 
   out[2] = smul(M::div(th, ml), nl);
   out[1] = sdiv(add(smul(d02h, out[2]), smul(d03h, out[3])), l01);  // Vector3 / f32: per component
   out[0] = smul(-1.0f, add(add(out[1], out[2]), out[3]));
+}
+
+// One component of `integrate`.
+template <class M>
+FP_HD void integrate1(const StepParams& P, float m, float x, float v, float F, float& xn, float& vn) {
+  const float a1 = M::div(F, m);
+  if (P.integration == FP_EULER) {
+    xn = x + v * P.dt;
+    vn = v + a1 * P.dt;
+    return;
+  }
+  const float z0 = m > 0.0f ? 0.0f : M::div(0.0f, m), a2 = F == 0.0f ? z0 : a1;
+  const float hh = P.dt_half, h = P.dt, h6 = P.dt6, h3 = P.dt3;
+  const float v2 = v + a1 * hh, v3 = v + a2 * hh, v4 = v + a2 * h;
+  xn = x + (((h6 * v + h3 * v2) + h3 * v3) + h6 * v4);
+  vn = v + (((h6 * a1 + h3 * a2) + h3 * a2) + h6 * a2);
 }
 
 // The explicit integrators of state.rs:75-106 applied to one Point record (springy_mesh.rs:223-240)
@@ -276,16 +295,21 @@ __device__ __forceinline__ int32_t first_hit(const ObsView& O, f3 old_p, f3 new_
       if (face_hit(load_face(O.faces, f), old_p, new_p, dt_d)) return (int32_t)f;
     return -1;
   }
+  const float lo[3] = {fminf(old_p.x, new_p.x) - O.margin, fminf(old_p.y, new_p.y) - O.margin,
+                       fminf(old_p.z, new_p.z) - O.margin};
+  const float hi[3] = {fmaxf(old_p.x, new_p.x) + O.margin, fmaxf(old_p.y, new_p.y) + O.margin,
+                       fmaxf(old_p.z, new_p.z) + O.margin};
+  // a segment whose grown box misses the faces' box meets no grid cell that lists a face: most vertices
+  // leave here, before the four grids' cell arithmetic
+  if (O.n_always == 0 && !(lo[0] <= O.box_hi[0] && hi[0] >= O.box_lo[0] && lo[1] <= O.box_hi[1] &&
+                           hi[1] >= O.box_lo[1] && lo[2] <= O.box_hi[2] && hi[2] >= O.box_lo[2]))
+    return -1;
   uint32_t best = 0xffffffffu;
   for (uint32_t k = 0; k < O.n_always; ++k) {
     const uint32_t f = O.always[k];
     if (f >= best) break;
     if (face_hit(load_face(O.faces, f), old_p, new_p, dt_d)) { best = f; break; }
   }
-  const float lo[3] = {fminf(old_p.x, new_p.x) - O.margin, fminf(old_p.y, new_p.y) - O.margin,
-                       fminf(old_p.z, new_p.z) - O.margin};
-  const float hi[3] = {fmaxf(old_p.x, new_p.x) + O.margin, fmaxf(old_p.y, new_p.y) + O.margin,
-                       fmaxf(old_p.z, new_p.z) + O.margin};
   for (int g = 0; g < 4; ++g) grid_hits(O.grid[g], O.faces, lo, hi, old_p, new_p, dt_d, best);
   return best == 0xffffffffu ? -1 : (int32_t)best;
 }
