@@ -355,6 +355,22 @@ __global__ void __launch_bounds__(kBlock) update_points_kernel(StepArgs A, const
   A.fx[i] = Fn.x; A.fy[i] = Fn.y; A.fz[i] = Fn.z;
 }
 
+// A workgroup's share of packed records, `words` floats each: between LDS and memory in 16-byte units,
+// so that every transaction is whole lines whatever the record's size (the other side may be
+// page-locked host memory, where each line crosses the bus once).  `n` is the records of this workgroup.
+__device__ __forceinline__ void records_to_lds(const float* __restrict__ src, float* lds, uint32_t words) {
+  const uint32_t quads = words / 4;
+  for (uint32_t k = threadIdx.x; k < quads; k += kBlock)
+    reinterpret_cast<float4*>(lds)[k] = reinterpret_cast<const float4*>(src)[k];
+  for (uint32_t k = 4 * quads + threadIdx.x; k < words; k += kBlock) lds[k] = src[k];
+}
+__device__ __forceinline__ void records_from_lds(const float* lds, float* __restrict__ dst, uint32_t words) {
+  const uint32_t quads = words / 4;
+  for (uint32_t k = threadIdx.x; k < quads; k += kBlock)
+    reinterpret_cast<float4*>(dst)[k] = reinterpret_cast<const float4*>(lds)[k];
+  for (uint32_t k = 4 * quads + threadIdx.x; k < words; k += kBlock) dst[k] = lds[k];
+}
+
 // The Stateful records [m, x, y, z, vx, vy, vz, Fx, Fy, Fz] (springy_mesh.rs:242-255) of device
 // vertices [base, base + n) in the reference's vertex order: record i from device slot
 // base + pos[i] (base + i without a permutation).
@@ -363,39 +379,64 @@ __global__ void __launch_bounds__(kBlock) pack_records_kernel(SoA S, const float
                                                                const float* __restrict__ fz,
                                                                const uint32_t* __restrict__ pos, uint32_t base,
                                                                uint32_t n, float* __restrict__ out) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t d = base + (pos != nullptr ? pos[i] : i);
-  float* o = out + 10ull * i;
-  o[0] = mass[d];
-  o[1] = S.x[d]; o[2] = S.y[d]; o[3] = S.z[d];
-  o[4] = S.vx[d]; o[5] = S.vy[d]; o[6] = S.vz[d];
-  o[7] = fx[d]; o[8] = fy[d]; o[9] = fz[d];
+  __shared__ float4 s_rec[10 * kBlock / 4];
+  const uint32_t first = blockIdx.x * kBlock, i = first + threadIdx.x;
+  if (i < n) {
+    const uint32_t d = base + (pos != nullptr ? pos[i] : i);
+    float* o = reinterpret_cast<float*>(s_rec) + 10 * threadIdx.x;
+    o[0] = mass[d];
+    o[1] = S.x[d]; o[2] = S.y[d]; o[3] = S.z[d];
+    o[4] = S.vx[d]; o[5] = S.vy[d]; o[6] = S.vz[d];
+    o[7] = fx[d]; o[8] = fy[d]; o[9] = fz[d];
+  }
+  __syncthreads();
+  records_from_lds(reinterpret_cast<const float*>(s_rec), out + 10ull * first, 10 * min(kBlock, n - first));
 }
 
 // The positions of device vertices [base, base + n) in the reference's vertex order, 3 floats each.
 __global__ void __launch_bounds__(kBlock) pack_positions_kernel(SoA S, const uint32_t* __restrict__ pos, uint32_t base,
                                                                  uint32_t n, float* __restrict__ out) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t d = base + (pos != nullptr ? pos[i] : i);
-  out[3ull * i] = S.x[d]; out[3ull * i + 1] = S.y[d]; out[3ull * i + 2] = S.z[d];
+  __shared__ float4 s_rec[3 * kBlock / 4];
+  const uint32_t first = blockIdx.x * kBlock, i = first + threadIdx.x;
+  if (i < n) {
+    const uint32_t d = base + (pos != nullptr ? pos[i] : i);
+    float* o = reinterpret_cast<float*>(s_rec) + 3 * threadIdx.x;
+    o[0] = S.x[d]; o[1] = S.y[d]; o[2] = S.z[d];
+  }
+  __syncthreads();
+  records_from_lds(reinterpret_cast<const float*>(s_rec), out + 3ull * first, 3 * min(kBlock, n - first));
 }
 
 // The inverse of pack_records_kernel: records in the reference's vertex order into the state,
-// masses and force records of device vertices [base, base + n).
+// masses and force records of device vertices [base, base + n).  scan (page-locked host memory, zero
+// before the launch) learns what the host would otherwise read every record for: whether any force
+// component is not +0, and whether any mass differs from the first.
 __global__ void __launch_bounds__(kBlock) unpack_records_kernel(const float* __restrict__ in, const uint32_t* __restrict__ pos,
                                                                  uint32_t base, uint32_t n, SoA S, float* __restrict__ mass,
                                                                  float* __restrict__ fx, float* __restrict__ fy,
-                                                                 float* __restrict__ fz) {
-  const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t d = base + (pos != nullptr ? pos[i] : i);
-  const float* q = in + 10ull * i;
-  mass[d] = q[0];
-  S.x[d] = q[1]; S.y[d] = q[2]; S.z[d] = q[3];
-  S.vx[d] = q[4]; S.vy[d] = q[5]; S.vz[d] = q[6];
-  fx[d] = q[7]; fy[d] = q[8]; fz[d] = q[9];
+                                                                 float* __restrict__ fz, RecordScan* scan) {
+  __shared__ float4 s_rec[10 * kBlock / 4];
+  const uint32_t first = blockIdx.x * kBlock, i = first + threadIdx.x;
+  const float m0 = in[0];
+  records_to_lds(in + 10ull * first, reinterpret_cast<float*>(s_rec), 10 * min(kBlock, n - first));
+  __syncthreads();
+  bool force = false, differs = false;
+  if (i < n) {
+    const uint32_t d = base + (pos != nullptr ? pos[i] : i);
+    const float* q = reinterpret_cast<const float*>(s_rec) + 10 * threadIdx.x;
+    const float m = q[0], f0 = q[7], f1 = q[8], f2 = q[9];
+    mass[d] = m;
+    S.x[d] = q[1]; S.y[d] = q[2]; S.z[d] = q[3];
+    S.vx[d] = q[4]; S.vy[d] = q[5]; S.vz[d] = q[6];
+    fx[d] = f0; fy[d] = f1; fz[d] = f2;
+    force = (__float_as_uint(f0) | __float_as_uint(f1) | __float_as_uint(f2)) != 0u;
+    differs = i > 0 && !(m == m0 && sign_positive(m) == sign_positive(m0));
+  }
+  const int forces = __syncthreads_or(force), masses = __syncthreads_or(differs);
+  if (threadIdx.x == 0) {  // every workgroup stores the same 1
+    if (forces) scan->force = 1u;
+    if (masses) scan->mass = 1u;
+  }
 }
 
 // Per mesh, the number of vertices whose position or velocity is not finite.
@@ -529,10 +570,10 @@ hipError_t launch_pack_positions(const SoA& st, const uint32_t* pos, uint32_t ba
 }
 
 hipError_t launch_unpack_records(const float* in, const uint32_t* pos, uint32_t base, uint32_t n, const SoA& st,
-                                 float* mass, float* fx, float* fy, float* fz, hipStream_t s) {
+                                 float* mass, float* fx, float* fy, float* fz, RecordScan* scan, hipStream_t s) {
   if (n == 0) return hipSuccess;
   unpack_records_kernel<<<dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s>>>(in, pos, base, n, st, mass, fx, fy,
-                                                                                 fz);
+                                                                                 fz, scan);
   return hipGetLastError();
 }
 

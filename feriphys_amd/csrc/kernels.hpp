@@ -170,9 +170,13 @@ hipError_t launch_pack_records(const SoA& st, const float* mass, const float* fx
 // The positions of device vertices [base, base + n), 3 floats each, in the reference's order.
 hipError_t launch_pack_positions(const SoA& st, const uint32_t* pos, uint32_t base, uint32_t n, float* out,
                                  hipStream_t s);
-// The inverse: 10 n floats of records (reference order) into the state, masses and forces.
+// The inverse: 10 n floats of records (reference order) into the state, masses and forces, with what
+// the host needs to know about them: any force component other than +0, any mass unlike the first.
+struct RecordScan {
+  uint32_t force, mass;
+};
 hipError_t launch_unpack_records(const float* in, const uint32_t* pos, uint32_t base, uint32_t n, const SoA& st,
-                                 float* mass, float* fx, float* fy, float* fz, hipStream_t s);
+                                 float* mass, float* fx, float* fy, float* fz, RecordScan* scan, hipStream_t s);
 
 constexpr uint32_t kBlock = 256;
 

@@ -167,14 +167,22 @@ int check_config(const fp_config* c) {
   return FP_OK;
 }
 
-// Re-derives whether the mesh's masses are all equal (the grid kernel and the scalar-mass path
-// need that) from its records.
-void refresh_mass(MeshSlot& ms, const float* rec, uint64_t n) {
+// Whether n masses, `stride` floats apart, are all equal (as values and in sign).
+bool equal_masses(const float* mass, uint64_t n, uint64_t stride) {
   bool uni = true;
-  float m0 = n ? rec[0] : 0.0f;
-  for (uint64_t i = 1; i < n && uni; ++i) uni = (rec[10 * i] == m0) && !(std::signbit(rec[10 * i]) != std::signbit(m0));
-  ms.uniform_mass = uni;
-  ms.params = make_params(ms.cfg, m0, uni);
+  for (uint64_t i = 1; i < n && uni; ++i)
+    uni = mass[stride * i] == mass[0] && std::signbit(mass[stride * i]) == std::signbit(mass[0]);
+  return uni;
+}
+
+// Records of mesh slot `m` now have first mass m0, all equal or not (the grid kernel and the
+// scalar-mass path need that); returns whether that changed the mesh's parameters.
+bool refresh_mass(MeshSlot& ms, float m0, bool uniform) {
+  const fp::StepParams p = make_params(ms.cfg, m0, uniform);
+  const bool same = uniform == ms.uniform_mass && std::memcmp(&p, &ms.params, sizeof(p)) == 0;
+  ms.uniform_mass = uniform;
+  ms.params = p;
+  return !same;
 }
 
 int upload_params(fp_sim* s) {
@@ -322,6 +330,25 @@ int check_mesh(const fp_mesh* m) {
 int check_sim_mesh(const fp_sim* s, uint64_t mesh) {
   if (!s) return fail(FP_EINVAL, "sim is NULL");
   if (mesh >= s->meshes.size()) return fail(FP_EINVAL, "mesh index out of range");
+  return FP_OK;
+}
+
+// `count` floats that `pack` writes on the device, into the caller's `dst`: straight into page-locked
+// memory and from there when they are few, otherwise through device memory and one copy.
+template <class Pack>
+int read_back(fp_sim* s, float* dst, uint64_t count, Pack pack) {
+  const size_t bytes = count * sizeof(float);
+  if (bytes <= fph::kDirectBytes) {
+    HIP_TRY(s->host_rec.reserve(fph::kDirectBytes));
+    HIP_TRY(pack(s->host_rec.floats()));
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    std::memcpy(dst, s->host_rec.p, bytes);
+    return FP_OK;
+  }
+  HIP_TRY(s->rec_stage.reserve(count));
+  HIP_TRY(pack(s->rec_stage.p));
+  HIP_TRY(hipMemcpyAsync(dst, s->rec_stage.p, bytes, hipMemcpyDeviceToHost, s->stream));
+  HIP_TRY(hipStreamSynchronize(s->stream));
   return FP_OK;
 }
 
@@ -872,7 +899,7 @@ int fp_sim_new(fp_mesh* const* meshes, uint64_t n_meshes, fp_obstacle* const* ob
     F += slot.host.n_faces();
     Sdir += 2 * slot.host.n_struts();
     Fent += 3 * slot.host.n_faces();
-    refresh_mass(slot, slot.host.rec.data(), slot.host.n);
+    refresh_mass(slot, slot.host.n ? slot.host.rec[0] : 0.0f, equal_masses(slot.host.rec.data(), slot.host.n, 10));
     if (slot.host.cloth.valid) slot.tile_shape = default_tile_shape(slot.host.cloth.rows, slot.host.cloth.cols);
     if (!slot.host.cloth.valid && slot.host.n > 1) {
       patch_order(slot.host, slot.perm, slot.bstart);
@@ -1115,16 +1142,13 @@ int fp_sim_get_points(fp_sim* s, uint64_t mesh, float* rec) {
   const MeshSlot& m = s->meshes[mesh];
   const uint64_t n = m.host.n, b = m.vbase;
   if (n == 0) return FP_OK;
-  // the records packed in the reference's order on the device, then one copy
-  HIP_TRY(s->rec_stage.reserve(10 * n));
+  // packed in the reference's order by the device
   const auto& st = s->state[s->cur];
   const fp::SoA cur{st[0].p, st[1].p, st[2].p, st[3].p, st[4].p, st[5].p};
-  HIP_TRY(fp::launch_pack_records(cur, s->mass.p, s->force[0].p, s->force[1].p, s->force[2].p,
-                                  m.pos.empty() ? nullptr : s->d_pos.p + b, (uint32_t)b, (uint32_t)n,
-                                  s->rec_stage.p, s->stream));
-  HIP_TRY(hipStreamSynchronize(s->stream));
-  HIP_TRY(hipMemcpy(rec, s->rec_stage.p, 10 * n * sizeof(float), hipMemcpyDeviceToHost));
-  return FP_OK;
+  return read_back(s, rec, 10 * n, [&](float* out) {
+    return fp::launch_pack_records(cur, s->mass.p, s->force[0].p, s->force[1].p, s->force[2].p,
+                                   m.pos.empty() ? nullptr : s->d_pos.p + b, (uint32_t)b, (uint32_t)n, out, s->stream);
+  });
 }
 
 int fp_sim_set_points(fp_sim* s, uint64_t mesh, const float* rec, uint64_t n) {
@@ -1132,22 +1156,32 @@ int fp_sim_set_points(fp_sim* s, uint64_t mesh, const float* rec, uint64_t n) {
   MeshSlot& m = s->meshes[mesh];
   if (n != m.host.n) return fail(FP_EINVAL, "State Vector incorrect size! (record count != point count)");
   if (n && !rec) return fail(FP_EINVAL, "records is NULL");
-  HIP_TRY(hipStreamSynchronize(s->stream));
-  if (n) {  // one copy, then the records scattered into the device order on the device
-    HIP_TRY(s->rec_stage.reserve(10 * n));
-    HIP_TRY(hipMemcpy(s->rec_stage.p, rec, 10 * n * sizeof(float), hipMemcpyHostToDevice));
-    const auto& st = s->state[s->cur];
-    const fp::SoA cur{st[0].p, st[1].p, st[2].p, st[3].p, st[4].p, st[5].p};
-    HIP_TRY(fp::launch_unpack_records(s->rec_stage.p, m.pos.empty() ? nullptr : s->d_pos.p + m.vbase,
-                                      (uint32_t)m.vbase, (uint32_t)n, cur, s->mass.p, s->force[0].p, s->force[1].p,
-                                      s->force[2].p, s->stream));
+  if (n == 0) {
     HIP_TRY(hipStreamSynchronize(s->stream));
+    return FP_OK;
   }
-  bool nonzero_f = false;
-  for (uint64_t i = 0; i < n && !nonzero_f; ++i)
-    for (int k = 7; k < 10; ++k) nonzero_f = nonzero_f || rec[10 * i + k] != 0.0f || std::signbit(rec[10 * i + k]);
-  s->forces_dirty = s->forces_dirty || nonzero_f;
-  refresh_mass(m, rec, n);
+  // scattered into the device order, and scanned for forces and unequal masses, by the device
+  const size_t bytes = 10 * n * sizeof(float);
+  const float* src;
+  HIP_TRY(s->scan.reserve(sizeof(fp::RecordScan)));
+  auto* scan = static_cast<fp::RecordScan*>(s->scan.p);
+  *scan = fp::RecordScan{0, 0};
+  if (bytes <= fph::kDirectBytes) {
+    HIP_TRY(s->host_rec.reserve(fph::kDirectBytes));
+    std::memcpy(s->host_rec.p, rec, bytes);
+    src = s->host_rec.floats();
+  } else {
+    HIP_TRY(s->rec_stage.reserve(10 * n));
+    HIP_TRY(hipMemcpyAsync(s->rec_stage.p, rec, bytes, hipMemcpyHostToDevice, s->stream));
+    src = s->rec_stage.p;
+  }
+  const auto& st = s->state[s->cur];
+  const fp::SoA cur{st[0].p, st[1].p, st[2].p, st[3].p, st[4].p, st[5].p};
+  HIP_TRY(fp::launch_unpack_records(src, m.pos.empty() ? nullptr : s->d_pos.p + m.vbase, (uint32_t)m.vbase, (uint32_t)n,
+                                    cur, s->mass.p, s->force[0].p, s->force[1].p, s->force[2].p, scan, s->stream));
+  HIP_TRY(hipStreamSynchronize(s->stream));
+  s->forces_dirty = s->forces_dirty || scan->force != 0;
+  if (!refresh_mass(m, rec[0], scan->mass == 0)) return FP_OK;
   if (int e = upload_params(s)) return e;
   return build_block_lists(s);
 }
@@ -1156,14 +1190,14 @@ int fp_sim_get_vertices(fp_sim* s, uint64_t mesh, float* pos, uint64_t* idx) {
   if (int e = check_sim_mesh(s, mesh)) return e;
   const MeshSlot& m = s->meshes[mesh];
   const uint64_t n = m.host.n;
-  if (pos && n) {  // positions packed in the reference's order on the device, one copy
-    HIP_TRY(s->rec_stage.reserve(3 * n));
+  if (pos && n) {  // positions packed in the reference's order by the device
     const auto& st = s->state[s->cur];
     const fp::SoA cur{st[0].p, st[1].p, st[2].p, st[3].p, st[4].p, st[5].p};
-    HIP_TRY(fp::launch_pack_positions(cur, m.pos.empty() ? nullptr : s->d_pos.p + m.vbase, (uint32_t)m.vbase,
-                                      (uint32_t)n, s->rec_stage.p, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    HIP_TRY(hipMemcpy(pos, s->rec_stage.p, 3 * n * sizeof(float), hipMemcpyDeviceToHost));
+    const int e = read_back(s, pos, 3 * n, [&](float* out) {
+      return fp::launch_pack_positions(cur, m.pos.empty() ? nullptr : s->d_pos.p + m.vbase, (uint32_t)m.vbase,
+                                       (uint32_t)n, out, s->stream);
+    });
+    if (e) return e;
   }
   if (idx) std::copy(m.host.f_v.begin(), m.host.f_v.end(), idx);
   return FP_OK;
@@ -1248,10 +1282,9 @@ int fp_sim_update_points(fp_sim* s, uint64_t mesh, const float* rec, uint64_t n)
   HIP_TRY(hipStreamSynchronize(s->stream));
   s->forces_dirty = true;
   // masses may have changed: re-derive the uniform-mass flag from the device copy
-  std::vector<float> mm(n), r10(10 * n, 0.0f);
+  std::vector<float> mm(n);  // device order: only the uniformity matters
   HIP_TRY(hipMemcpy(mm.data(), s->mass.p + m.vbase, n * sizeof(float), hipMemcpyDeviceToHost));
-  for (uint64_t i = 0; i < n; ++i) r10[10 * i] = mm[i];  // device order: only the uniformity matters
-  refresh_mass(m, r10.data(), n);
+  refresh_mass(m, mm[0], equal_masses(mm.data(), n, 1));
   if (int e = upload_params(s)) return e;
   return build_block_lists(s);
 }
