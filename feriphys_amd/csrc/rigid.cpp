@@ -2,6 +2,7 @@
 // host, rigidbody::Simulation on the device (rigid_kernels.hip), one 29-float record per body.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <memory>
 #include <vector>
@@ -25,9 +26,8 @@ struct fp_rigid_sim {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   uint64_t pitch = 0;  // floats per field of the device records (n rounded up to kRigidAlign)
-  DBuf<float> rec[2];  // ping-pong, field-major (rigid.hpp)
+  DBuf<float> rec;     // field-major (rigid.hpp), stepped in place: bodies do not interact
   DBuf<float> stage;   // the caller's layout (29 floats per body) for one copy each way
-  int cur = 0;
   fph::ObstacleSet obst;
   fp_rigid_config cfg{};
   ~fp_rigid_sim() {
@@ -172,8 +172,7 @@ int fp_rigid_sim_new(fp_rigid* const* bodies, uint64_t n_bodies, fp_obstacle* co
   std::vector<float> h(fp::kRigidRecord * s->pitch + 1, 0.0f);
   for (uint64_t i = 0; i < n_bodies; ++i)
     for (int k = 0; k < fp::kRigidRecord; ++k) h[k * s->pitch + i] = bs[i]->rec[k];
-  HIP_TRY(s->rec[0].upload(h.data(), h.size()));
-  HIP_TRY(s->rec[1].upload(h.data(), h.size()));
+  HIP_TRY(s->rec.upload(h.data(), h.size()));
   std::vector<fp::HostObstacle> obs;
   for (auto& o : os) obs.push_back(std::move(o->o));
   if (int e = fph::upload_obstacles(s->obst, obs)) return e;
@@ -203,13 +202,15 @@ int fp_rigid_sim_get_config(const fp_rigid_sim* s, fp_rigid_config* c) {
   return FP_OK;
 }
 
+// Steps per launch: enough that a launch's own cost and its record traffic vanish among them, few
+// enough that a launch over the largest batches ends within milliseconds.
+constexpr uint64_t kRigidChunk = 64;
+
 static int run_rigid(fp_rigid_sim* s, uint64_t n) {
   const fp::RigidParams p = params_of(s->cfg);
-  for (uint64_t k = 0; k < n; ++k) {
-    HIP_TRY(fp::launch_rigid_step(s->rec[s->cur].p, s->rec[s->cur ^ 1].p, (uint32_t)s->n, (uint32_t)s->pitch, p,
-                                  s->obst.view, s->stream));
-    s->cur ^= 1;
-  }
+  for (uint64_t k = 0; k < n; k += kRigidChunk)
+    HIP_TRY(fp::launch_rigid_steps(s->rec.p, (uint32_t)s->n, (uint32_t)s->pitch, p, s->obst.view,
+                                   (uint32_t)std::min(kRigidChunk, n - k), s->stream));
   return FP_OK;
 }
 
@@ -233,10 +234,9 @@ int fp_rigid_sim_time_steps(fp_rigid_sim* s, uint64_t n_steps, float* ms) {
 
 int fp_rigid_sim_get_states(fp_rigid_sim* s, float* records) {
   if (!s || (!records && s->n)) return fail(FP_EINVAL, "NULL argument");
-  HIP_TRY(hipStreamSynchronize(s->stream));
   if (s->n == 0) return FP_OK;
   HIP_TRY(s->stage.reserve(fp::kRigidRecord * s->n));
-  HIP_TRY(fp::launch_rigid_records(s->rec[s->cur].p, s->stage.p, (uint32_t)s->n, (uint32_t)s->pitch, true, s->stream));
+  HIP_TRY(fp::launch_rigid_records(s->rec.p, s->stage.p, (uint32_t)s->n, (uint32_t)s->pitch, true, s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   HIP_TRY(hipMemcpy(records, s->stage.p, fp::kRigidRecord * s->n * sizeof(float), hipMemcpyDeviceToHost));
   return FP_OK;
@@ -250,7 +250,7 @@ int fp_rigid_sim_set_states(fp_rigid_sim* s, const float* records, uint64_t n) {
   if (n == 0) return FP_OK;
   HIP_TRY(s->stage.reserve(fp::kRigidRecord * n));
   HIP_TRY(hipMemcpy(s->stage.p, records, fp::kRigidRecord * n * sizeof(float), hipMemcpyHostToDevice));
-  HIP_TRY(fp::launch_rigid_records(s->stage.p, s->rec[s->cur].p, (uint32_t)n, (uint32_t)s->pitch, false, s->stream));
+  HIP_TRY(fp::launch_rigid_records(s->stage.p, s->rec.p, (uint32_t)n, (uint32_t)s->pitch, false, s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   return FP_OK;
 }
@@ -260,7 +260,7 @@ int fp_rigid_sim_apply_impulse(fp_rigid_sim* s, uint64_t body, const float impul
   if (body >= s->n) return fail(FP_EINVAL, "body index out of range");
   HIP_TRY(hipStreamSynchronize(s->stream));
   float r[fp::kRigidRecord];
-  float* d = s->rec[s->cur].p + body;  // field k at d + k * pitch
+  float* d = s->rec.p + body;  // field k at d + k * pitch
   const size_t fp_bytes = s->pitch * sizeof(float);
   HIP_TRY(hipMemcpy2D(r, sizeof(float), d, fp_bytes, sizeof(float), fp::kRigidRecord, hipMemcpyDeviceToHost));
   apply_impulse(r, impulse, position);

@@ -33,8 +33,8 @@ struct RigidParams {
 // inverse.
 hipError_t launch_rigid_records(const float* in, float* out, uint32_t n, uint32_t pitch, bool pack, hipStream_t s);
 
-// One Simulation::step of n bodies: records in -> out (field-major, `pitch` floats per field).
-hipError_t launch_rigid_step(const float* in, float* out, uint32_t n, uint32_t pitch, const RigidParams& p,
-                             const ObsView& obs, hipStream_t s);
+// `steps` Simulation::steps of n bodies in place (field-major, `pitch` floats per field).
+hipError_t launch_rigid_steps(float* rec, uint32_t n, uint32_t pitch, const RigidParams& p, const ObsView& obs,
+                              uint32_t steps, hipStream_t s);
 
 }  // namespace fp

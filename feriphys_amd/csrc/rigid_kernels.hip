@@ -48,100 +48,280 @@ __device__ __forceinline__ M3 from_quat(Q q) {
   return M3{{f3{1.0f - yy2 - zz2, xy2 + sz2, xz2 - sy2}, f3{xy2 - sz2, 1.0f - xx2 - zz2, yz2 + sx2},
              f3{xz2 + sy2, yz2 - sx2, 1.0f - xx2 - yy2}}};
 }
-__device__ __forceinline__ Q rot(const float* S) { return Q{S[6], f3{S[3], S[4], S[5]}}; }
-__device__ __forceinline__ M3 inertia0(const float* S) {
-  return M3{{f3{S[14], S[15], S[16]}, f3{S[17], S[18], S[19]}, f3{S[20], S[21], S[22]}}};
-}
 // State::get_moment_of_inertia_inverted (rigidbody.rs:33-36): (R I0^-1) R^T
-__device__ __forceinline__ M3 inertia_inv(const float* S) {
-  const M3 R = from_quat(rot(S));
-  return mm(mm(R, inertia0(S)), tr(R));
+__device__ __forceinline__ M3 inertia_inv(Q q, const M3& I0) {
+  const M3 R = from_quat(q);
+  return mm(mm(R, I0), tr(R));
 }
 
-// Stateful::derivative (rigidbody.rs:94-157)
-__device__ __forceinline__ void derivative(const float* S, float* D) {
-  const float m = S[13];
-  const f3 v = f3{S[7] / m, S[8] / m, S[9] / m};  // linear_momentum / mass
-  const f3 w = mv(inertia_inv(S), f3{S[10], S[11], S[12]});
-  const Q qd = qmul(Q{0.5f * 0.0f, f3{0.5f * w.x, 0.5f * w.y, 0.5f * w.z}}, rot(S));
-  D[0] = v.x; D[1] = v.y; D[2] = v.z;
-  D[3] = qd.v.x; D[4] = qd.v.y; D[5] = qd.v.z; D[6] = qd.s;
-  for (int k = 7; k < 13; ++k) D[k] = S[k + 16];  // force, torque
+// The fields of a record that a step changes; the mass and I0^-1 stay, force and torque are cleared.
+struct Body {
+  f3 x;
+  Q q;
+  f3 p, l;  // linear and angular momentum
+};
+// Stateful::derivative (rigidbody.rs:94-157) of those fields; the momenta's are force and torque.
+__device__ __forceinline__ void derivative(const Body& S, float m, const M3& I0, f3& dx, Q& dq) {
+  dx = ExactMath::div3(S.p, m);  // linear_momentum / mass
+  const f3 w = mv(inertia_inv(S.q, I0), S.l);
+  dq = qmul(Q{0.5f * 0.0f, f3{0.5f * w.x, 0.5f * w.y, 0.5f * w.z}}, S.q);
+}
+// Makes values opaque where they stand: the compiler otherwise interleaves the four stages (the momenta's
+// slopes, and so every stage's division, are known from the start) and holds 210 registers.
+__device__ __forceinline__ void settle(f3& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z)); }
+__device__ __forceinline__ void settle(Q& q) { asm volatile("" : "+v"(q.s), "+v"(q.v.x), "+v"(q.v.y), "+v"(q.v.z)); }
+__device__ __forceinline__ void settle(Body& b) { settle(b.x); settle(b.q); settle(b.p); settle(b.l); }
+// From the second stage on a -0 in the mass or the inertia has become +0 (every field advances by its
+// slope, and theirs is 0); formed anew per stage, not held.
+__device__ __forceinline__ void derivative_later(const Body& S, float m, M3 I0, f3& dx, Q& dq) {
+  for (int c = 0; c < 3; ++c) {
+    settle(I0.c[c]);
+    I0.c[c] = add(I0.c[c], f3{0.0f, 0.0f, 0.0f});
+  }
+  derivative(S, m + 0.0f, I0, dx, dq);
+}
+// a + s b, per component, as the reference's vec_add and scale round it
+__device__ __forceinline__ f3 axpy(f3 a, float s, f3 b) { return f3{a.x + b.x * s, a.y + b.y * s, a.z + b.z * s}; }
+__device__ __forceinline__ Q axpy(Q a, float s, Q b) { return Q{a.s + b.s * s, axpy(a.v, s, b.v)}; }
+
+// The world offsets of the cube's corners, R c with c = (+-1/2, +-1/2, +-1/2): with a = R / 2 (exact),
+// row by row (+-a0 +- a1) +- a2, where negation is exact: corner k is +-(s or d) +- a2 with s = a0 + a1
+// and d = a0 - a1.
+struct Corners {
+  f3 s, d, a;
+};
+__device__ __forceinline__ Corners corners_of(const M3& R) {
+  const f3 a0 = smul(0.5f, R.c[0]), a1 = smul(0.5f, R.c[1]);
+  return Corners{add(a0, a1), sub(a0, a1), smul(0.5f, R.c[2])};
+}
+// Corner k of kCubeCorner's order at body position x: the offsets are -(s - a), d + a, s + a, -(d - a),
+// -(s + a), d - a, s - a, -(d + a).
+__device__ __forceinline__ f3 corner_at(const Corners& C, f3 x, int k) {
+  const f3 b = k % 2 == 0 ? C.s : C.d;
+  const bool minus = k == 0 || k == 3 || k == 5 || k == 6, negative = k == 0 || k == 3 || k == 4 || k == 7;
+  const f3 v = minus ? sub(b, C.a) : add(b, C.a);
+  return negative ? sub(x, v) : add(v, x);
+}
+// The same for a corner number of each lane's own, by selects and sign flips (b - a is b + (-a), x - v is
+// (-v) + x).
+__device__ __forceinline__ f3 corner_of_lane(const Corners& C, f3 x, uint32_t k) {
+  const bool even = (k & 1u) == 0u;
+  const uint32_t minus = (0x69u >> k & 1u) << 31, negative = (0x99u >> k & 1u) << 31;
+  auto flip = [](float v, uint32_t sign) { return __uint_as_float(__float_as_uint(v) ^ sign); };
+  auto one = [&](float s, float d, float a, float xc) { return flip((even ? s : d) + flip(a, minus), negative) + xc; };
+  return f3{one(C.s.x, C.d.x, C.a.x, x.x), one(C.s.y, C.d.y, C.a.y, x.y), one(C.s.z, C.d.z, C.a.z, x.z)};
+}
+
+// Obstacle face f (the same for the whole wave): never written while a kernel runs, so read through the
+// constant address space, which puts it in scalar registers.
+__device__ __forceinline__ ObsFace uniform_face(const ObsView& O, uint32_t f) {
+  const auto* F = (const __attribute__((address_space(4))) ObsFace*)(O.faces + f);
+  ObsFace q;
 #pragma unroll
-  for (int k = 13; k < kRigidRecord; ++k) D[k] = 0.0f;
+  for (int c = 0; c < 3; ++c) {
+    q.v0[c] = F->v0[c];
+    q.v1[c] = F->v1[c];
+    q.v2[c] = F->v2[c];
+    q.n[c] = F->n[c];
+  }
+  q.axis = F->axis;
+  return q;
 }
 
-__global__ void __launch_bounds__(kBlock) rigid_step_kernel(const float* __restrict__ in, float* __restrict__ out,
-                                                             uint32_t n, uint32_t pitch, RigidParams P, ObsView O) {
+// The corners (bit k: corner k) that can meet an obstacle between the two poses: with few faces, those
+// that change sides of some face's plane (the first test of face_hit, as it computes it); with the
+// grids, all or none, by the box around all the corners against the faces' box.
+template <bool GRID>
+__device__ __forceinline__ uint32_t may_hit(const ObsView& O, const Corners& Co, f3 xo, const Corners& Cn, f3 xn) {
+  if constexpr (!GRID) {
+    uint32_t any = 0;
+    for (uint32_t f = 0; f < O.n_faces; ++f) {
+      const ObsFace F = uniform_face(O, f);
+      const f3 v0 = f3{F.v0[0], F.v0[1], F.v0[2]}, n = f3{F.n[0], F.n[1], F.n[2]};
+      uint32_t crossed = 0;
+#pragma unroll
+      for (int k = 7; k >= 0; --k) {
+        if (k % 2 == 1) {  // the sixteen corner positions formed as they are needed, not held in 48 registers
+          settle(xo);
+          settle(xn);
+        }
+        const float od = dot(sub(corner_at(Co, xo, k), v0), n), nd = dot(sub(corner_at(Cn, xn, k), v0), n);
+        crossed = __builtin_amdgcn_alignbit(crossed, __float_as_uint(od) ^ __float_as_uint(nd), 31);
+      }
+      any |= crossed;
+    }
+    return any;
+  } else {
+    if (O.n_always != 0) return 0xffu;
+    // a corner's offset is at most max(|s|, |d|) + |a| in each row
+    auto meets = [&](float s0, float d0, float a0, float x0, float s1, float d1, float a1, float x1, float lo, float hi) {
+      const float e0 = fmaxf(fabsf(s0), fabsf(d0)) + fabsf(a0), e1 = fmaxf(fabsf(s1), fabsf(d1)) + fabsf(a1);
+      // 2 margin: the corners' own test grows by one; the other covers the rounding of these sums (the
+      // margin is at least 1e-4 of the largest obstacle coordinate)
+      return !(fminf(x0 - e0, x1 - e1) - 2.0f * O.margin > hi) && !(fmaxf(x0 + e0, x1 + e1) + 2.0f * O.margin < lo);
+    };
+    const bool near = meets(Co.s.x, Co.d.x, Co.a.x, xo.x, Cn.s.x, Cn.d.x, Cn.a.x, xn.x, O.box_lo[0], O.box_hi[0]) &&
+                      meets(Co.s.y, Co.d.y, Co.a.y, xo.y, Cn.s.y, Cn.d.y, Cn.a.y, xn.y, O.box_lo[1], O.box_hi[1]) &&
+                      meets(Co.s.z, Co.d.z, Co.a.z, xo.z, Cn.s.z, Cn.d.z, Cn.a.z, xn.z, O.box_lo[2], O.box_hi[2]);
+    return near ? 0xffu : 0u;
+  }
+}
+
+// The face that a segment hits first (first_hit), and the face itself.
+template <bool GRID>
+__device__ __forceinline__ bool hit_face(const ObsView& O, f3 op, f3 np, float dt_d, f3& n, f3& v0) {
+  if constexpr (!GRID) {
+    for (uint32_t f = 0; f < O.n_faces; ++f) {
+      const ObsFace F = uniform_face(O, f);
+      if (face_hit(F, op, np, dt_d)) {
+        n = f3{F.n[0], F.n[1], F.n[2]};
+        v0 = f3{F.v0[0], F.v0[1], F.v0[2]};
+        return true;
+      }
+    }
+    return false;
+  } else {
+    const int32_t hit = first_hit(O, op, np, dt_d);
+    if (hit < 0) return false;
+    const ObsFace& F = O.faces[hit];
+    n = f3{F.n[0], F.n[1], F.n[2]};
+    v0 = f3{F.v0[0], F.v0[1], F.v0[2]};
+    return true;
+  }
+}
+
+// `steps` steps of every body, one thread per body, the record in registers from the first to the last
+// (bodies do not interact) and stored in place: the 13 fields that change, and the others only where
+// they hold something else than what the reference leaves there.  Bound by vector issue (~1,400
+// operations a body-step in free fall): 1,048,576 cubes 30 us a step falling and 44 lying on a floor,
+// where a launch per step, the record through memory each time and eight obstacle searches a body took
+// 71 and 74; 131,072 cubes 4.7 and 7.7 (15.4 and 18.3); below ~20,000, one wave's chain, 3.5 and 5.5.
+template <bool GRID>
+__global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ rec, uint32_t n, uint32_t pitch,
+                                                             RigidParams P, ObsView O, uint32_t steps) {
   const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
   if (b >= n) return;
-  float S[kRigidRecord], T[kRigidRecord], K[kRigidRecord], A[kRigidRecord];
-  // field-major records: each field is one coalesced wavefront load
-#pragma unroll
-  for (int k = 0; k < kRigidRecord; ++k) S[k] = in[(size_t)k * pitch + b];
-  // accumulate_forces, accumulate_torques
-  S[23] = S[23] + P.gravity.x; S[24] = S[24] + P.gravity.y; S[25] = S[25] + P.gravity.z;
-  S[26] = S[26] + P.torque.x; S[27] = S[27] + P.torque.y; S[28] = S[28] + P.torque.z;
+  // one coalesced wavefront access: a uniform base per field and a 32-bit byte offset per lane
+  auto field = [&](int k) -> float& { return *(float*)((char*)(rec + (size_t)k * pitch) + b * 4u); };
+  Body S{f3{field(0), field(1), field(2)}, Q{field(6), f3{field(3), field(4), field(5)}},
+         f3{field(7), field(8), field(9)}, f3{field(10), field(11), field(12)}};
+  float m = field(13);
+  M3 I{{f3{field(14), field(15), field(16)}, f3{field(17), field(18), field(19)}, f3{field(20), field(21), field(22)}}};
+  f3 F = f3{field(23), field(24), field(25)}, tau = f3{field(26), field(27), field(28)};
+  // cleared at the end of every step: stored only where the record holds something else
+  auto bits = [](f3 v) { return __float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z); };
+  if (steps != 0 && (bits(F) | bits(tau)) != 0u)
+    for (int k = 23; k < kRigidRecord; ++k) field(k) = 0.0f;
   const float h = P.dt;
-  if (P.integration == FP_EULER) {  // S + S' h (state.rs:75-83)
-    derivative(S, K);
-#pragma unroll
-    for (int k = 0; k < kRigidRecord; ++k) T[k] = S[k] + K[k] * h;
-  } else {  // state.rs:86-106, delta accumulated left to right
-    const float hh = h * 0.5f, h6 = h / 6.0f, h3 = h / 3.0f;
-    derivative(S, K);
-#pragma unroll
-    for (int k = 0; k < kRigidRecord; ++k) { A[k] = h6 * K[k]; T[k] = S[k] + K[k] * hh; }
-    derivative(T, K);
-#pragma unroll
-    for (int k = 0; k < kRigidRecord; ++k) { A[k] = A[k] + h3 * K[k]; T[k] = S[k] + K[k] * hh; }
-    derivative(T, K);
-#pragma unroll
-    for (int k = 0; k < kRigidRecord; ++k) { A[k] = A[k] + h3 * K[k]; T[k] = S[k] + K[k] * h; }
-    derivative(T, K);
-#pragma unroll
-    for (int k = 0; k < kRigidRecord; ++k) { A[k] = A[k] + h6 * K[k]; T[k] = S[k] + A[k]; }
-  }
-  // normalize_rotation: q * (1 / sqrt(s s + v . v))
-  {
-    const float inv = 1.0f / __builtin_sqrtf(T[6] * T[6] + ((T[3] * T[3] + T[4] * T[4]) + T[5] * T[5]));
-    T[3] = T[3] * inv; T[4] = T[4] * inv; T[5] = T[5] * inv; T[6] = T[6] * inv;
-  }
-  // update_state: the cube's vertices against the obstacles
-  if (O.n_faces != 0) {
-    const M3 R_old = from_quat(rot(S)), R_new = from_quat(rot(T));
-    const f3 x_old = f3{S[0], S[1], S[2]}, x_new = f3{T[0], T[1], T[2]};
-    const M3 I_old = inertia_inv(S);
-    const float m = S[13];
-    const f3 vel = f3{S[7] / m, S[8] / m, S[9] / m};
-    const f3 w = mv(I_old, f3{S[10], S[11], S[12]});
-    for (int k = 0; k < 8; ++k) {
-      const f3 c = f3{kCubeCorner[k][0], kCubeCorner[k][1], kCubeCorner[k][2]};
-      const f3 op = add(mv(R_old, c), x_old), np = add(mv(R_new, c), x_new);
-      const int32_t hit = first_hit(O, op, np, P.dt_d);
-      if (hit < 0) continue;
-      const ObsFace& f = O.faces[hit];
-      const f3 nrm = f3{f.n[0], f.n[1], f.n[2]}, v0 = f3{f.v0[0], f.v0[1], f.v0[2]};
-      const float od = dot(sub(op, v0), nrm), nd = dot(sub(np, v0), nrm);
-      const f3 r = sub(op, x_old);
-      const float frac = od / (od - nd);
-      const f3 cv = add(vel, cross(w, r));
-      const f3 cp = add(op, smul(P.dt * frac, cv));
-      const float vn = dot(cv, nrm);
-      const float j = (-(1.0f + P.restitution) * vn) / (1.0f / m + dot(nrm, mv(I_old, cross(cross(r, nrm), r))));
-      const f3 imp = smul(j, nrm);
-      const f3 pos = add(sub(cp, r), smul(0.0001f * 2.0f, nrm));  // consts::EPSILON * 2.0
-      T[0] = pos.x; T[1] = pos.y; T[2] = pos.z;
-      T[7] = T[7] + imp.x; T[8] = T[8] + imp.y; T[9] = T[9] + imp.z;  // apply_impulse (:38-41)
-      const f3 dl = cross(r, imp);
-      T[10] = T[10] + dl.x; T[11] = T[11] + dl.y; T[12] = T[12] + dl.z;
+  for (uint32_t step = 0; step < steps; ++step) {
+    // accumulate_forces, accumulate_torques
+    F = add(F, P.gravity);
+    tau = add(tau, P.torque);
+    Body T;
+    f3 dx;
+    Q dq;
+    derivative(S, m, I, dx, dq);
+    const f3 z = f3{0.0f, 0.0f, 0.0f};
+    if (P.integration == FP_EULER) {  // S + S' h (state.rs:75-83)
+      T = Body{axpy(S.x, h, dx), axpy(S.q, h, dq), axpy(S.p, h, F), axpy(S.l, h, tau)};
+    } else {  // state.rs:86-106, delta accumulated left to right
+      const float hh = h * 0.5f, h6 = h / 6.0f, h3 = h / 3.0f;
+      f3 ax = smul(h6, dx);
+      Q aq = Q{h6 * dq.s, smul(h6, dq.v)};
+      T = Body{axpy(S.x, hh, dx), axpy(S.q, hh, dq), axpy(S.p, hh, F), axpy(S.l, hh, tau)};
+      settle(T); settle(ax); settle(aq);
+      derivative_later(T, m, I, dx, dq);
+      ax = axpy(ax, h3, dx);
+      aq = axpy(aq, h3, dq);
+      T = Body{axpy(S.x, hh, dx), axpy(S.q, hh, dq), axpy(S.p, hh, add(F, z)), axpy(S.l, hh, add(tau, z))};
+      settle(T); settle(ax); settle(aq);
+      derivative_later(T, m, I, dx, dq);
+      ax = axpy(ax, h3, dx);
+      aq = axpy(aq, h3, dq);
+      T = Body{axpy(S.x, h, dx), axpy(S.q, h, dq), axpy(S.p, h, add(F, z)), axpy(S.l, h, add(tau, z))};
+      settle(T); settle(ax); settle(aq);
+      derivative_later(T, m, I, dx, dq);
+      ax = axpy(ax, h6, dx);
+      aq = axpy(aq, h6, dq);
+      const f3 F2 = add(F, z), tau2 = add(tau, z);
+      const f3 ap = axpy(axpy(axpy(smul(h6, F), h3, F2), h3, F2), h6, F2);
+      const f3 al = axpy(axpy(axpy(smul(h6, tau), h3, tau2), h3, tau2), h6, tau2);
+      T = Body{add(S.x, ax), Q{S.q.s + aq.s, add(S.q.v, aq.v)}, add(S.p, ap), add(S.l, al)};
+      settle(T);
+    }
+    // normalize_rotation: q * (1 / sqrt(s s + v . v))
+    {
+      float root, inv;
+      sqrt_rcp_rn(T.q.s * T.q.s + dot(T.q.v, T.q.v), root, inv);
+      T.q = Q{T.q.s * inv, f3{T.q.v.x * inv, T.q.v.y * inv, T.q.v.z * inv}};
+    }
+    // update_state: the cube's vertices against the obstacles
+    if (O.n_faces != 0) {
+      uint32_t near = may_hit<GRID>(O, corners_of(from_quat(S.q)), S.x, corners_of(from_quat(T.q)), T.x);
+      if (near != 0) {
+        // the corners are formed again (opaque rotations), not held across the test above
+        Q q_old = S.q, q_new = T.q;
+        settle(q_old);
+        settle(q_new);
+        const Corners Co = corners_of(from_quat(q_old)), Cn = corners_of(from_quat(q_new));
+        const f3 x_new = T.x;
+        // what the response needs of the old pose: once for the few-face scenes, whose marked corners mostly
+        // hit, and per hit with the grids, where the search needs the registers
+        M3 I_old;
+        f3 vel, w;
+        auto pose = [&] {
+          I_old = inertia_inv(q_old, I);
+          vel = ExactMath::div3(S.p, m);
+          w = mv(I_old, S.l);
+        };
+        if (!GRID) pose();
+        // each lane its own marked corners in ascending order: as many rounds as the body with the most
+        // has, not eight
+        while (near != 0) {
+          const uint32_t k = (uint32_t)__builtin_ctz(near);
+          near &= near - 1u;
+          const f3 op = corner_of_lane(Co, S.x, k), np = corner_of_lane(Cn, x_new, k);
+          f3 nrm, v0;
+          if (!hit_face<GRID>(O, op, np, P.dt_d, nrm, v0)) continue;
+          if (GRID) {
+            settle(q_old);
+            pose();
+          }
+          const float od = dot(sub(op, v0), nrm), nd = dot(sub(np, v0), nrm);
+          const f3 r = sub(op, S.x);
+          const float frac = od / (od - nd);
+          const f3 cv = add(vel, cross(w, r));
+          const f3 cp = add(op, smul(P.dt * frac, cv));
+          const float vn = dot(cv, nrm);
+          const float j = (-(1.0f + P.restitution) * vn) / (1.0f / m + dot(nrm, mv(I_old, cross(cross(r, nrm), r))));
+          const f3 imp = smul(j, nrm);
+          T.x = add(sub(cp, r), smul(0.0001f * 2.0f, nrm));  // consts::EPSILON * 2.0
+          T.p = add(T.p, imp);  // apply_impulse (:38-41)
+          T.l = add(T.l, cross(r, imp));
+        }
+      }
+    }
+    S = T;
+    // clear_forces, clear_torques
+    F = tau = f3{0.0f, 0.0f, 0.0f};
+    if (step == 0) {  // a -0 of the record among the constant fields becomes +0
+      auto plus = [&](int k, float& v) {
+        const float w = v + 0.0f;
+        if (__float_as_uint(v) != __float_as_uint(w)) field(k) = w;
+        v = w;
+      };
+      plus(13, m);
+      for (int c = 0; c < 3; ++c) {
+        plus(14 + 3 * c, I.c[c].x);
+        plus(15 + 3 * c, I.c[c].y);
+        plus(16 + 3 * c, I.c[c].z);
+      }
     }
   }
-  // clear_forces, clear_torques
-#pragma unroll
-  for (int k = 23; k < kRigidRecord; ++k) T[k] = 0.0f;
-#pragma unroll
-  for (int k = 0; k < kRigidRecord; ++k) out[(size_t)k * pitch + b] = T[k];
+  field(0) = S.x.x; field(1) = S.x.y; field(2) = S.x.z;
+  field(3) = S.q.v.x; field(4) = S.q.v.y; field(5) = S.q.v.z; field(6) = S.q.s;
+  field(7) = S.p.x; field(8) = S.p.y; field(9) = S.p.z;
+  field(10) = S.l.x; field(11) = S.l.y; field(12) = S.l.z;
 }
 
 // Field-major device records <-> the caller's 29-float records, body after body.
@@ -171,11 +351,18 @@ hipError_t launch_rigid_records(const float* in, float* out, uint32_t n, uint32_
   return hipGetLastError();
 }
 
-hipError_t launch_rigid_step(const float* in, float* out, uint32_t n, uint32_t pitch, const RigidParams& p,
-                             const ObsView& obs, hipStream_t s) {
-  if (n == 0) return hipSuccess;
+hipError_t launch_rigid_steps(float* rec, uint32_t n, uint32_t pitch, const RigidParams& p, const ObsView& obs,
+                              uint32_t steps, hipStream_t s) {
+  if (n == 0 || steps == 0) return hipSuccess;
   if (pitch < n) return hipErrorInvalidValue;
-  rigid_step_kernel<<<dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s>>>(in, out, n, pitch, p, obs);
+  constexpr uint32_t kMost = 1u << 28;  // bodies a launch: the kernel's byte offsets are 32 bits
+  for (uint32_t first = 0; first < n; first += kMost) {
+    const uint32_t count = n - first < kMost ? n - first : kMost;
+    const dim3 g((count + kBlock - 1) / kBlock), b(kBlock);
+    if (obs.use_grid) rigid_step_kernel<true><<<g, b, 0, s>>>(rec + first, count, pitch, p, obs, steps);
+    else rigid_step_kernel<false><<<g, b, 0, s>>>(rec + first, count, pitch, p, obs, steps);
+    if (n - first <= kMost) break;
+  }
   return hipGetLastError();
 }
 
