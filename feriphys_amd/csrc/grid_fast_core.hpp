@@ -64,17 +64,14 @@ FP_HD float sqrt_f(float x) {
   return sqrtf(x);
 #endif
 }
-// The correctly rounded square root for every input but subnormals (where it is within one ulp):
-// the hardware square root and the choice among it and its two neighbours by the exact residuals
-// (sqrt_rn of exact_ops.hpp without its range check, which only subnormal and huge inputs need;
-// zero, infinity and NaN come out right through the same selects).
+// The correctly rounded square root of x >= 2^-96 (sqrt_in_range of exact_ops.hpp): the hardware
+// reciprocal root r, g = x r and one Newton step with the exact residual x - g g, four operations where
+// choosing among the hardware root and its two neighbours took eight.  Zero (whose strut or face has no
+// direction anyway) gives NaN, tinier inputs a root within an ulp or two.
 FP_HD float sqrt_cr(float x) {
 #ifdef __HIP_DEVICE_COMPILE__
-  const float s = __builtin_amdgcn_sqrtf(x);
-  const float dn = __uint_as_float(__float_as_uint(s) - 1u), up = __uint_as_float(__float_as_uint(s) + 1u);
-  const float rdn = __builtin_fmaf(-dn, s, x), rup = __builtin_fmaf(-up, s, x);
-  const float t = rdn <= 0.0f ? dn : s;
-  return rup > 0.0f ? up : t;
+  const float r = __builtin_amdgcn_rsqf(x), g = x * r;
+  return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * r, g);
 #else
   return sqrtf(x);
 #endif
@@ -304,7 +301,8 @@ FP_HD f3 phase1(Lds<TR, TC>& L, const StepParams& P, const ClothView& G, int r0,
   f3 f_sh;
   {
     const float dx = L.tab[S::H0 + j].d, dy = L.tab[S::V0 + i].d;
-    const float Ls = sqrt_cr(dx * dx + dy * dy);
+    const float Ls2 = dx * dx + dy * dy;
+    const float Ls = Ls2 > 0.0f ? sqrt_cr(Ls2) : Ls2;  // a cloth of spacing 0 keeps its rest length 0
     const float inv = rcp_f(Ls);
     const f3 f = strut_f(pB, uB, pC, uC, inv * G.sk, inv * G.sc, Ls);
     f_sh = INTERIOR ? f : sel3(quad, f, z);
