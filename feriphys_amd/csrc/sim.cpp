@@ -213,6 +213,8 @@ uint64_t tile_count(const fp::ClothDesc& d, int shape) {
 // against 9.0 up to 128 x 128 vertices, 256 tiles; 8.1 against 9.4 at 192 x 192, 576 tiles); at 256 x
 // 256, 1,024 tiles, both take 9.6, and beyond it the larger tiles' fewer operations win.
 constexpr uint64_t kSmallTiles = 768;
+// Tiles resident at once: six workgroups on each of 256 CUs.
+constexpr uint64_t kResidentTiles = 1536;
 
 // Runs of the tile list per XCD (see xcd_order).
 constexpr size_t kTilePieces = 8;
@@ -256,6 +258,23 @@ int build_block_lists(fp_sim* s) {
   for (const auto& m : s->meshes)
     if (m.host.cloth.valid && m.uniform_mass) n_small += tile_count(m.host.cloth, fp::TILE_8x8);
   const bool small = s->math == FP_MATH_EXACT && n_small <= kSmallTiles;
+  // Meshes of different tile shapes cost a launch per shape and step.  While all their tiles together are
+  // resident at once, a launch is one tile's latency and a second one as long again, so every mesh takes
+  // the shape that most tiles have.
+  const auto launched = [&](int shape) {
+    return s->math == FP_MATH_FAST && shape == fp::TILE_16x16 ? (int)fp::TILE_15x15 : shape;
+  };
+  uint64_t per_shape[fp::N_LAUNCH_SHAPES] = {};
+  for (const auto& m : s->meshes)
+    if (m.host.cloth.valid && m.uniform_mass)
+      per_shape[launched(m.tile_shape)] += tile_count(m.host.cloth, launched(m.tile_shape));
+  int common = 0;
+  for (int sh = 1; sh < fp::N_TILE_SHAPES; ++sh)
+    if (per_shape[sh] > per_shape[common]) common = sh;
+  uint64_t n_common = 0;
+  for (const auto& m : s->meshes)
+    if (m.host.cloth.valid && m.uniform_mass) n_common += tile_count(m.host.cloth, common);
+  const bool one_shape = n_common <= kResidentTiles;
   for (uint32_t mi = 0; mi < s->meshes.size(); ++mi) {
     MeshSlot& ms = s->meshes[mi];
     const bool grid_ok = ms.host.cloth.valid && ms.uniform_mass;
@@ -265,9 +284,8 @@ int build_block_lists(fp_sim* s) {
     ms.tile_begin = ms.tile_end = (uint32_t)all_tiles.size();
     ms.on_patch = false;
     if (ms.kernel == MK_GRID_TILED) {
-      // the fast kernel has one quad per thread: 15x15 and 7x31 tiles (16x16 becomes 15x15)
-      ms.launch_shape = small ? fp::TILE_8x8
-                        : s->math == FP_MATH_FAST && ms.tile_shape == fp::TILE_16x16 ? fp::TILE_15x15 : ms.tile_shape;
+      // (the fast kernel has one quad per thread: 15x15 and 7x31 tiles; 16x16 becomes 15x15)
+      ms.launch_shape = small ? (int)fp::TILE_8x8 : one_shape ? common : launched(ms.tile_shape);
       std::vector<fp::TileRange> mt;
       cloth_tiles(mi, ms.host.cloth, ms.launch_shape, mt);
       by_shape[ms.launch_shape].insert(by_shape[ms.launch_shape].end(), mt.begin(), mt.end());
