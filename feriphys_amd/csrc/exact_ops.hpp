@@ -37,16 +37,22 @@ FP_HD float rcp_rn(float x) {
 // transcendental and four other operations (choosing among the hardware square root and its two
 // neighbours by their residuals took eight); checked on every such input against the full sequence
 // (fp_selftest_exact_math).  Other inputs take the full sequence.
-#ifdef __HIP_DEVICE_COMPILE__
 FP_HD float sqrt_in_range(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
   const float r = __builtin_amdgcn_rsqf(x), g = x * r;
   return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * r, g);
+#else
+  return __builtin_sqrtf(x);
+#endif
 }
 FP_HD float rcp_in_range(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
   const float r = __builtin_amdgcn_rcpf(x);
   return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
-}
+#else
+  return 1.0f / x;
 #endif
+}
 FP_HD float sqrt_rn(float x) {
 #ifdef __HIP_DEVICE_COMPILE__
   if (x >= 0x1p-96f && x <= 3.40282347e38f) return sqrt_in_range(x);

@@ -254,7 +254,7 @@ FP_HD void corner(Lds<TR, TC, ROOM>& L, int k, int e, int lr, int lc) {
   int rn, cn, rp, cp;
   corner_ends(k, rn, cn, rp, cp);
   const int a = lr + 2, b = lc + 2;
-  L.w[k][e] = corner_weight<M>(pos(L, a, b), pos(L, a + rn, b + cn), pos(L, a + rp, b + cp), L.atab);
+  L.w[k][e] = corner_weight<M, true>(pos(L, a, b), pos(L, a + rn, b + cn), pos(L, a + rp, b + cp), L.atab);
 }
 
 // N components, from component q0 on, of vertex (lr, lc)'s force: the reference adds the mesh struts,

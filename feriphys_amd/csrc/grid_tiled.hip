@@ -155,7 +155,7 @@ __device__ __forceinline__ void gather_vertex(gtile::Lds<TR, TC, CONSTANTS>& L, 
   auto face = [&](int k, const float* f) {
     int rn, cn, rp, cp;
     gtile::corner_ends(k, rn, cn, rp, cp);
-    const float w = corner_weight<M>(p, pos(rn, cn), pos(rp, cp), L.atab);
+    const float w = corner_weight<M, true>(p, pos(rn, cn), pos(rp, cp), L.atab);
     F = add(F, f3{w * f[0], w * f[S::QC], w * f[2 * S::QC]});
     settle();
   };

@@ -19,13 +19,20 @@ __device__ __forceinline__ void store_state(const SoA& o, uint32_t i, f3 x, f3 v
 }
 
 // Integration, collision and pins: the tail of Simulation::step for one vertex
-// (springy/simulation.rs:145-155 -> state.rs, springy_mesh.rs:423-497).
+// (springy/simulation.rs:145-155 -> state.rs, springy_mesh.rs:423-497).  `scanned`: a copy in LDS of the
+// faces of an obstacle that is scanned face by face, or nullptr.
 template <class M>
 __device__ __forceinline__ void finish_step(const StepArgs& A, const StepParams& P, uint32_t i, float m, f3 p, f3 v,
-                                            f3 F, bool pin) {
+                                            f3 F, bool pin, const ObsFace* scanned = nullptr) {
   f3 xn, vn;
   integrate<M>(P, m, p, v, F, xn, vn);
-  int32_t hit = first_hit(A.obs, p, xn, P.dt_d);
+  int32_t hit = -1;
+  if (scanned != nullptr) {
+    for (uint32_t f = 0; f < A.obs.n_faces && hit < 0; ++f)
+      if (face_hit(load_face(scanned, f), p, xn, P.dt_d)) hit = (int32_t)f;
+  } else {
+    hit = first_hit(A.obs, p, xn, P.dt_d);
+  }
   if (hit >= 0) collide_response(A.obs.faces[hit], P, m, p, v, F, xn, vn);
   if (pin) { xn = p; vn = v; }  // pinned points keep their pre-step record (:492-496)
   store_state(A.out, i, xn, vn);
@@ -102,10 +109,73 @@ __global__ void __launch_bounds__(kBlock) csr_kernel(StepArgs A, CsrView T, cons
   finish_step<M>(A, P, i, m, p, v, F, pin);
 }
 
+// N struts (corners) of one vertex abreast: the forms that hold for ordinary lengths for all of them at
+// once, and the general ones for all where some lane needs them.
+template <class M, int N>
+__device__ __forceinline__ void strut_group(f3 p, f3 v, const PatchStrut* se, const float2* cls, const float4* pos,
+                                            const float2* vel, f3* a, f3* b) {
+  f3 d[N], dv[N];
+  float d2[N], len[N], inv[N];
+  uint32_t far = 0;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float4 q = pos[se[j].loc];
+    const float2 r = vel[se[j].loc];
+    d[j] = sub(f3{q.x, q.y, q.z}, p);
+    dv[j] = sub(f3{q.w, r.x, r.y}, v);
+    d2[j] = dot(d[j], d[j]);  // unfused: see strut_accumulate
+    len[j] = sqrt_in_range(d2[j]);
+    inv[j] = M::kExact ? rcp_in_range(len[j]) : M::rcp(len[j]);
+    const uint32_t over = __float_as_uint(d2[j]) - __float_as_uint(0x1p-96f);
+    far = over > far ? over : far;
+  }
+  if (far > __float_as_uint(0x1p96f) - __float_as_uint(0x1p-96f)) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if constexpr (M::kExact) {
+        M::sqrt_rcp(d2[j], len[j], inv[j]);
+      } else {
+        len[j] = sqrt_rn(d2[j]);
+        inv[j] = M::rcp(len[j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float2 kc = cls[se[j].cls()];
+    const float il = rcp_in_range(se[j].len);
+    strut_from<M>(d[j], len[j], inv[j], dv[j], il * kc.x, il * kc.y, se[j].len, a[j], b[j]);
+  }
+}
+template <class M, int N, class PL>
+__device__ __forceinline__ void corner_group(f3 p, const PatchCorner* ce, const float4* ffs, const float (*tab)[4],
+                                             PL Pl, f3* a) {
+  float w[N], n2[N], d[N];
+  bool ok = true;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {  // corner_weight
+    const f3 ea = sub(Pl(ce[j].prev()), p), eb = sub(Pl(ce[j].next()), p);
+    const f3 x = cross(ea, eb);
+    n2[j] = M::dot(x, x);
+    d[j] = M::dot(ea, eb);
+    ok = M::template corner_in_range<true>(n2[j], d[j], w[j], tab) && ok;
+  }
+  if (!ok) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) w[j] = M::div_pi(M::atan2_(M::sqrt_(n2[j]), d[j]));
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const float4 ff = ffs[ce[j].face()];
+    a[j] = f3{w[j] * ff.x, w[j] * ff.y, w[j] * ff.z};
+  }
+}
+
 // The step of one patch of a general mesh per workgroup (the operations of face_kernel and
 // csr_kernel, in the same order per vertex):
-//   phase 0  stage the states of the patch and its halo in LDS with one pass of loads, and the
-//            mesh's table of nominal strut constants;
+//   phase 0  stage the states of the patch and its halo in LDS with one pass of loads, the mesh's
+//            table of nominal strut constants, the corner weights' reduction table and the faces of
+//            an obstacle small enough to be scanned;
 //   phase 1  drag + lift of every face with a corner in the patch into LDS (a face on the patch
 //            border is computed by each patch that holds one of its corners);
 //   phase 2  every patch vertex: struts in strut order (8-byte entries, neighbour states from LDS),
@@ -113,53 +183,116 @@ __global__ void __launch_bounds__(kBlock) csr_kernel(StepArgs A, CsrView T, cons
 //            face's drag + lift; integrate, collide, pin, store.
 // LDS: the staged states as (x, y, z, vx) and (vy, vz) at fixed strides (one address per
 // neighbour, two wide reads), and the face forces sized per launch, nf_cap float4.
+//
+// The entries' places follow from the patch record alone and their number is the slice's, so the
+// first ones are asked for together with the states, each later group while the one before it is
+// computed.  The groups that every lane of a wavefront has (all but a few vertices', on a regular
+// surface) run without masks, two abreast; what a slice's larger vertices have beyond is masked.
+//
+// Bound by the lanes' arithmetic (1,877 vector instructions a vertex in exact arithmetic, 684 of them
+// the 12 struts', 606 the six corners') with five workgroups at most on a CU, and on one mesh alone by
+// one wavefront's chain.  281,000 vertices in eight meshes, exact: 20.7 us a step, 24.3 when the strut
+// and corner entries (8 bytes each then) were looked up per vertex and waited for; fast 17.4 and 19.2.
+// 40,962 vertices: 9.6 and 12.4, fast 7.9 and 9.8.  Tried: four or six struts abreast or all entries
+// loaded up front 21.3 to 24, four lanes a vertex 34.7 (9.1 against 9.6 on 642 vertices), patches of 128
+// vertices 24.1.
 template <class M>
 __global__ void __launch_bounds__(kBlock) patch_kernel(StepArgs A, CsrView T, const PatchRange* __restrict__ patches) {
+  constexpr uint32_t kStruts = 2, kCorners = 2;  // a lane's at a time
   __shared__ float4 s_p[kPatchLocal];  // x, y, z, vx
   __shared__ float2 s_w[kPatchLocal];  // vy, vz
   __shared__ float2 s_cls[kPatchClasses];
+  __shared__ float4 s_obs[4 * kScanFaces];
+  __shared__ alignas(16) float s_atan[kFdlEntries][4];
   extern __shared__ float4 s_ff[];     // per patch face: drag + lift
-  const PatchRange R = patches[blockIdx.x];
-  const uint32_t np = R.end - R.begin, nl = np + R.n_halo;
+  const uint32_t t = threadIdx.x;
+  const PatchRange* R = patches + blockIdx.x;
+  const uint32_t begin = R->begin, np = R->end - begin, nl = np + R->n_halo, mesh = R->mesh, n_faces = R->n_faces;
   const SoA& S = A.in;
-  const StepParams P = A.params[R.mesh];
-  if (threadIdx.x < kPatchClasses) s_cls[threadIdx.x] = T.p_cls[R.mesh * kPatchClasses + threadIdx.x];
-  for (uint32_t e = threadIdx.x; e < nl; e += kBlock) {
-    const uint32_t g = e < np ? R.begin + e : T.halo[R.halo_begin + (e - np)];
-    s_p[e] = make_float4(S.x[g], S.y[g], S.z[g], S.vx[g]);
-    s_w[e] = make_float2(S.vy[g], S.vz[g]);
+  const StepParams P = A.params[mesh];
+  // the lane's slice and, of its entries, the first ones
+  const uint32_t w = __builtin_amdgcn_readfirstlane(t / kSlice);
+  const uint32_t s_min = R->s_min[w], s_max = R->s_max[w], f_min = R->f_min[w], f_max = R->f_max[w];
+  const PatchStrut* ent = T.p_ent + (R->s_base[w] + t % kSlice);
+  const PatchCorner* cor = T.p_corner + (R->f_base[w] + t % kSlice);
+  const PatchFace* faces = T.patch_faces + R->face_begin;
+  const uint32_t* halo = T.halo + R->halo_begin;
+  auto entry = [](uint32_t j, uint32_t n) { return kSlice * (j < n ? j : n ? n - 1 : 0u); };
+  constexpr uint32_t kRounds = kPatchLocal / kBlock;
+  uint32_t g[kRounds];
+#pragma unroll
+  for (uint32_t r = 0; r < kRounds; ++r) {
+    const uint32_t e = t + r * kBlock;
+    g[r] = e < np || e >= nl ? begin + (e < np ? e : 0u) : halo[e - np];
   }
+  PatchStrut se[kStruts];
+  PatchCorner ce[kCorners];
+#pragma unroll
+  for (uint32_t j = 0; j < kStruts; ++j) se[j] = ent[entry(j, s_max)];
+#pragma unroll
+  for (uint32_t j = 0; j < kCorners; ++j) ce[j] = cor[entry(j, f_max)];
+  PatchFace pf = faces[t < n_faces ? t : 0u];
+  const uint32_t i = begin + (t < np ? t : np - 1);
+  const float m = P.uniform_mass ? P.mass : A.mass[i];
+  const bool pin = pinned(A.pins, i);
+#pragma unroll
+  for (uint32_t r = 0; r < kRounds; ++r) {
+    const uint32_t e = t + r * kBlock;
+    const float4 a = make_float4(S.x[g[r]], S.y[g[r]], S.z[g[r]], S.vx[g[r]]);
+    const float2 b = make_float2(S.vy[g[r]], S.vz[g[r]]);
+    if (e < nl) {
+      s_p[e] = a;
+      s_w[e] = b;
+    }
+  }
+  if (t < kPatchClasses) s_cls[t] = T.p_cls[mesh * kPatchClasses + t];
+  const bool scan = !A.obs.use_grid && A.obs.n_faces <= kScanFaces;
+  if (scan && t < 4 * A.obs.n_faces) s_obs[t] = reinterpret_cast<const float4*>(A.obs.faces)[t];
+  if (M::kExact && t < kFdlEntries) fdl_entry(t, s_atan[t]);
   __syncthreads();
   auto Pl = [&](uint32_t l) { const float4 a = s_p[l]; return f3{a.x, a.y, a.z}; };
   auto Vl = [&](uint32_t l) { const float4 a = s_p[l]; const float2 b = s_w[l]; return f3{a.w, b.x, b.y}; };
-  for (uint32_t q = threadIdx.x; q < R.n_faces; q += kBlock) {
-    const PatchFace pf = T.patch_faces[R.face_begin + q];
-    const f3 sum = face_force<M>(Pl(pf.v[0]), Pl(pf.v[1]), Pl(pf.v[2]), Vl(pf.v[0]), Vl(pf.v[1]), Vl(pf.v[2]), P);
-    s_ff[q] = make_float4(sum.x, sum.y, sum.z, 0.0f);
+  for (uint32_t k = t; k < n_faces; k += kBlock) {
+    const PatchFace next = faces[k + kBlock < n_faces ? k + kBlock : k];
+    const uint32_t a = pf.v(0), b = pf.v(1), c = pf.v(2);
+    const f3 sum = face_force<M>(Pl(a), Pl(b), Pl(c), Vl(a), Vl(b), Vl(c), P);
+    s_ff[k] = make_float4(sum.x, sum.y, sum.z, 0.0f);
+    pf = next;
   }
   __syncthreads();
-  if (threadIdx.x >= np) return;
-  const uint32_t t = threadIdx.x, i = R.begin + t;
+  if (t >= np) return;
   const f3 p = Pl(t), v = Vl(t);
-  const float m = P.uniform_mass ? P.mass : A.mass[i];
   f3 F = A.force_init ? f3{A.fx[i], A.fy[i], A.fz[i]} : f3{0.0f, 0.0f, 0.0f};
   F = add(F, P.gravity);  // apply_external_point_forces (:527-531)
+
   // apply_strut_forces (:533-551), in strut order; each strut's stiffness and damping rebuilt as
   // Strut::new makes them, (1.0 / len) * nominal (:83-84)
   {
-    const PatchStrut* ent = T.p_ent + T.s_first[i];
-    const uint32_t ns = T.s_cnt[i];
-    for (uint32_t e = 0; e < ns; e += 4) {
-      PatchStrut se[4];
+    uint32_t e = 0;
+#pragma unroll 1
+    for (; e + kStruts <= s_min; e += kStruts) {
+      PatchStrut next[kStruts];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) se[j] = ent[kSlice * (e + j < ns ? e + j : e)];
+      for (uint32_t j = 0; j < kStruts; ++j) next[j] = ent[entry(e + kStruts + j, s_max)];
+      f3 a[kStruts], b[kStruts];
+      strut_group<M, kStruts>(p, v, se, s_cls, s_p, s_w, a, b);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (e + j < ns) {
-          const float2 kc = s_cls[se[j].cls];
-          const float il = rcp_rn(se[j].len);
-          strut_accumulate<M>(F, p, v, Pl(se[j].loc), Vl(se[j].loc), il * kc.x, il * kc.y, se[j].len);
+      for (uint32_t k = 0; k < kStruts; ++k) F = add(add(F, a[k]), b[k]);
+#pragma unroll
+      for (uint32_t j = 0; j < kStruts; ++j) se[j] = next[j];
+    }
+    if (e < s_max) {
+      PatchStrut re = ent[entry(e, s_max)];
+#pragma unroll 1
+      while (e < s_max) {
+        const PatchStrut next = ent[entry(++e, s_max)];
+        if (re.valid()) {
+          const float2 kc = s_cls[re.cls()];
+          const float il = rcp_rn(re.len);
+          strut_accumulate<M>(F, p, v, Pl(re.loc), Vl(re.loc), il * kc.x, il * kc.y, re.len);
         }
+        re = next;
+      }
     }
   }
   // apply_torsional_forces, when the step includes it (see csr_kernel)
@@ -178,24 +311,35 @@ __global__ void __launch_bounds__(kBlock) patch_kernel(StepArgs A, CsrView T, co
   // apply_face_forces (:629-654): in face order, this vertex's corner weight (vertex_angle / PI,
   // :647-649) times the face's drag + lift (:650-652)
   {
-    const PatchCorner* cor = T.p_corner + T.f_first[i];
-    const uint32_t nf = T.f_cnt[i];
-    for (uint32_t j = 0; j < nf; j += 4) {
-      PatchCorner ce[4];
+    uint32_t e = 0;
+#pragma unroll 1
+    for (; e + kCorners <= f_min; e += kCorners) {
+      PatchCorner next[kCorners];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) ce[k] = cor[kSlice * (j + k < nf ? j + k : j)];
+      for (uint32_t j = 0; j < kCorners; ++j) next[j] = cor[entry(e + kCorners + j, f_max)];
+      f3 a[kCorners];
+      corner_group<M, kCorners>(p, ce, s_ff, s_atan, Pl, a);
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (j + k < nf) {
-          const float w = corner_weight<M>(p, Pl(ce[k].next), Pl(ce[k].prev));
-          const float4 ff = s_ff[ce[k].q];
-          F = add(F, f3{w * ff.x, w * ff.y, w * ff.z});
+      for (uint32_t k = 0; k < kCorners; ++k) F = add(F, a[k]);
+#pragma unroll
+      for (uint32_t j = 0; j < kCorners; ++j) ce[j] = next[j];
+    }
+    if (e < f_max) {
+      PatchCorner re = cor[entry(e, f_max)];
+#pragma unroll 1
+      while (e < f_max) {
+        const PatchCorner next = cor[entry(++e, f_max)];
+        if (re.valid()) {
+          f3 a;
+          corner_group<M, 1>(p, &re, s_ff, s_atan, Pl, &a);
+          F = add(F, a);
         }
+        re = next;
+      }
     }
   }
-  const bool pin = pinned(A.pins, i);
   if (pin) F = f3{0.0f, 0.0f, 0.0f};  // (:522-524)
-  finish_step<M>(A, P, i, m, p, v, F, pin);
+  finish_step<M>(A, P, i, m, p, v, F, pin, scan ? reinterpret_cast<const ObsFace*>(s_obs) : nullptr);
 }
 
 // Drag + lift (springy_mesh.rs:631-646) and the three corner weights angle / PI (:647-649) of every
@@ -497,9 +641,9 @@ __global__ void __launch_bounds__(kBlock) selftest_kernel(unsigned long long* __
     const float ys[2] = {1.0f, -1.7f};
     for (int j = 0; j < 2; ++j) b[3] += differ(fdlibm_atan2f(ys[j], x), fdlibm_atan2f_ref(ys[j], x));
     float w;
-    if (ExactMath::corner_in_range(1.0f, x, w, tab)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
-    if (ExactMath::corner_in_range(1.0f, x, w)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
-    if (x >= 0.0f && ExactMath::corner_in_range(x, -0.37f, w))
+    if (ExactMath::corner_in_range<true>(1.0f, x, w, tab)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
+    if (ExactMath::corner_in_range<false>(1.0f, x, w, nullptr)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
+    if (x >= 0.0f && ExactMath::corner_in_range<false>(x, -0.37f, w, nullptr))
       b[3] += differ(w, fdlibm_atan2f_ref(__builtin_sqrtf(x), -0.37f) / pi);
     const float sr = __builtin_sqrtf(x);
     float root, inv;
@@ -519,7 +663,7 @@ hipError_t launch_patches(const StepArgs& a, const CsrView& t, const PatchRange*
                           uint32_t nf_cap, bool exact, hipStream_t s) {
   if (n_patches == 0) return hipSuccess;
   if (nf_cap > kPatchFaceCap) return hipErrorInvalidValue;
-  const size_t lds = sizeof(float4) * (size_t)nf_cap;
+  const size_t lds = sizeof(float4) * (size_t)(nf_cap ? nf_cap : 1);
   if (exact) patch_kernel<ExactMath><<<dim3(n_patches), dim3(kBlock), lds, s>>>(a, t, patches);
   else patch_kernel<FastMath><<<dim3(n_patches), dim3(kBlock), lds, s>>>(a, t, patches);
   return hipGetLastError();

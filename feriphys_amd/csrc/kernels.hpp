@@ -27,33 +27,49 @@ struct HingeEnt {
   float k, c, rest, pad;
 };
 
+constexpr uint32_t kSlice = 64;  // device vertices whose entries are interleaved (see CsrView)
+
 // One workgroup of the patch kernel: device vertices [begin, end) of mesh `mesh` (a connected patch
 // of at most kBlock vertices), its halo, halo[halo_begin .. halo_begin + n_halo) (every vertex
 // outside the patch that a patch vertex's struts or faces reach; patch plus halo is at most
 // kPatchLocal), and its faces, patch_faces[face_begin .. face_begin + n_faces) (every face with a
-// corner in the patch, at most kPatchFaceCap).
+// corner in the patch, at most kPatchFaceCap).  Per slice of the patch: where its strut and face
+// entries begin and the smallest and the largest number of them that a vertex has (s_min 0 as well
+// where a strut's length or its inverse is not a normal number); a patch of fewer slices repeats
+// the first.
 struct PatchRange {
   uint32_t mesh, begin, end, halo_begin, n_halo, face_begin, n_faces, pad;
+  uint32_t s_base[4], s_min[4], s_max[4], f_base[4], f_min[4], f_max[4];
 };
 constexpr uint32_t kPatchLocal = 512;
 constexpr uint32_t kPatchFaceCap = 2048;
-// A face of a patch: its corners' indices in the patch's LDS copy.
-struct alignas(8) PatchFace {
-  uint16_t v[3], pad;
+// A face of a patch: its corners' indices in the patch's LDS copy, nine bits each.
+struct PatchFace {
+  uint32_t bits;
+  __host__ __device__ uint32_t v(int c) const { return bits >> (9 * c) & 511u; }
 };
 // A face corner of a patch vertex (one per face entry of the vertex, in face-index order): the
-// face's index in its patch's face list and the LDS indices of the face's next and previous
-// corners, the operands of Face::vertex_angle for this corner.
-struct alignas(8) PatchCorner {
-  uint16_t q, next, prev, pad;
+// face's index in its patch's face list (11 bits) and the LDS indices of the face's next and previous
+// corners (9 bits each), the operands of Face::vertex_angle for this corner.  The entries that fill a
+// slice up are zero and not valid.
+struct PatchCorner {
+  uint32_t bits;
+  __host__ __device__ uint32_t face() const { return bits & 2047u; }
+  __host__ __device__ uint32_t next() const { return bits >> 11 & 511u; }
+  __host__ __device__ uint32_t prev() const { return bits >> 20 & 511u; }
+  __host__ __device__ bool valid() const { return bits >> 31; }
 };
+static_assert(kPatchLocal <= 512 && kPatchFaceCap <= 2048, "packed indices");
 // A strut entry of a patch vertex (8 bytes): the rest length, the neighbour's index in the patch's
 // LDS copy and the strut's class, an index into its mesh's table of nominal (stiffness, damping)
 // pairs.  Strut::new scales both by NOMINAL_STRUT_LENGTH / length = 1.0 / len
-// (springy_mesh.rs:74-90), so the kernel recomputes them bit for bit as (1.0 / len) * nominal.
+// (springy_mesh.rs:74-90), so the kernel recomputes them bit for bit as (1.0 / len) * nominal.  The
+// entries that fill a slice up have length 1 and are not valid.
 struct alignas(8) PatchStrut {
   float len;
-  uint16_t loc, cls;
+  uint16_t loc, flags;
+  __host__ __device__ uint32_t cls() const { return flags & 0x7fffu; }
+  __host__ __device__ bool valid() const { return flags >> 15; }
 };
 constexpr uint32_t kPatchClasses = 16;  // classes per mesh; a mesh with more stays on the CSR kernel
 
@@ -61,7 +77,6 @@ constexpr uint32_t kPatchClasses = 16;  // classes per mesh; a mesh with more st
 // a sliced layout: the vertices of one mesh are cut into slices of kSlice consecutive ids (one
 // wavefront), and entry j of a vertex is at first[v] + kSlice * j, so that one load instruction of
 // a wavefront reads kSlice consecutive entries.
-constexpr uint32_t kSlice = 64;
 struct CsrView {
   const uint32_t* s_first;  // per vertex: its strut entries, in strut-index order
   const uint32_t* s_cnt;
@@ -179,5 +194,6 @@ hipError_t launch_unpack_records(const float* in, const uint32_t* pos, uint32_t 
                                  float* mass, float* fx, float* fy, float* fz, RecordScan* scan, hipStream_t s);
 
 constexpr uint32_t kBlock = 256;
+static_assert(kBlock <= 4 * kSlice, "slices of a patch");
 
 }  // namespace fp

@@ -191,7 +191,7 @@ int upload_obstacles(ObstacleSet& s, const std::vector<fp::HostObstacle>& obstac
     s.hit_box.lo[k] = -INFINITY;
     s.hit_box.hi[k] = INFINITY;
   }
-  if (faces.size() <= 8) return FP_OK;  // scan every face in order
+  if (faces.size() <= fp::kScanFaces) return FP_OK;  // scan every face in order
 
   std::vector<uint32_t> always, ids[4];
   for (uint32_t f = 0; f < faces.size(); ++f) {

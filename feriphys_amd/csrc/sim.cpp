@@ -522,7 +522,7 @@ int build_incidence(fp_sim* s) {
   std::vector<uint16_t> sloc(n_sent + 1, 0);
   std::vector<uint32_t> halo;
   std::vector<fp::PatchFace> pfaces;
-  std::vector<fp::PatchCorner> pcorner(n_fent + 1, fp::PatchCorner{0, 0, 0, 0});
+  std::vector<fp::PatchCorner> pcorner(n_fent + fp::kSlice, fp::PatchCorner{0});
   std::vector<int32_t> mark(N, -1);
   for (uint32_t mi = 0; mi < s->meshes.size(); ++mi) {
     auto& ms_ = s->meshes[mi];
@@ -540,7 +540,12 @@ int build_incidence(fp_sim* s) {
     std::vector<uint8_t> fseen(ms_.patch_ok ? h.n_faces() : 0, 0);
     for (size_t b = 0; b + 1 < ms_.bstart.size(); ++b) {
       const uint32_t b0 = (uint32_t)ms_.vbase + ms_.bstart[b], b1 = (uint32_t)ms_.vbase + ms_.bstart[b + 1];
-      fp::PatchRange pr{mi, b0, b1, (uint32_t)halo.size(), 0u, (uint32_t)pfaces.size(), 0u, 0u};
+      fp::PatchRange pr{};
+      pr.mesh = mi;
+      pr.begin = b0;
+      pr.end = b1;
+      pr.halo_begin = (uint32_t)halo.size();
+      pr.face_begin = (uint32_t)pfaces.size();
       if (ms_.patch_ok) {
         const size_t h0 = halo.size(), q0 = pfaces.size();
         auto local = [&](uint32_t g) -> uint32_t {  // LDS index of device vertex g (adds it to the halo)
@@ -559,11 +564,11 @@ int build_incidence(fp_sim* s) {
             if (!fseen[vf[k]]) { fseen[vf[k]] = 1; fl.push_back(vf[k]); }
         for (uint32_t qi = 0; qi < (uint32_t)fl.size(); ++qi) {
           const uint32_t f = fl[qi];
-          fp::PatchFace pf{};
+          fp::PatchFace pf{0};
           uint32_t g3[3];
           for (int c = 0; c < 3; ++c) {
             g3[c] = (uint32_t)ms_.dev(h.f_v[3 * (uint64_t)f + c]);
-            pf.v[c] = (uint16_t)std::min<uint32_t>(local(g3[c]), fp::kPatchLocal - 1);
+            pf.bits |= std::min<uint32_t>(local(g3[c]), fp::kPatchLocal - 1) << (9 * c);
           }
           // corner c of a patch vertex: Face::vertex_angle's operands are the next and the
           // previous corner (springy_mesh.rs:163-172), in the entry of the face's rank among
@@ -571,8 +576,8 @@ int build_incidence(fp_sim* s) {
           for (int c = 0; c < 3; ++c)
             if (g3[c] >= b0 && g3[c] < b1)
               pcorner[ffirst[g3[c]] + fp::kSlice * frank[3 * (ms_.fbase + f) + c]] =
-                  fp::PatchCorner{(uint16_t)std::min<uint32_t>(qi, fp::kPatchFaceCap - 1), pf.v[(c + 1) % 3],
-                                  pf.v[(c + 2) % 3], 0};
+                  fp::PatchCorner{std::min<uint32_t>(qi, fp::kPatchFaceCap - 1) | pf.v((c + 1) % 3) << 11 |
+                                  pf.v((c + 2) % 3) << 20 | 1u << 31};
           pfaces.push_back(pf);
         }
         for (uint32_t f : fl) fseen[f] = 0;
@@ -580,6 +585,21 @@ int build_incidence(fp_sim* s) {
         pr.n_faces = (uint32_t)(pfaces.size() - q0);
         if ((b1 - b0) + pr.n_halo > fp::kPatchLocal || pr.n_faces > fp::kPatchFaceCap) ms_.patch_ok = false;
         for (size_t k = h0; k < halo.size(); ++k) mark[halo[k]] = -1;
+        for (uint32_t w = 0; w < 4; ++w) {
+          const uint32_t v0 = b0 + fp::kSlice * w < b1 ? b0 + fp::kSlice * w : b0;
+          const uint32_t v1 = std::min(v0 + fp::kSlice, b1);
+          pr.s_base[w] = sfirst[v0];
+          pr.f_base[w] = ffirst[v0];
+          pr.s_min[w] = *std::min_element(scnt.begin() + v0, scnt.begin() + v1);
+          pr.s_max[w] = *std::max_element(scnt.begin() + v0, scnt.begin() + v1);
+          pr.f_min[w] = *std::min_element(fcnt.begin() + v0, fcnt.begin() + v1);
+          pr.f_max[w] = *std::max_element(fcnt.begin() + v0, fcnt.begin() + v1);
+          for (uint32_t i = v0; i < v1; ++i)
+            for (uint32_t j = 0; j < scnt[i]; ++j) {
+              const float len = std::fabs(sent[sfirst[i] + fp::kSlice * j].len);
+              if (!(len >= 0x1p-126f && len <= 0x1p126f)) pr.s_min[w] = 0;
+            }
+        }
       }
       s->h_patches.push_back(pr);
     }
@@ -588,8 +608,12 @@ int build_incidence(fp_sim* s) {
   HIP_TRY(s->patch_faces.upload(pfaces.data(), pfaces.size()));
   HIP_TRY(s->p_corner.upload(pcorner.data(), pcorner.size()));
   {
-    std::vector<fp::PatchStrut> pent(n_sent + 1);
-    for (uint64_t e = 0; e <= n_sent; ++e) pent[e] = fp::PatchStrut{sent[e].len, sloc[e], scls[e]};
+    std::vector<fp::PatchStrut> pent(n_sent + fp::kSlice, fp::PatchStrut{1.0f, 0, 0});
+    for (uint64_t i = 0; i < N; ++i)
+      for (uint32_t j = 0; j < scnt[i]; ++j) {
+        const uint32_t e = sfirst[i] + fp::kSlice * j;
+        pent[e] = fp::PatchStrut{sent[e].len, sloc[e], (uint16_t)(scls[e] | 0x8000u)};
+      }
     HIP_TRY(s->p_ent.upload(pent.data(), pent.size()));
     HIP_TRY(s->p_cls.upload(cls_tab.data(), cls_tab.size()));
   }

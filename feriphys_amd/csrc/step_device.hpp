@@ -75,6 +75,8 @@ struct GridView {
   const uint32_t* cell_faces;
 };
 
+constexpr uint32_t kScanFaces = 8;  // obstacles of at most this many faces in all are scanned face by face
+
 struct ObsView {
   const ObsFace* faces;
   uint32_t n_faces;
@@ -98,6 +100,15 @@ __device__ __forceinline__ f3 ld3(const float* __restrict__ x, const float* __re
 // the gathering vertex as v0 yields that same value bit for bit, because p_a - p_b = -(p_b - p_a)
 // and every later product carries the sign through exactly.
 template <class M>
+__device__ __forceinline__ void strut_from(f3 d, float len, float inv, f3 dv, float k, float c, float rest, f3& spring,
+                                           f3& damp) {
+  f3 u = f3{d.x * inv, d.y * inv, d.z * inv};
+  float s = k * (len - rest);
+  spring = f3{s * u.x, s * u.y, s * u.z};
+  float dd = c * M::dot(dv, u);
+  damp = f3{dd * u.x, dd * u.y, dd * u.z};
+}
+template <class M>
 __device__ __forceinline__ void strut_accumulate(f3& F, f3 p_self, f3 v_self, f3 p_nbr, f3 v_nbr, float k, float c,
                                                  float rest) {
   f3 d = sub(p_nbr, p_self);
@@ -110,11 +121,9 @@ __device__ __forceinline__ void strut_accumulate(f3& F, f3 p_self, f3 v_self, f3
     len = sqrt_rn(dot(d, d));
     inv = M::rcp(len);
   }
-  f3 u = f3{d.x * inv, d.y * inv, d.z * inv};
-  float s = k * (len - rest);
-  F = add(F, f3{s * u.x, s * u.y, s * u.z});
-  float dd = c * M::dot(sub(v_nbr, v_self), u);
-  F = add(F, f3{dd * u.x, dd * u.y, dd * u.z});
+  f3 spring, damp;
+  strut_from<M>(d, len, inv, sub(v_nbr, v_self), k, c, rest, spring, damp);
+  F = add(add(F, spring), damp);
 }
 
 // Drag + lift on one face (springy_mesh.rs:631-646); the weighted share for corner `corner` is
@@ -146,7 +155,7 @@ FP_HD f3 face_force(f3 p0, f3 p1, f3 p2, f3 u0, f3 u1, f3 u2, const StepParams& 
 
 // Face::vertex_angle (springy_mesh.rs:163-172): angle between (p_b - p_a) and (p_c - p_a) at p_a,
 // called as (p2 - p0).angle(p1 - p0) for corner 0 etc.; returns angle / PI.
-template <class M>
+template <class M, bool TAB = false>
 FP_HD float corner_weight(f3 pa, f3 pnext, f3 pprev, const float (*tab)[4] = nullptr) {
   // vertex_angle(v0, v1, v2) = (p[v2] - p[v0]).angle(p[v1] - p[v0]); angle = atan2(|a x b|, a.b)
   f3 a = sub(pprev, pa);
@@ -154,7 +163,7 @@ FP_HD float corner_weight(f3 pa, f3 pnext, f3 pprev, const float (*tab)[4] = nul
   f3 axb = cross(a, b);
   const float n2 = M::dot(axb, axb), d = M::dot(a, b);
   float w;
-  if (M::corner_in_range(n2, d, w, tab)) return w;
+  if (M::template corner_in_range<TAB>(n2, d, w, tab)) return w;
   return M::div_pi(M::atan2_(M::sqrt_(n2), d));  // Rad / Rad(PI), PI = std::f32::consts::PI
 }
 

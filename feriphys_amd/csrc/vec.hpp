@@ -65,14 +65,15 @@ struct ExactMath {
   FP_HD static float div_pi(float x) { return div_pi_rn(x); }
   // atan2(sqrt(n2), d) / PI where every quotient on the way is within div_by_rcp's range (returns
   // true): the same roundings as div_pi(atan2_(sqrt_(n2), d)) in a quarter fewer operations.  With
-  // `tab`, the kFdlEntries entries of fdl_entry, one wide LDS read stands for the selects that pick
+  // TAB, `tab` the kFdlEntries entries of fdl_entry, one wide LDS read stands for the selects that pick
   // the reduction interval (13 of a corner's 112 operations).
-  FP_HD static bool corner_in_range(float n2, float d, float& w, const float (*tab)[4] = nullptr) {
+  template <bool TAB>
+  FP_HD static bool corner_in_range(float n2, float d, float& w, const float (*tab)[4]) {
 #ifdef __HIP_DEVICE_COMPILE__
     const float y = sqrt_in_range(n2), ad = __builtin_fabsf(d);
     const float t = div_by_rcp(y, ad, rcp_in_range(ad));
     FdlReduced q;
-    if (tab != nullptr) {
+    if constexpr (TAB) {
       const float4 k = *reinterpret_cast<const float4*>(tab[(uint32_t)fminf(t * 16.0f, 39.0f)]);
       q = FdlReduced{__builtin_fmaf(t, k.x, -k.y), k.x + t * k.y, k.z, k.w};
     } else {
@@ -126,7 +127,8 @@ struct FastMath {
   __device__ static f3 div3(f3 v, float s) { return f3{div(v.x, s), div(v.y, s), div(v.z, s)}; }
   __device__ static float atan2_(float y, float x) { return fast_atan2(y, x); }
   __device__ static float div_pi(float x) { return div(x, 3.14159274101257324f); }
-  __device__ static bool corner_in_range(float n2, float d, float& w, const float (*tab)[4] = nullptr) {
+  template <bool TAB>
+  __device__ static bool corner_in_range(float n2, float d, float& w, const float (*)[4]) {
     w = div_pi(atan2_(sqrt_(n2), d));
     return true;
   }
