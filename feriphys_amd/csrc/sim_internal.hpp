@@ -121,6 +121,8 @@ struct fp_sim {
     fph::DBuf<float> slot_k, da, work;
     fph::DBuf<fp::StepParams> big_params;
     fph::DBuf<fp::DiagOut> diag;
+    fph::DBuf<fp::MeshSlots> mesh_slots;
+    fph::HostBuf mesh_diag;  // per mesh, written by the kernel
     fph::DBuf<float> keep[6];  // surrogate results of the meshes that keep them during a fallback
     fph::DBuf<uint32_t> mesh_of, ids;
     std::vector<fp::SlotEnt> h_slots;

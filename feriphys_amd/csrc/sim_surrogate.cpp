@@ -24,8 +24,8 @@ namespace {
 int build_slots(fp_sim* s) {
   auto& S = s->sur;
   const uint64_t N = s->N;
-  S.h_slots.assign(N * fp::kSlots, fp::SlotEnt{fp::kNoSlot, 1.0f});
-  std::vector<float> sk(N * fp::kSlots, 0.0f);
+  S.h_slots.assign(fp::slot_count(N), fp::SlotEnt{fp::kNoSlot, 1.0f});
+  std::vector<float> sk(fp::slot_count(N), 0.0f);
   std::vector<uint32_t> mesh_of(N), ids;
   std::vector<uint8_t> used(N, 0);
   static const int offs[10][2] = {{0, 1}, {0, -1}, {1, 0}, {-1, 0}, {-1, 1}, {1, -1}, {0, 2}, {0, -2}, {2, 0}, {-2, 0}};
@@ -54,11 +54,20 @@ int build_slots(fp_sim* s) {
           slot = used[gi]++;
         }
         if (slot < 0) continue;
-        S.h_slots[gi * fp::kSlots + slot] = fp::SlotEnt{(uint32_t)ms.dev(other), h.s_len[k]};
-        sk[gi * fp::kSlots + slot] = h.s_k[k];
+        S.h_slots[fp::slot_at((uint32_t)gi, slot)] = fp::SlotEnt{(uint32_t)ms.dev(other), h.s_len[k]};
+        sk[fp::slot_at((uint32_t)gi, slot)] = h.s_k[k];
       }
     }
   }
+  std::vector<fp::MeshSlots> mesh_slots;
+  for (const auto& ms : s->meshes) {
+    fp::MeshSlots r{ms.blk_begin, ms.blk_end, 0u, 0u};
+    for (uint64_t i = ms.vbase; i < ms.vbase + ms.host.n; ++i)
+      for (uint32_t j = r.n_slots; j < (uint32_t)fp::kSlots; ++j)
+        if (S.h_slots[fp::slot_at((uint32_t)i, (int)j)].nbr != fp::kNoSlot) r.n_slots = j + 1;
+    mesh_slots.push_back(r);
+  }
+  HIP_TRY(S.mesh_slots.upload(mesh_slots.data(), mesh_slots.size()));
   HIP_TRY(S.slots.upload(S.h_slots.data(), S.h_slots.size()));
   HIP_TRY(S.slot_k.upload(sk.data(), sk.size()));
   HIP_TRY(S.mesh_of.upload(mesh_of.data(), mesh_of.size()));
@@ -92,6 +101,7 @@ int prepare_surrogate(fp_sim* s, const fp_surrogate_config& c) {
   HIP_TRY(s->sur.da.reserve(3 * s->N + 1));
   HIP_TRY(s->sur.work.reserve(s->N + 1));
   HIP_TRY(s->sur.diag.reserve(s->h_blocks.size() + 1));
+  HIP_TRY(s->sur.mesh_diag.reserve((s->meshes.size() + 1) * sizeof(fp::MeshDiag)));
   return FP_OK;
 }
 
@@ -137,25 +147,15 @@ int sur_big_step(fp_sim* s, fp_surrogate_stats& st, float* mlp_ms) {
   if (fused)
     for (int sh = 0; sh < fp::N_LAUNCH_SHAPES; ++sh)
       HIP_TRY(fp::launch_grid_tiled(a, s->cloths.p, s->tiles[sh].p, s->n_tiles[sh], sh, fp::MODE_SURROGATE, s->stream));
+  const fp::MeshDiag* d = static_cast<const fp::MeshDiag*>(S.mesh_diag.p);
   HIP_TRY(fp::launch_sur_diag(a.in, a.out, S.slots.p, S.slot_k.p, S.big_params.p, s->mass.p, S.work.p, s->all_blocks.p,
-                              nblk, S.diag.p, s->stream));
-  std::vector<fp::DiagOut> d(nblk);
-  HIP_TRY(hipMemcpyAsync(d.data(), S.diag.p, nblk * sizeof(fp::DiagOut), hipMemcpyDeviceToHost, s->stream));
+                              nblk, S.mesh_slots.p, (uint32_t)M, S.diag.p, static_cast<fp::MeshDiag*>(S.mesh_diag.p),
+                              s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   if (mlp_ms) {
     float t = 0.0f;
     HIP_TRY(hipEventElapsedTime(&t, s->ev0, s->ev1));
     *mlp_ms += t;
-  }
-  std::vector<double> eo(M, 0.0), en(M, 0.0), em(M, 0.0);
-  std::vector<float> ds(M, 0.0f);
-  for (uint32_t b = 0; b < nblk; ++b) {
-    const uint32_t m = s->h_blocks[b].mesh;
-    const float x = d[b].max_dstrain;
-    ds[m] = (x > ds[m] || x != x) ? x : ds[m];
-    eo[m] += d[b].e_old;
-    en[m] += d[b].e_new;
-    em[m] += d[b].emech_old;
   }
   std::vector<uint8_t> bad(M, 0);
   size_t nbad = 0;
@@ -166,12 +166,12 @@ int sur_big_step(fp_sim* s, fp_surrogate_stats& st, float* mlp_ms) {
       ++nbad;
       continue;
     }
-    const float er = (float)((en[m] - eo[m]) / std::max(em[m], 1e-30));
-    bad[m] = !(ds[m] <= S.cfg.strain_limit) || !(er <= S.cfg.energy_limit);
+    const float er = (float)((d[m].e_new - d[m].e_old) / std::max(d[m].emech_old, 1e-30)), ds = d[m].max_dstrain;
+    bad[m] = !(ds <= S.cfg.strain_limit) || !(er <= S.cfg.energy_limit);
     nbad += bad[m];
     S.backoff[m] = bad[m] ? std::min<uint32_t>(S.backoff[m] ? 2 * S.backoff[m] : 1, 16) : 0;
     S.skip[m] = bad[m] ? S.backoff[m] : 0;
-    st.max_strain_residual = (ds[m] > st.max_strain_residual || ds[m] != ds[m]) ? ds[m] : st.max_strain_residual;
+    st.max_strain_residual = (ds > st.max_strain_residual || ds != ds) ? ds : st.max_strain_residual;
     st.max_energy_residual = (er > st.max_energy_residual || er != er) ? er : st.max_energy_residual;
   }
   ++st.big_steps;
@@ -393,7 +393,7 @@ int fp_sim_surrogate_slots(fp_sim* s, uint64_t mesh, int64_t* nbr, float* rest) 
   const MeshSlot& m = s->meshes[mesh];
   for (uint64_t i = 0; i < m.host.n; ++i)
     for (int j = 0; j < fp::kSlots; ++j) {
-      const fp::SlotEnt e = s->sur.h_slots[m.dev(i) * fp::kSlots + j];
+      const fp::SlotEnt e = s->sur.h_slots[fp::slot_at((uint32_t)m.dev(i), j)];
       nbr[i * fp::kSlots + j] = e.nbr == fp::kNoSlot ? -1 : (int64_t)m.ref(e.nbr - m.vbase);
       rest[i * fp::kSlots + j] = e.nbr == fp::kNoSlot ? 0.0f : e.rest;
     }

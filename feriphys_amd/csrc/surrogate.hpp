@@ -46,6 +46,14 @@ struct SlotEnt {
   float rest;
 };
 
+// Where slot j of vertex i stands: the vertices in slices of 64, each slot's 64 entries together, so
+// that one load of a wavefront over consecutive vertices reads consecutive entries (an array of 12
+// entries a vertex spread each load over as many lines as lanes).
+__host__ __device__ inline size_t slot_at(uint32_t i, int j) {
+  return (size_t)(i / 64) * (64 * kSlots) + (size_t)(64 * j) + i % 64;
+}
+inline size_t slot_count(uint64_t n) { return (n + 63) / 64 * (64 * kSlots); }
+
 struct FeatParams {
   float H;             // big step (s)
   float strain_scale;  // position features: strain_scale * (|d| - L) / L * d / |d|
@@ -58,6 +66,16 @@ struct DiagOut {
   float max_dstrain, e_old, e_new, emech_old;
 };
 
+// The same of a whole mesh, summed in double.
+struct MeshDiag {
+  double e_old, e_new, emech_old;
+  float max_dstrain, pad;
+};
+// A mesh's blocks, and the number of slots that a vertex of it has at most.
+struct MeshSlots {
+  uint32_t blk_begin, blk_end, n_slots, pad;
+};
+
 // variant: vertices per wave / 16 (2: 1024-thread workgroups, the default; 4: 512 threads)
 hipError_t launch_sur_mlp(const SoA& st, const SlotEnt* slots, uint32_t n, const void* image, FeatParams fp,
                           float out_scale, float* da, int grid, int variant, hipStream_t s);
@@ -66,9 +84,11 @@ hipError_t launch_sur_mlp(const SoA& st, const SlotEnt* slots, uint32_t n, const
 // each vertex's face-force work over the step.
 hipError_t launch_sur_integrate(const StepArgs& a, const CsrView& t, const BlockRange* blocks, uint32_t n_blocks,
                                 const float* da, float* work, bool struts, hipStream_t s);
+// Diagnostics of the big step from `in` to `out`: per block in `diag`, then per mesh in `per_mesh`.
 hipError_t launch_sur_diag(const SoA& in, const SoA& out, const SlotEnt* slots, const float* slot_k,
                            const StepParams* params, const float* mass, const float* work, const BlockRange* blocks,
-                           uint32_t n_blocks, DiagOut* diag, hipStream_t s);
+                           uint32_t n_blocks, const MeshSlots* meshes, uint32_t n_meshes, DiagOut* diag,
+                           MeshDiag* per_mesh, hipStream_t s);
 // Per block of `blocks`: max over its vertices of |v| / vmax and |strain| / smax (+inf when any
 // value is not finite).
 hipError_t launch_sur_health(const SoA& st, const SlotEnt* slots, const BlockRange* blocks, uint32_t n_blocks,

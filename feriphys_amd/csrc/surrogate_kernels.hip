@@ -19,9 +19,10 @@ __device__ __forceinline__ void store_state(const SoA& o, uint32_t i, f3 x, f3 v
 // can issue every load of a pass before the first feature is computed.
 __device__ __forceinline__ void slot_feat_from(f3 p, f3 v, f3 q, f3 w, float rest, bool has, FeatParams fp, float* f) {
   const f3 d = sub(q, p);
-  const float len = __builtin_sqrtf(d.x * d.x + d.y * d.y + d.z * d.z);
+  const float d2 = d.x * d.x + d.y * d.y + d.z * d.z;
+  const float len = sqrt_in_range(d2);  // (exact but for d2 < 2^-96, where it may be an ulp off)
   const float il = __builtin_amdgcn_rcpf(rest);
-  const float st = (has && len > 0.0f) ? fp.strain_scale * ((len - rest) * il) * __builtin_amdgcn_rcpf(len) : 0.0f;
+  const float st = (has && d2 > 0.0f) ? fp.strain_scale * ((len - rest) * il) * __builtin_amdgcn_rcpf(len) : 0.0f;
   const float hv = has ? fp.H * il : 0.0f;
   f[0] = st * d.x; f[1] = st * d.y; f[2] = st * d.z;
   f[3] = (w.x - v.x) * hv; f[4] = (w.y - v.y) * hv; f[5] = (w.z - v.z) * hv;
@@ -37,14 +38,17 @@ __device__ __forceinline__ void slot_feat(const SoA& S, f3 p, f3 v, uint32_t sel
 __device__ __forceinline__ float unit_open(uint64_t h) { return ((float)(h >> 40) + 0.5f) * (1.0f / 16777216.0f); }
 
 // ---------------------------------------------------------------------------------------------
-// Inference: a workgroup takes 512 vertices per pass, NT MFMA column tiles of 16 vertices per wave
-// (NT = 2: 16 waves of 32 vertices, 4 waves per SIMD within 128 registers; NT = 4: 8 waves of 64).
+// Inference: a workgroup takes a contiguous run of units, NT MFMA column tiles of 16 vertices, one
+// unit a wave at a time (NT = 2: 16 waves of 32 vertices, 4 waves per SIMD within 128 registers; NT =
+// 4: 8 waves of 64).  The units are shared out evenly, so that in the last round every CU has a part
+// of its waves busy and not some CUs all of them, and few units are one to a CU.  Bound by the vector
+// instructions (768 of a unit's 1,400 are the activation): 330,880 vertices 45.3 us where whole passes
+// of 512 vertices a workgroup took 54.0, 1,024 vertices 11.2 (17.1), 1,048,576 vertices 125 (127.5).
 // Neurons are the MFMA rows, vertices the columns, so a layer's f32 output tile already holds, per
 // lane, 4 consecutive neurons of one vertex; two such tiles form the next layer's 8-element bf16
 // operand once the weights' K index is permuted the same way (done when the image is packed).  The
 // activations never leave registers; the weights stay in LDS for the whole (persistent) launch.
 
-constexpr int kMlpTile = 512;
 
 // One layer, acc = W B + bias then the activation, pipelined by output block: the 16 neurons of
 // block mt accumulate (KB MFMAs per column tile, the bias as the accumulators' initial value)
@@ -92,10 +96,14 @@ __global__ void __launch_bounds__(2048 / NT) sur_mlp_kernel(SoA S, const SlotEnt
   const __bf16* W3 = reinterpret_cast<const __bf16*>(img + kImgW3);
   const __bf16* W4 = reinterpret_cast<const __bf16*>(img + kImgW4);
   const float* Bias = reinterpret_cast<const float*>(img + kImgB);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
-  for (uint32_t t0 = blockIdx.x * kMlpTile; t0 < n; t0 += gridDim.x * kMlpTile) {
-    const uint32_t v0 = t0 + wave * 16 * NT;
-    if (v0 >= n) continue;
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t units = (n + 16 * NT - 1) / (16 * NT);
+  const uint32_t u0 = (uint32_t)((uint64_t)blockIdx.x * units / gridDim.x);
+  const uint32_t u1 = (uint32_t)((uint64_t)(blockIdx.x + 1) * units / gridDim.x);
+  for (uint32_t r0 = u0; r0 < u1; r0 += kThreads / 64) {
+    if (r0 + wave >= u1) continue;
+    const uint32_t v0 = (r0 + wave) * 16 * NT;
     // features: lane group g computes slots 3g..3g+2 of its vertex (18 values, then 6 zeros), which
     // are its 8-element K slices of the three 32-wide K blocks of layer 1.  Every load is
     // unconditional (past-the-end columns read vertex n-1, empty slots the vertex itself; both are
@@ -107,12 +115,13 @@ __global__ void __launch_bounds__(2048 / NT) sur_mlp_kernel(SoA S, const SlotEnt
     for (int nt = 0; nt < NT; ++nt) {
       const uint32_t iv = v0 + nt * 16 + col;
       const uint32_t i = iv < n ? iv : n - 1;
+      const SlotEnt* at = slots + slot_at(i, 3 * g);
       p[nt] = ld3(S.x, S.y, S.z, i);
       v[nt] = ld3(S.vx, S.vy, S.vz, i);
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        se[nt][j] = slots[(size_t)i * kSlots + 3 * g + j];
-        if (iv >= n) se[nt][j].nbr = kNoSlot;
+        se[nt][j] = at[64 * j];
+        se[nt][j].nbr = iv < n ? se[nt][j].nbr : kNoSlot;
       }
     }
 #pragma unroll
@@ -121,7 +130,10 @@ __global__ void __launch_bounds__(2048 / NT) sur_mlp_kernel(SoA S, const SlotEnt
       const uint32_t i = iv < n ? iv : n - 1;
       float f[24];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) slot_feat(S, p[nt], v[nt], i, se[nt][j], fp, f + 6 * j);
+      for (int j = 0; j < 3; ++j) {
+        slot_feat(S, p[nt], v[nt], i, se[nt][j], fp, f + 6 * j);
+        __builtin_amdgcn_sched_barrier(0x20);  // loads may pass, arithmetic not: slots interleaved spill
+      }
 #pragma unroll
       for (int k = 18; k < 24; ++k) f[k] = 0.0f;
 #pragma unroll
@@ -201,12 +213,16 @@ __global__ void __launch_bounds__(kBlock) sur_integrate_kernel(StepArgs A, CsrVi
 // Diagnostics of a big step over the vertices of `blocks`: the largest change of any strut strain
 // (each strut seen from both ends; NaN propagates), energies before and after (kinetic, spring
 // with each strut counted half from each end, gravity potential -F_g . x), the face-force work
-// subtracted from the energy after.
+// subtracted from the energy after.  Bound by the slots' bytes (12 for each of a cloth's ten) and the
+// vector instructions (696 a vertex); 330,880 vertices: 17.5 us, 23.7 before the slots were sliced, one
+// group of them held at a time and the roots short.
 __global__ void __launch_bounds__(kBlock) sur_diag_kernel(SoA I, SoA O, const SlotEnt* __restrict__ slots,
                                                            const float* __restrict__ slot_k,
                                                            const StepParams* __restrict__ params,
                                                            const float* __restrict__ mass, const float* __restrict__ work,
-                                                           const BlockRange* __restrict__ blocks, DiagOut* __restrict__ out) {
+                                                           const BlockRange* __restrict__ blocks,
+                                                           const MeshSlots* __restrict__ meshes,
+                                                           DiagOut* __restrict__ out) {
   __shared__ float s_ds[kBlock], s_eo[kBlock], s_en[kBlock], s_em[kBlock];
   const BlockRange br = blocks[blockIdx.x];
   const uint32_t iv = br.begin + threadIdx.x;
@@ -218,34 +234,53 @@ __global__ void __launch_bounds__(kBlock) sur_diag_kernel(SoA I, SoA O, const Sl
     const float m = P.uniform_mass ? P.mass : mass[i];
     const f3 po = ld3(I.x, I.y, I.z, i), pn = ld3(O.x, O.y, O.z, i);
     const f3 vo = ld3(I.vx, I.vy, I.vz, i), vn = ld3(O.vx, O.vy, O.vz, i);
-    // all slot entries first, then all neighbour positions (empty slots read the vertex itself), so
-    // the loads are in flight together
-    SlotEnt e[kSlots];
-    float k[kSlots];
-#pragma unroll
-    for (int j = 0; j < kSlots; ++j) {
-      e[j] = slots[(size_t)i * kSlots + j];
-      k[j] = slot_k[(size_t)i * kSlots + j];
-    }
-    f3 qo[kSlots], qn[kSlots];
-#pragma unroll
-    for (int j = 0; j < kSlots; ++j) {
-      const uint32_t nb = e[j].nbr != kNoSlot ? e[j].nbr : i;
-      qo[j] = ld3(I.x, I.y, I.z, nb);
-      qn[j] = ld3(O.x, O.y, O.z, nb);
-    }
+    // five slots at a time (a cloth's vertex has ten): their entries, then their neighbours' positions
+    // (empty slots read the vertex itself), so the loads are in flight together
+    constexpr int kGroup = 5;
     float so = 0.0f, sn = 0.0f;
+    const int n_slots = (int)meshes[br.mesh].n_slots;
+#pragma unroll 1
+    for (int j0 = 0; j0 < n_slots; j0 += kGroup) {
+      SlotEnt e[kGroup];
+      float k[kGroup];
 #pragma unroll
-    for (int j = 0; j < kSlots; ++j) {
-      const bool has = e[j].nbr != kNoSlot;
-      const f3 d_o = sub(qo[j], po), d_n = sub(qn[j], pn);
-      const float r = has ? e[j].rest : 1.0f;
-      const float lo = __builtin_sqrtf(dot(d_o, d_o)) - r, ln = __builtin_sqrtf(dot(d_n, d_n)) - r;
-      const float d = has ? __builtin_fabsf(ln - lo) * __builtin_amdgcn_rcpf(r) : 0.0f;
-      ds = (d > ds || d != d) ? d : ds;
-      const float kk = has ? 0.25f * k[j] : 0.0f;
-      so += kk * lo * lo;
-      sn += kk * ln * ln;
+      for (int j = 0; j < kGroup; ++j) {
+        const bool any = j0 + j < kSlots;
+        e[j] = slots[slot_at(i, any ? j0 + j : 0)];
+        k[j] = slot_k[slot_at(i, any ? j0 + j : 0)];
+        if (!any) e[j].nbr = kNoSlot;
+      }
+      float o2[kGroup], n2[kGroup], lo[kGroup], ln[kGroup];
+      uint32_t far = 0;
+#pragma unroll
+      for (int j = 0; j < kGroup; ++j) {
+        const bool has = e[j].nbr != kNoSlot;
+        const uint32_t nb = has ? e[j].nbr : i;
+        const f3 d_o = sub(ld3(I.x, I.y, I.z, nb), po), d_n = sub(ld3(O.x, O.y, O.z, nb), pn);
+        o2[j] = has ? dot(d_o, d_o) : 1.0f;
+        n2[j] = has ? dot(d_n, d_n) : 1.0f;
+        lo[j] = sqrt_in_range(o2[j]);
+        ln[j] = sqrt_in_range(n2[j]);
+        far = max(far, max(__float_as_uint(o2[j]) - __float_as_uint(0x1p-96f), __float_as_uint(n2[j]) - __float_as_uint(0x1p-96f)));
+      }
+      if (far > __float_as_uint(3.40282347e38f) - __float_as_uint(0x1p-96f)) {
+#pragma unroll
+        for (int j = 0; j < kGroup; ++j) {
+          lo[j] = sqrt_rn(o2[j]);
+          ln[j] = sqrt_rn(n2[j]);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < kGroup; ++j) {
+        const bool has = e[j].nbr != kNoSlot;
+        const float r = has ? e[j].rest : 1.0f;
+        const float xo = lo[j] - r, xn = ln[j] - r;
+        const float d = has ? __builtin_fabsf(xn - xo) * __builtin_amdgcn_rcpf(r) : 0.0f;
+        ds = (d > ds || d != d) ? d : ds;
+        const float kk = has ? 0.25f * k[j] : 0.0f;
+        so += kk * xo * xo;
+        sn += kk * xn * xn;
+      }
     }
     const float ko = 0.5f * m * dot(vo, vo), kn = 0.5f * m * dot(vn, vn);
     em = ko + so + kn + sn;
@@ -255,17 +290,54 @@ __global__ void __launch_bounds__(kBlock) sur_diag_kernel(SoA I, SoA O, const Sl
   }
   s_ds[threadIdx.x] = ds; s_eo[threadIdx.x] = eo; s_en[threadIdx.x] = en; s_em[threadIdx.x] = em;
   __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      const float a = s_ds[threadIdx.x], b = s_ds[threadIdx.x + w];
-      s_ds[threadIdx.x] = (b > a || b != b) ? b : a;
-      s_eo[threadIdx.x] += s_eo[threadIdx.x + w];
-      s_en[threadIdx.x] += s_en[threadIdx.x + w];
-      s_em[threadIdx.x] += s_em[threadIdx.x + w];
+  static_assert(kBlock == 256, "four wavefronts");
+  // the pairs of a halving tree over the workgroup: two levels from memory, six within a wavefront
+  if (threadIdx.x >= 64) return;
+  const uint32_t t = threadIdx.x;
+  const auto worse = [](float a, float b) { return (b > a || b != b) ? b : a; };
+  ds = worse(worse(s_ds[t], s_ds[t + 128]), worse(s_ds[t + 64], s_ds[t + 192]));
+  eo = (s_eo[t] + s_eo[t + 128]) + (s_eo[t + 64] + s_eo[t + 192]);
+  en = (s_en[t] + s_en[t + 128]) + (s_en[t + 64] + s_en[t + 192]);
+  em = (s_em[t] + s_em[t + 128]) + (s_em[t + 64] + s_em[t + 192]);
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) {
+    ds = worse(ds, __shfl_down(ds, w));
+    eo += __shfl_down(eo, w);
+    en += __shfl_down(en, w);
+    em += __shfl_down(em, w);
+  }
+  if (t == 0) out[blockIdx.x] = DiagOut{ds, eo, en, em};
+}
+
+// The blocks' diagnostics of one mesh a workgroup.
+__global__ void __launch_bounds__(kBlock) sur_mesh_diag_kernel(const DiagOut* __restrict__ part,
+                                                                const MeshSlots* __restrict__ meshes,
+                                                                MeshDiag* __restrict__ out) {
+  __shared__ double s_e[3][kBlock];
+  __shared__ float s_ds[kBlock];
+  const MeshSlots R = meshes[blockIdx.x];
+  const uint32_t t = threadIdx.x;
+  double e[3] = {0.0, 0.0, 0.0};
+  float ds = 0.0f;
+  for (uint32_t b = R.blk_begin + t; b < R.blk_end; b += kBlock) {
+    const DiagOut d = part[b];
+    ds = (d.max_dstrain > ds || d.max_dstrain != d.max_dstrain) ? d.max_dstrain : ds;
+    e[0] += d.e_old;
+    e[1] += d.e_new;
+    e[2] += d.emech_old;
+  }
+  s_ds[t] = ds;
+  for (int k = 0; k < 3; ++k) s_e[k][t] = e[k];
+  __syncthreads();
+  for (uint32_t w = kBlock / 2; w > 0; w >>= 1) {
+    if (t < w) {
+      const float b = s_ds[t + w];
+      s_ds[t] = (b > s_ds[t] || b != b) ? b : s_ds[t];
+      for (int k = 0; k < 3; ++k) s_e[k][t] += s_e[k][t + w];
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = DiagOut{s_ds[0], s_eo[0], s_en[0], s_em[0]};
+  if (t == 0) out[blockIdx.x] = MeshDiag{s_e[0][0], s_e[1][0], s_e[2][0], s_ds[0], 0.0f};
 }
 
 // Health of the plain trajectories that feed training: per block, the largest of |v| / vmax and
@@ -281,7 +353,7 @@ __global__ void __launch_bounds__(kBlock) sur_health_kernel(SoA S, const SlotEnt
     const f3 p = ld3(S.x, S.y, S.z, i), v = ld3(S.vx, S.vy, S.vz, i);
     h = __builtin_sqrtf(dot(v, v)) / vmax;
     for (int j = 0; j < kSlots; ++j) {
-      const SlotEnt e = slots[(size_t)i * kSlots + j];
+      const SlotEnt e = slots[slot_at(i, j)];
       if (e.nbr == kNoSlot) continue;
       const f3 d = sub(ld3(S.x, S.y, S.z, e.nbr), p);
       h = fmaxf(h, __builtin_fabsf(__builtin_sqrtf(dot(d, d)) - e.rest) / (e.rest * smax));
@@ -304,7 +376,7 @@ __global__ void __launch_bounds__(kBlock) sur_features_kernel(SoA S, const SlotE
   if (j >= n) return;
   const uint32_t i = ids[j];
   const f3 p = ld3(S.x, S.y, S.z, i), v = ld3(S.vx, S.vy, S.vz, i);
-  for (int s = 0; s < kSlots; ++s) slot_feat(S, p, v, i, slots[(size_t)i * kSlots + s], fp, out + (size_t)j * kFeat + 6 * s);
+  for (int s = 0; s < kSlots; ++s) slot_feat(S, p, v, i, slots[slot_at(i, s)], fp, out + (size_t)j * kFeat + 6 * s);
 }
 
 __global__ void __launch_bounds__(kBlock) sur_noise_kernel(Pos3 prev, Pos3 cur, SoA o, const uint32_t* __restrict__ pins,
@@ -341,7 +413,7 @@ __global__ void __launch_bounds__(kBlock) sur_samples_kernel(StepArgs A, CsrView
   const f3 p = ld3(S.x, S.y, S.z, i), v = ld3(S.vx, S.vy, S.vz, i);
   float f[kFeat];
   bool ok = true;
-  for (int s = 0; s < kSlots; ++s) slot_feat(S, p, v, i, slots[(size_t)i * kSlots + s], fp, f + 6 * s);
+  for (int s = 0; s < kSlots; ++s) slot_feat(S, p, v, i, slots[slot_at(i, s)], fp, f + 6 * s);
   for (int c = 0; c < kFeat; ++c) ok = ok && __builtin_isfinite(f[c]);
   const float m = P.uniform_mass ? P.mass : A.mass[i];
   f3 F = P.gravity;
@@ -375,8 +447,8 @@ inline unsigned blocks_for(long n) { return (unsigned)((n + kBlock - 1) / kBlock
 hipError_t launch_sur_mlp(const SoA& st, const SlotEnt* slots, uint32_t n, const void* image, FeatParams fp,
                           float out_scale, float* da, int grid, int variant, hipStream_t s) {
   if (n == 0) return hipSuccess;
-  const int tiles = (int)((n + kMlpTile - 1) / kMlpTile);
-  const dim3 g(grid < tiles ? grid : tiles);
+  const uint32_t units = (n + 16 * variant - 1) / (16 * variant);
+  const dim3 g((uint32_t)grid < units ? (uint32_t)grid : units);
   if (variant == 4)
     hipLaunchKernelGGL(sur_mlp_kernel<4>, g, dim3(512), 0, s, st, slots, n, reinterpret_cast<const uint4*>(image), fp,
                        out_scale, da);
@@ -398,10 +470,12 @@ hipError_t launch_sur_integrate(const StepArgs& a, const CsrView& t, const Block
 
 hipError_t launch_sur_diag(const SoA& in, const SoA& out, const SlotEnt* slots, const float* slot_k,
                            const StepParams* params, const float* mass, const float* work, const BlockRange* blocks,
-                           uint32_t n_blocks, DiagOut* diag, hipStream_t s) {
-  if (n_blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(sur_diag_kernel, dim3(n_blocks), dim3(kBlock), 0, s, in, out, slots, slot_k, params, mass, work,
-                     blocks, diag);
+                           uint32_t n_blocks, const MeshSlots* meshes, uint32_t n_meshes, DiagOut* diag,
+                           MeshDiag* per_mesh, hipStream_t s) {
+  if (n_blocks)
+    hipLaunchKernelGGL(sur_diag_kernel, dim3(n_blocks), dim3(kBlock), 0, s, in, out, slots, slot_k, params, mass, work,
+                       blocks, meshes, diag);
+  if (n_meshes) hipLaunchKernelGGL(sur_mesh_diag_kernel, dim3(n_meshes), dim3(kBlock), 0, s, diag, meshes, per_mesh);
   return hipGetLastError();
 }
 
