@@ -61,9 +61,10 @@ struct Body {
   f3 p, l;  // linear and angular momentum
 };
 // Stateful::derivative (rigidbody.rs:94-157) of those fields; the momenta's are force and torque.
-__device__ __forceinline__ void derivative(const Body& S, float m, const M3& I0, f3& dx, Q& dq) {
+__device__ __forceinline__ void derivative(const Body& S, float m, const M3& I0, f3& dx, Q& dq, M3& I, f3& w) {
   dx = ExactMath::div3(S.p, m);  // linear_momentum / mass
-  const f3 w = mv(inertia_inv(S.q, I0), S.l);
+  I = inertia_inv(S.q, I0);
+  w = mv(I, S.l);
   dq = qmul(Q{0.5f * 0.0f, f3{0.5f * w.x, 0.5f * w.y, 0.5f * w.z}}, S.q);
 }
 // Makes values opaque where they stand: the compiler otherwise interleaves the four stages (the momenta's
@@ -78,7 +79,9 @@ __device__ __forceinline__ void derivative_later(const Body& S, float m, M3 I0, 
     settle(I0.c[c]);
     I0.c[c] = add(I0.c[c], f3{0.0f, 0.0f, 0.0f});
   }
-  derivative(S, m + 0.0f, I0, dx, dq);
+  M3 I;
+  f3 w;
+  derivative(S, m + 0.0f, I0, dx, dq, I, w);
 }
 // a + s b, per component, as the reference's vec_add and scale round it
 __device__ __forceinline__ f3 axpy(f3 a, float s, f3 b) { return f3{a.x + b.x * s, a.y + b.y * s, a.z + b.z * s}; }
@@ -128,43 +131,42 @@ __device__ __forceinline__ ObsFace uniform_face(const ObsView& O, uint32_t f) {
   return q;
 }
 
-// The corners (bit k: corner k) that can meet an obstacle between the two poses: with few faces, those
-// that change sides of some face's plane (the first test of face_hit, as it computes it); with the
-// grids, all or none, by the box around all the corners against the faces' box.
-template <bool GRID>
-__device__ __forceinline__ uint32_t may_hit(const ObsView& O, const Corners& Co, f3 xo, const Corners& Cn, f3 xn) {
-  if constexpr (!GRID) {
-    uint32_t any = 0;
-    for (uint32_t f = 0; f < O.n_faces; ++f) {
-      const ObsFace F = uniform_face(O, f);
-      const f3 v0 = f3{F.v0[0], F.v0[1], F.v0[2]}, n = f3{F.n[0], F.n[1], F.n[2]};
-      uint32_t crossed = 0;
+// Few faces: on which side of each face's plane the eight corners of a pose are, the first test of
+// face_hit as it computes it: bit 8 f + k is the sign of corner k's distance from face f.
+static_assert(kScanFaces * 8 <= 64, "a bit for each face and corner");
+__device__ __forceinline__ uint64_t corner_sides(const ObsView& O, const Corners& C, f3 x) {
+  uint64_t sides = 0;
+  for (uint32_t f = 0; f < O.n_faces; f += 2) {  // two at a time, so that each corner is formed half as often
+    // (of an odd number the last one twice)
+    const ObsFace F = uniform_face(O, f), G = uniform_face(O, f + 1 < O.n_faces ? f + 1 : f);
+    const f3 v0 = f3{F.v0[0], F.v0[1], F.v0[2]}, n = f3{F.n[0], F.n[1], F.n[2]};
+    const f3 w0 = f3{G.v0[0], G.v0[1], G.v0[2]}, o = f3{G.n[0], G.n[1], G.n[2]};
+    uint32_t side = 0, other = 0;
 #pragma unroll
-      for (int k = 7; k >= 0; --k) {
-        if (k % 2 == 1) {  // the sixteen corner positions formed as they are needed, not held in 48 registers
-          settle(xo);
-          settle(xn);
-        }
-        const float od = dot(sub(corner_at(Co, xo, k), v0), n), nd = dot(sub(corner_at(Cn, xn, k), v0), n);
-        crossed = __builtin_amdgcn_alignbit(crossed, __float_as_uint(od) ^ __float_as_uint(nd), 31);
-      }
-      any |= crossed;
+    for (int k = 7; k >= 0; --k) {
+      if (k % 2 == 1) settle(x);  // the corners' positions formed as they are needed, not held in 24 registers
+      const f3 c = corner_at(C, x, k);
+      side = __builtin_amdgcn_alignbit(side, __float_as_uint(dot(sub(c, v0), n)), 31);
+      other = __builtin_amdgcn_alignbit(other, __float_as_uint(dot(sub(c, w0), o)), 31);
     }
-    return any;
-  } else {
-    if (O.n_always != 0) return 0xffu;
-    // a corner's offset is at most max(|s|, |d|) + |a| in each row
-    auto meets = [&](float s0, float d0, float a0, float x0, float s1, float d1, float a1, float x1, float lo, float hi) {
-      const float e0 = fmaxf(fabsf(s0), fabsf(d0)) + fabsf(a0), e1 = fmaxf(fabsf(s1), fabsf(d1)) + fabsf(a1);
-      // 2 margin: the corners' own test grows by one; the other covers the rounding of these sums (the
-      // margin is at least 1e-4 of the largest obstacle coordinate)
-      return !(fminf(x0 - e0, x1 - e1) - 2.0f * O.margin > hi) && !(fmaxf(x0 + e0, x1 + e1) + 2.0f * O.margin < lo);
-    };
-    const bool near = meets(Co.s.x, Co.d.x, Co.a.x, xo.x, Cn.s.x, Cn.d.x, Cn.a.x, xn.x, O.box_lo[0], O.box_hi[0]) &&
-                      meets(Co.s.y, Co.d.y, Co.a.y, xo.y, Cn.s.y, Cn.d.y, Cn.a.y, xn.y, O.box_lo[1], O.box_hi[1]) &&
-                      meets(Co.s.z, Co.d.z, Co.a.z, xo.z, Cn.s.z, Cn.d.z, Cn.a.z, xn.z, O.box_lo[2], O.box_hi[2]);
-    return near ? 0xffu : 0u;
+    sides |= (uint64_t)(side | other << 8) << (8 * f);
   }
+  return sides;
+}
+// The grids: whether any corner can meet an obstacle between the two poses, by the box around all the
+// corners against the faces' box.
+__device__ __forceinline__ bool near_box(const ObsView& O, const Corners& Co, f3 xo, const Corners& Cn, f3 xn) {
+  if (O.n_always != 0) return true;
+  // a corner's offset is at most max(|s|, |d|) + |a| in each row
+  auto meets = [&](float s0, float d0, float a0, float x0, float s1, float d1, float a1, float x1, float lo, float hi) {
+    const float e0 = fmaxf(fabsf(s0), fabsf(d0)) + fabsf(a0), e1 = fmaxf(fabsf(s1), fabsf(d1)) + fabsf(a1);
+    // 2 margin: the corners' own test grows by one; the other covers the rounding of these sums (the
+    // margin is at least 1e-4 of the largest obstacle coordinate)
+    return !(fminf(x0 - e0, x1 - e1) - 2.0f * O.margin > hi) && !(fmaxf(x0 + e0, x1 + e1) + 2.0f * O.margin < lo);
+  };
+  return meets(Co.s.x, Co.d.x, Co.a.x, xo.x, Cn.s.x, Cn.d.x, Cn.a.x, xn.x, O.box_lo[0], O.box_hi[0]) &&
+         meets(Co.s.y, Co.d.y, Co.a.y, xo.y, Cn.s.y, Cn.d.y, Cn.a.y, xn.y, O.box_lo[1], O.box_hi[1]) &&
+         meets(Co.s.z, Co.d.z, Co.a.z, xo.z, Cn.s.z, Cn.d.z, Cn.a.z, xn.z, O.box_lo[2], O.box_hi[2]);
 }
 
 // The face that a segment hits first (first_hit), and the face itself.
@@ -190,16 +192,51 @@ __device__ __forceinline__ bool hit_face(const ObsView& O, f3 op, f3 np, float d
   }
 }
 
+// What a step forms of its poses early and needs again only where a corner hits, in the lane's own words of
+// LDS: the old pose's world inertia, angular velocity and velocity, and the corners of both poses (the new
+// one's are the next step's old ones).  Held in registers it would cost a third wave a SIMD; formed again
+// it was 260 operations a step with a hit.  The clobbers keep it from staying in registers all the same.
+struct Kept {
+  float4 (*at)[kBlock];
+  __device__ float4& word(int k) const { return at[k][threadIdx.x]; }
+  __device__ void pose(const M3& I, f3 w, f3 vel) const {
+    word(0) = make_float4(I.c[0].x, I.c[0].y, I.c[0].z, w.x);
+    word(1) = make_float4(I.c[1].x, I.c[1].y, I.c[1].z, w.y);
+    word(2) = make_float4(I.c[2].x, I.c[2].y, I.c[2].z, w.z);
+    word(3) = make_float4(vel.x, vel.y, vel.z, 0.0f);
+  }
+  __device__ void get_pose(M3& I, f3& w, f3& vel) const {
+    asm volatile("" ::: "memory");
+    const float4 a = word(0), b = word(1), c = word(2), d = word(3);
+    I = M3{{f3{a.x, a.y, a.z}, f3{b.x, b.y, b.z}, f3{c.x, c.y, c.z}}};
+    w = f3{a.w, b.w, c.w};
+    vel = f3{d.x, d.y, d.z};
+  }
+  __device__ void corners(uint32_t which, const Corners& C) const {
+    word(4 + 3 * which) = make_float4(C.s.x, C.s.y, C.s.z, 0.0f);
+    word(5 + 3 * which) = make_float4(C.d.x, C.d.y, C.d.z, 0.0f);
+    word(6 + 3 * which) = make_float4(C.a.x, C.a.y, C.a.z, 0.0f);
+  }
+  __device__ Corners get_corners(uint32_t which) const {
+    asm volatile("" ::: "memory");
+    const float4 s = word(4 + 3 * which), d = word(5 + 3 * which), a = word(6 + 3 * which);
+    return Corners{f3{s.x, s.y, s.z}, f3{d.x, d.y, d.z}, f3{a.x, a.y, a.z}};
+  }
+};
+
 // `steps` steps of every body, one thread per body, the record in registers from the first to the last
 // (bodies do not interact) and stored in place: the 13 fields that change, and the others only where
-// they hold something else than what the reference leaves there.  Bound by vector issue (~1,400
-// operations a body-step in free fall): 1,048,576 cubes 30 us a step falling and 44 lying on a floor,
+// they hold something else than what the reference leaves there.  Bound by vector issue (~1,250
+// operations a body-step in free fall): 1,048,576 cubes 27.6 us a step falling and 39.2 lying on a floor,
 // where a launch per step, the record through memory each time and eight obstacle searches a body took
-// 71 and 74; 131,072 cubes 4.7 and 7.7 (15.4 and 18.3); below ~20,000, one wave's chain, 3.5 and 5.5.
+// 71 and 74 (30.4 and 42.7 before the corners' sides and the old pose's values were carried); 131,072
+// cubes 4.4 and 7.2 (15.4 and 18.3); below ~20,000, one wave's chain, 3.1 and 5.2.
 template <bool GRID>
 __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ rec, uint32_t n, uint32_t pitch,
                                                              RigidParams P, ObsView O, uint32_t steps) {
   const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
+  __shared__ float4 s_kept[10][kBlock];
+  const Kept keep{s_kept};
   if (b >= n) return;
   // one coalesced wavefront access: a uniform base per field and a 32-bit byte offset per lane
   auto field = [&](int k) -> float& { return *(float*)((char*)(rec + (size_t)k * pitch) + b * 4u); };
@@ -213,6 +250,13 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
   if (steps != 0 && (bits(F) | bits(tau)) != 0u)
     for (int k = 23; k < kRigidRecord; ++k) field(k) = 0.0f;
   const float h = P.dt;
+  // the sides on which a step's last pose left the corners are the next step's old ones
+  uint64_t sides = 0;
+  if (steps != 0 && O.n_faces != 0) {
+    const Corners C = corners_of(from_quat(S.q));
+    keep.corners(0, C);
+    if (!GRID) sides = corner_sides(O, C, S.x);
+  }
   for (uint32_t step = 0; step < steps; ++step) {
     // accumulate_forces, accumulate_torques
     F = add(F, P.gravity);
@@ -220,7 +264,12 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
     Body T;
     f3 dx;
     Q dq;
-    derivative(S, m, I, dx, dq);
+    {
+      M3 I_old;
+      f3 w;
+      derivative(S, m, I, dx, dq, I_old, w);
+      keep.pose(I_old, w, dx);
+    }
     const f3 z = f3{0.0f, 0.0f, 0.0f};
     if (P.integration == FP_EULER) {  // S + S' h (state.rs:75-83)
       T = Body{axpy(S.x, h, dx), axpy(S.q, h, dq), axpy(S.p, h, F), axpy(S.l, h, tau)};
@@ -257,24 +306,33 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
     }
     // update_state: the cube's vertices against the obstacles
     if (O.n_faces != 0) {
-      uint32_t near = may_hit<GRID>(O, corners_of(from_quat(S.q)), S.x, corners_of(from_quat(T.q)), T.x);
+      // the corners (bit k: corner k) that can meet an obstacle: with few faces, those that change sides
+      // of some face's plane; with the grids, all or none
+      uint32_t near = 0;
+      const uint32_t was = step & 1u, is = was ^ 1u;
+      {
+        const Corners C = corners_of(from_quat(T.q));
+        keep.corners(is, C);
+        if constexpr (GRID) {
+          near = near_box(O, keep.get_corners(was), S.x, C, T.x) ? 0xffu : 0u;
+        } else {
+          const uint64_t now = corner_sides(O, C, T.x);
+          uint64_t crossed = now ^ sides;
+          sides = now;
+          crossed |= crossed >> 32;
+          near = (uint32_t)crossed | (uint32_t)crossed >> 16;
+          near = (near | near >> 8) & 0xffu;
+        }
+      }
       if (near != 0) {
-        // the corners are formed again (opaque rotations), not held across the test above
-        Q q_old = S.q, q_new = T.q;
-        settle(q_old);
-        settle(q_new);
-        const Corners Co = corners_of(from_quat(q_old)), Cn = corners_of(from_quat(q_new));
+        const Corners Co = keep.get_corners(was), Cn = keep.get_corners(is);
         const f3 x_new = T.x;
         // what the response needs of the old pose: once for the few-face scenes, whose marked corners mostly
         // hit, and per hit with the grids, where the search needs the registers
         M3 I_old;
         f3 vel, w;
-        auto pose = [&] {
-          I_old = inertia_inv(q_old, I);
-          vel = ExactMath::div3(S.p, m);
-          w = mv(I_old, S.l);
-        };
-        if (!GRID) pose();
+        if (!GRID) keep.get_pose(I_old, w, vel);
+        bool moved = false;
         // each lane its own marked corners in ascending order: as many rounds as the body with the most
         // has, not eight
         while (near != 0) {
@@ -283,10 +341,7 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
           const f3 op = corner_of_lane(Co, S.x, k), np = corner_of_lane(Cn, x_new, k);
           f3 nrm, v0;
           if (!hit_face<GRID>(O, op, np, P.dt_d, nrm, v0)) continue;
-          if (GRID) {
-            settle(q_old);
-            pose();
-          }
+          if (GRID) keep.get_pose(I_old, w, vel);
           const float od = dot(sub(op, v0), nrm), nd = dot(sub(np, v0), nrm);
           const f3 r = sub(op, S.x);
           const float frac = od / (od - nd);
@@ -298,7 +353,9 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
           T.x = add(sub(cp, r), smul(0.0001f * 2.0f, nrm));  // consts::EPSILON * 2.0
           T.p = add(T.p, imp);  // apply_impulse (:38-41)
           T.l = add(T.l, cross(r, imp));
+          moved = true;
         }
+        if (!GRID && moved) sides = corner_sides(O, Cn, T.x);
       }
     }
     S = T;
