@@ -12,7 +12,9 @@
 // dependent layers) rather than a rate.  The layer-by-layer form this replaces launched 22 kernels a
 // step, wrote every f32 pre-activation to HBM and formed each weight gradient in four workgroups
 // that walked the whole batch: a call that sets the parameters, takes 8 steps of 16,384 rows and reads
-// the parameters back took 65.3 ms, and takes 0.50 ms in this form.
+// the parameters back took 65.3 ms, and takes 0.43 ms in this form.  (The chain kernel itself took 30 us
+// while its weights were staged a load at a time and the workgroup waited at every layer, and 21.6 now.  The
+// weight kernel reads the 32 MB workspace in 15 us; four blocks in flight instead of one did not change it.)
 //
 // Each MFMA accumulates the same 32-wide K blocks in the same order from zero, biases are added
 // afterwards and activations are rounded to bf16 where they always were, so every per-row value
@@ -40,16 +42,36 @@ __device__ __forceinline__ u32x2 pack4(const __bf16 (&h)[4]) {
   return q;
 }
 
-// Stages `rows` rows of K bf16 (16-byte units) into LDS rows of `ld` elements, zero up to kpad.
-template <int K, int KPAD, int LD, int THREADS>
-__device__ __forceinline__ void stage_rows(__bf16* dst, const __bf16* __restrict__ src, int rows, int pad_rows) {
-  constexpr int kU = KPAD / 8;
-  for (int e = threadIdx.x; e < pad_rows * kU; e += THREADS) {
-    const int r = e / kU, u = e - r * kU;
-    uint4 q = make_uint4(0, 0, 0, 0);
-    if (r < rows && u < K / 8) q = *reinterpret_cast<const uint4*>(src + r * K + 8 * u);
-    *reinterpret_cast<uint4*>(dst + r * LD + 8 * u) = q;
+// `ROWS` rows of K bf16 (16-byte units) on their way to LDS rows of LD elements, zero up to KPAD: every
+// load of a thread is issued by `load`, before the first is waited for by `store` (a load, its wait and
+// its LDS write in turn cost the latency 24 times).
+template <int K, int KPAD, int LD, int ROWS, int THREADS>
+struct Staged {
+  static constexpr int kU = KPAD / 8, kRounds = (ROWS * kU + THREADS - 1) / THREADS;
+  uint4 q[kRounds];
+  __device__ __forceinline__ void load(const __bf16* __restrict__ src, int rows) {
+#pragma unroll
+    for (int j = 0; j < kRounds; ++j) {
+      const int e = threadIdx.x + j * THREADS, r = e / kU, u = e - r * kU;
+      q[j] = make_uint4(0, 0, 0, 0);
+      if (r < rows && u < K / 8) q[j] = *reinterpret_cast<const uint4*>(src + r * K + 8 * u);
+    }
   }
+  __device__ __forceinline__ void store(__bf16* dst) const {
+#pragma unroll
+    for (int j = 0; j < kRounds; ++j) {
+      const int e = threadIdx.x + j * THREADS, r = e / kU, u = e - r * kU;
+      if (ROWS * kU % THREADS == 0 || r < ROWS) *reinterpret_cast<uint4*>(dst + r * LD + 8 * u) = q[j];
+    }
+  }
+};
+
+// Between a wave's LDS writes and its own reads of them (its activations are its own: no other wave waits).
+__device__ __forceinline__ void own_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 template <int WAVES>
@@ -59,6 +81,7 @@ __global__ void __launch_bounds__(64 * WAVES) train_chain_kernel(TrainBatch A) {
   __shared__ uint4 s_act[WAVES][kActBytes / 16];
   __shared__ __bf16 s_dy[WAVES][16][4];
   __shared__ float s_loss[WAVES];
+  __shared__ float s_bias[3][kHid];
   char* img = reinterpret_cast<char*>(s_img);
   __bf16 *W1 = reinterpret_cast<__bf16*>(img + kImgW1), *W2 = reinterpret_cast<__bf16*>(img + kImgW2),
          *W3 = reinterpret_cast<__bf16*>(img + kImgW3), *W4 = reinterpret_cast<__bf16*>(img + kImgW4);
@@ -81,26 +104,51 @@ __global__ void __launch_bounds__(64 * WAVES) train_chain_kernel(TrainBatch A) {
   };
   bf16x8 xf[3];
   features(xf);
-  stage_rows<kFeat, 96, kLd1, kThreads>(W1, A.wb + kOffW1, kHid, kHid);
-  stage_rows<kHid, kHid, kLd, kThreads>(W2, A.wb + kOffW2, kHid, kHid);
-  stage_rows<kHid, kHid, kLd, kThreads>(W3, A.wb + kOffW3, kHid, kHid);
-  stage_rows<kHid, kHid, kLd, kThreads>(W4, A.wb + kOffW4, kOut, 16);
-  __syncthreads();
+  {
+    Staged<kFeat, 96, kLd1, kHid, kThreads> w1;
+    Staged<kHid, kHid, kLd, kHid, kThreads> w2, w3;
+    Staged<kHid, kHid, kLd, 16, kThreads> w4;
+    w1.load(A.wb + kOffW1, kHid);
+    w2.load(A.wb + kOffW2, kHid);
+    w3.load(A.wb + kOffW3, kHid);
+    w4.load(A.wb + kOffW4, kOut);
+    for (int k = threadIdx.x; k < 3 * kHid; k += kThreads) {
+      const int l = k / kHid, n = k - l * kHid;
+      s_bias[l][n] = A.P[(l == 0 ? kOffB1 : l == 1 ? kOffB2 : kOffB3) + n];
+    }
+    w1.store(W1);
+    w2.store(W2);
+    w3.store(W3);
+    w4.store(W4);
+  }
+  // the targets of the lane's output rows (the eight-wave form has no registers to hold them)
+  auto target_of = [&](int r) {
+    const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)src, 4 * g + r, 64),
+                   hi = (uint32_t)__shfl((int)(uint32_t)(src >> 32), 4 * g + r, 64);
+    const uint64_t from = (uint64_t)hi << 32 | lo;
+    return row0 + 4 * g + r < A.rows && col < kOut ? A.T[from * kOut + col] : 0.0f;
+  };
+  float target[4];
+  if constexpr (WAVES == 4)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) target[r] = target_of(r);
 
   const size_t pitch = (size_t)A.pitch;
   // the lane's four values of an operand row to the workspace (the grid covers the pitch); rows past
   // the batch are stored as zero
-  auto put = [&](int operand_row, const __bf16(&h)[4]) {
+  // (a uniform base and a 32-bit byte offset per lane: 16 rows of the pitch are below 4 GB)
+  const uint32_t put_at = 2u * ((uint32_t)col * (uint32_t)A.pitch + (uint32_t)(row0 + 4 * g));
+  auto put = [&](int operand_rows, const __bf16(&h)[4]) {
     __bf16 v[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] = row0 + 4 * g + r < A.rows ? h[r] : (__bf16)0.0f;
-    *reinterpret_cast<u32x2*>(A.tr + (size_t)operand_row * pitch + row0 + 4 * g) = pack4(v);
+    *reinterpret_cast<u32x2*>(reinterpret_cast<char*>(A.tr + (size_t)operand_rows * pitch) + put_at) = pack4(v);
   };
   f32x4 z1[8], z2[8], z3[8];
   bf16x8 hf[4];
   // activations of one layer from its pre-activations: to LDS (row-major, the next operand) and to
   // the workspace (transposed)
-  auto activate = [&](f32x4(&z)[8], const float* bias, int tr_row) {
+  auto activate = [&](f32x4(&z)[8], const float (&bias)[kHid], int tr_row) {
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt) {
       const float b = bias[16 * mt + col];
@@ -111,7 +159,7 @@ __global__ void __launch_bounds__(64 * WAVES) train_chain_kernel(TrainBatch A) {
         h[r] = (__bf16)gelu(z[mt][r]);
         act[(4 * g + r) * kLd + 16 * mt + col] = h[r];
       }
-      put(tr_row + 16 * mt + col, h);
+      put(tr_row + 16 * mt, h);
     }
   };
   auto fragments = [&]() {
@@ -128,6 +176,19 @@ __global__ void __launch_bounds__(64 * WAVES) train_chain_kernel(TrainBatch A) {
       z[mt] = acc;
     }
   };
+  // the features, transposed
+#pragma unroll
+  for (int kb = 0; kb < 3; ++kb) *reinterpret_cast<bf16x8*>(act + col * kLd + kb * 32 + 8 * g) = xf[kb];
+  own_lds();
+#pragma unroll
+  for (int mt = 0; mt < 5; ++mt) {
+    __bf16 x[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[r] = act[(4 * g + r) * kLd + 16 * mt + col];
+    put(kTrX + 16 * mt, x);
+  }
+  own_lds();
+  __syncthreads();  // the weights are staged
 #pragma unroll
   for (int mt = 0; mt < 8; ++mt) {
     f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -136,18 +197,18 @@ __global__ void __launch_bounds__(64 * WAVES) train_chain_kernel(TrainBatch A) {
       acc = mfma(xf[kb], *reinterpret_cast<const bf16x8*>(W1 + (16 * mt + col) * kLd1 + kb * 32 + 8 * g), acc);
     z1[mt] = acc;
   }
-  activate(z1, A.P + kOffB1, kTrH1);
-  __syncthreads();
+  activate(z1, s_bias[0], kTrH1);
+  own_lds();
   fragments();
-  __syncthreads();
+  own_lds();
   layer(W2, z2);
-  activate(z2, A.P + kOffB2, kTrH2);
-  __syncthreads();
+  activate(z2, s_bias[1], kTrH2);
+  own_lds();
   fragments();
-  __syncthreads();
+  own_lds();
   layer(W3, z3);
-  activate(z3, A.P + kOffB3, kTrH3);
-  __syncthreads();
+  activate(z3, s_bias[2], kTrH3);
+  own_lds();
   fragments();
   f32x4 y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -157,31 +218,36 @@ __global__ void __launch_bounds__(64 * WAVES) train_chain_kernel(TrainBatch A) {
   float e2 = 0.0f;
   {
     const float b4 = col < kOut ? A.P[kOffB4 + col] : 0.0f;
+    if constexpr (WAVES != 4)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) target[r] = target_of(r);
     __bf16 d4[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int row = row0 + 4 * g + r;
-      const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)src, 4 * g + r, 64),
-                     hi = (uint32_t)__shfl((int)(uint32_t)(src >> 32), 4 * g + r, 64);
-      const uint64_t from = (uint64_t)hi << 32 | lo;
       d4[r] = (__bf16)0.0f;
       if (row < A.rows && col < kOut) {
         const float v = y[r] + b4;
         if (A.Y) A.Y[(size_t)row * kOut + col] = v;
-        const float d = v - A.T[from * kOut + col];
+        const float d = v - target[r];
         e2 += d * d;
         d4[r] = (__bf16)(2.0f * d / (3.0f * (float)A.rows));
       }
       if (col < 4) s_dy[wave][4 * g + r][col] = d4[r];
     }
-    put(kTrY + col, d4);  // rows 3..15 of the operand are zero
+    put(kTrY, d4);  // rows 3..15 of the operand are zero
   }
 #pragma unroll
   for (int w = 32; w > 0; w >>= 1) e2 += __shfl_xor(e2, w, 64);
   if (lane == 0) s_loss[wave] = e2;
   __syncthreads();  // every wave is done with the forward weights
-  stage_rows<kHid, kHid, kLd, kThreads>(W3t, A.wbt + kHid * kHid, kHid, kHid);
-  stage_rows<kHid, kHid, kLd, kThreads>(W2t, A.wbt, kHid, kHid);
+  {
+    Staged<kHid, kHid, kLd, kHid, kThreads> w3t, w2t;
+    w3t.load(A.wbt + kHid * kHid, kHid);
+    w2t.load(A.wbt, kHid);
+    w3t.store(W3t);
+    w2t.store(W2t);
+  }
   if (threadIdx.x == 0) {
     float s = 0.0f;
 #pragma unroll
@@ -210,32 +276,20 @@ __global__ void __launch_bounds__(64 * WAVES) train_chain_kernel(TrainBatch A) {
         d[r] = (__bf16)(dh[mt][r] * gelu_grad(z[mt][r]));
         if (next) act[(4 * g + r) * kLd + 16 * mt + col] = d[r];
       }
-      put(tr_row + 16 * mt + col, d);
+      put(tr_row + 16 * mt, d);
     }
   };
   backward(z3, kTrZ3, true);
-  __syncthreads();  // also: the transposed weights are staged
+  __syncthreads();  // the transposed weights are staged
   fragments();
-  __syncthreads();
+  own_lds();
   layer(W3t, dh);
   backward(z2, kTrZ2, true);
-  __syncthreads();
+  own_lds();
   fragments();
-  __syncthreads();
+  own_lds();
   layer(W2t, dh);
   backward(z1, kTrZ1, false);
-  // the features, transposed (read again: kept, they would cost the eight-wave form its registers)
-  features(xf);
-#pragma unroll
-  for (int kb = 0; kb < 3; ++kb) *reinterpret_cast<bf16x8*>(act + col * kLd + kb * 32 + 8 * g) = xf[kb];
-  __syncthreads();
-#pragma unroll
-  for (int mt = 0; mt < 5; ++mt) {
-    __bf16 x[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) x[r] = act[(4 * g + r) * kLd + 16 * mt + col];
-    put(kTrX + 16 * mt + col, x);
-  }
 }
 
 // One layer's gradient over one slice of the batch: dW[n][k] = sum over rows of dZ[n] H[k], and
