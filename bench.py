@@ -44,7 +44,7 @@ COMMON = ["step_device.hpp", "vec.hpp", "exact_ops.hpp", "fdlibm_atan2f.hpp", "k
 KERNEL_SOURCES = {
     # sim.cpp deals the tiles to the XCDs, which sets how often halo rows are fetched twice;
     # obstacles.cpp builds the broad-phase grids the collision search walks
-    "grid_tiled_kernel<ExactMath,16,16>": ["grid_tiled.hip", "obstacles.cpp", "sim.cpp"] + COMMON,
+    "grid_tiled_kernel<ExactMath,16,16>": ["grid_tiled.hip", "grid_tile_core.hpp", "obstacles.cpp", "sim.cpp"] + COMMON,
     "grid_fast_kernel<15,15>": ["grid_fast.hip", "grid_fast_core.hpp", "grid_fast.hpp", "obstacles.cpp", "sim.cpp"] + COMMON,
     "patch_kernel<ExactMath>": ["kernels.hip"] + COMMON,
 }
@@ -52,7 +52,19 @@ KERNEL_SOURCES = {
 # FETCH_SIZE and WRITE_SIZE in KiB, each scaled by what the same counter reads for the calibration
 # copy (bench.py --only copy: 2.000 and 1.000); SQ_INSTS_VALU and SQ_WAVES summed over the chip and
 # GRBM_GUI_ACTIVE summed over the 8 XCDs (the commands are in the profiles named)
-MEASURED = {}
+MEASURED = {
+    ("grid_tiled_kernel<ExactMath,16,16>", "cloth1024"): {
+        "src_sha": "b6283279234d70d0", "fetch_kib": 16062, "write_kib": 24578,
+        "valu_insts": 2.6680e7, "waves": 16384, "grbm_gui_active": 8.9018e5,
+        "profiles": ["profiles/grid_tiled_exact_cloth1024.md", "profiles/grid_tiled_cloth1024_pmc.md"]},
+    ("grid_fast_kernel<15,15>", "cloth1024"): {
+        "src_sha": "7e84dc1e72c2d368", "fetch_kib": 16218, "write_kib": 24734,
+        "valu_insts": 1.1356e7, "waves": 19044, "grbm_gui_active": 5.2896e5,
+        "profiles": ["profiles/grid_fast_cloth1024.md"]},
+    ("patch_kernel<ExactMath>", "icospheres64"): {
+        "src_sha": "575da6d694571edb", "fetch_kib": 165123, "write_kib": 50312,
+        "profiles": ["profiles/batched_and_surfaces.md"]},
+}
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0
 SIMDS, XCDS = 1024, 8
 
@@ -680,7 +692,8 @@ def rigid_scene(np, n, seed=0):
 
 
 RIGID_BODIES = 1 << 20
-RIGID_BYTES_PER_BODY_STEP = 2 * 29 * 4  # the 29-float record read and written once per body-step
+RIGID_BYTES_PER_BODY = 2 * 29 * 4  # the 29-float record read and written once per launch
+RIGID_STEPS_PER_LAUNCH = 64        # kRigidChunk of rigid.cpp: the record stays in registers between them
 
 
 def rigid_plain(args, np, fa):
@@ -704,13 +717,15 @@ def rigid_plain(args, np, fa):
     wall = time.perf_counter() - t0
     out = sim.states()
     kernel_avg_s = kernel_ms * 1e-3 / args.steps
-    bytes_step = RIGID_BYTES_PER_BODY_STEP * n
-    achieved = bytes_step / kernel_avg_s / 1e9
+    launches = -(-args.steps // RIGID_STEPS_PER_LAUNCH)
+    bytes_launch = RIGID_BYTES_PER_BODY * n
+    achieved = bytes_launch * launches / (kernel_ms * 1e-3) / 1e9
     rates = {"workload": f"rigidbody::Simulation::step of {n} unit cubes (random impulses, restitution 0) onto a "
                          f"ground plane, RK4 dt=1/600 s", "bodies": n, "steps": args.steps,
              "sim_s_per_s": args.steps * dt / wall, "ms_per_step": wall * 1e3 / args.steps,
              "body_steps_per_s": args.steps * n / wall, "kernel_avg_us": kernel_avg_s * 1e6,
-             "bytes_per_launch": bytes_step, "achieved_gbs": achieved, "hbm_frac": achieved / HBM_PEAK_GBS,
+             "launches": launches,
+             "bytes_per_launch": bytes_launch, "achieved_gbs": achieved, "hbm_frac": achieved / HBM_PEAK_GBS,
              "finite": bool(np.isfinite(out).all())}
     return rates, (pos, mass, floor), rec, dt
 
@@ -747,7 +762,7 @@ def bench_rigid(args, np, fa, wl):
         "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": rates["workload"], "bodies": n},
         "body_steps_per_s": rates["body_steps_per_s"],
-        "roofline": {"bound": "hbm", "achieved": rates["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
+        "roofline": {"bound": "valu", "achieved": rates["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": rates["hbm_frac"], "traffic": None, "kernel_avg_us": rates["kernel_avg_us"],
                      "bytes_per_launch": rates["bytes_per_launch"]},
         "cpu_baseline": cpu,
