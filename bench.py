@@ -54,15 +54,15 @@ KERNEL_SOURCES = {
 # GRBM_GUI_ACTIVE summed over the 8 XCDs (the commands are in the profiles named)
 MEASURED = {
     ("grid_tiled_kernel<ExactMath,16,16>", "cloth1024"): {
-        "src_sha": "b6283279234d70d0", "fetch_kib": 16062, "write_kib": 24578,
-        "valu_insts": 2.6680e7, "waves": 16384, "grbm_gui_active": 8.9018e5,
+        "src_sha": "44c6e11c38609e71", "fetch_kib": 16043, "write_kib": 24577,
+        "valu_insts": 2.6651e7, "waves": 16384, "grbm_gui_active": 8.8612e5,
         "profiles": ["profiles/grid_tiled_exact_cloth1024.md", "profiles/grid_tiled_cloth1024_pmc.md"]},
     ("grid_fast_kernel<15,15>", "cloth1024"): {
-        "src_sha": "7e84dc1e72c2d368", "fetch_kib": 16218, "write_kib": 24734,
-        "valu_insts": 1.1356e7, "waves": 19044, "grbm_gui_active": 5.2896e5,
+        "src_sha": "6cd356afb506531a", "fetch_kib": 16218, "write_kib": 24734,
+        "valu_insts": 1.1358e7, "waves": 19044, "grbm_gui_active": 5.2546e5,
         "profiles": ["profiles/grid_fast_cloth1024.md"]},
     ("patch_kernel<ExactMath>", "icospheres64"): {
-        "src_sha": "575da6d694571edb", "fetch_kib": 165123, "write_kib": 50312,
+        "src_sha": "2906e54087b1bb00", "fetch_kib": 165096, "write_kib": 50329,
         "profiles": ["profiles/batched_and_surfaces.md"]},
 }
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0

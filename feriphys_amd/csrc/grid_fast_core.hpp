@@ -194,15 +194,6 @@ FP_HD void phase0(Lds<TR, TC>& L, const StepArgs& A, const ClothView& G, int r0,
                     *(const float*)(bu + ob)};
       w[k] = float2{*(const float*)(bv + ob), *(const float*)(bw + ob)};
     }
-#pragma unroll
-    for (int k = 0; k < RND; ++k) {
-      const int e = tid + k * nthreads;
-      if (e < NS) {
-        FP_LDS_CHECK(e >= 0 && e < NS);
-        L.pv[e] = q[k];
-        L.vw[e] = w[k];
-      }
-    }
   } else {
 #pragma unroll
     for (int k = 0; k < RND; ++k) {
@@ -212,17 +203,6 @@ FP_HD void phase0(Lds<TR, TC>& L, const StepArgs& A, const ClothView& G, int r0,
       const uint32_t g = G.base + (uint32_t)(r * C + c);
       q[k] = float4{A.in.x[g], A.in.y[g], A.in.z[g], A.in.vx[g]};
       w[k] = float2{A.in.vy[g], A.in.vz[g]};
-    }
-#pragma unroll
-    for (int k = 0; k < RND; ++k) {
-      const int e = tid + k * nthreads;
-      const int lr = e / S::SW, lc = e - lr * S::SW;
-      const int r = r0 - 2 + lr, c = c0 - 2 + lc;
-      if (e < NS && r >= 0 && r < R && c >= 0 && c < C) {
-        FP_LDS_CHECK(e >= 0 && e < NS);
-        L.pv[e] = q[k];
-        L.vw[e] = w[k];
-      }
     }
   }
   // the tables are computed by the upper half of the workgroup (waves 2 and 3 of 4), which store one
@@ -237,6 +217,19 @@ FP_HD void phase0(Lds<TR, TC>& L, const StepArgs& A, const ClothView& G, int r0,
     const float d = cols ? grid_x(G, first) - grid_x(G, first + reach) : grid_y(G, first) - grid_y(G, first + reach);
     FP_LDS_CHECK(e >= 0 && e < S::NTAB);
     L.tab[e] = ktab(d, bend ? G.bk : G.tk, bend ? G.bc : G.tc);
+  }
+  // the states last: the tables are formed while they are on their way (32 x 32 vertices: 4.66 -> 4.48 us
+  // a step, 400 x 400: 7.1 -> 7.0, 1024 x 1024 the same)
+#pragma unroll
+  for (int k = 0; k < RND; ++k) {
+    const int e = tid + k * nthreads;
+    const int lr = e / S::SW, lc = e - lr * S::SW;
+    const int r = r0 - 2 + lr, c = c0 - 2 + lc;
+    if (e < NS && (INTERIOR || (r >= 0 && r < R && c >= 0 && c < C))) {
+      FP_LDS_CHECK(e >= 0 && e < NS);
+      L.pv[e] = q[k];
+      L.vw[e] = w[k];
+    }
   }
 }
 

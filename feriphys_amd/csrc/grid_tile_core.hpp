@@ -122,15 +122,6 @@ FP_HD void stage(Lds<TR, TC, ROOM>& L, const StepArgs& A, const ClothView& G, in
     q[k][0] = at(A.in.x); q[k][1] = at(A.in.y); q[k][2] = at(A.in.z);
     q[k][3] = at(A.in.vx); q[k][4] = at(A.in.vy); q[k][5] = at(A.in.vz);
   }
-#pragma unroll
-  for (int k = 0; k < RND; ++k) {
-    const int e = tid + k * NT, lr = e / S::SW, lc = e - lr * S::SW, r = r0 - 2 + lr, c = c0 - 2 + lc;
-    if (e < NS && (interior || (r >= 0 && r < R && c >= 0 && c < C))) {
-      float* row = &L.st[lr][lc];
-#pragma unroll
-      for (int f = 0; f < 6; ++f) row[f * S::SW] = q[k][f];
-    }
-  }
   for (int e = tid; e < kFdlEntries; e += nthreads) fdl_entry(e, L.atab[e]);
   // the constant tables, by the workgroup's last threads (the first ones may have a second round of
   // states): columns' struts, rows' struts, columns' bends, rows' bends
@@ -143,6 +134,17 @@ FP_HD void stage(Lds<TR, TC, ROOM>& L, const StepArgs& A, const ClothView& G, in
     const float d = (((float)first * G.spacing - o) + p) - (((float)second * G.spacing - o) + p);
     const KTab K = ktab(d, bend ? G.bk : G.tk, bend ? G.bc : G.tc);
     (cols ? (bend ? L.tbh : L.th) : (bend ? L.tbv : L.tv))[j] = K;
+  }
+  // the states last: the tables are formed while they are on their way (32 x 32 vertices: 5.1 -> 4.9 us a
+  // step, 256 x 256: 9.4 -> 9.1)
+#pragma unroll
+  for (int k = 0; k < RND; ++k) {
+    const int e = tid + k * NT, lr = e / S::SW, lc = e - lr * S::SW, r = r0 - 2 + lr, c = c0 - 2 + lc;
+    if (e < NS && (interior || (r >= 0 && r < R && c >= 0 && c < C))) {
+      float* row = &L.st[lr][lc];
+#pragma unroll
+      for (int f = 0; f < 6; ++f) row[f * S::SW] = q[k][f];
+    }
   }
 }
 

@@ -16,8 +16,8 @@ using gtile::CONSTANTS;
 // 64-vertex tiles, twelve waves: two of struts, one of struts reaching in, three of faces, six of
 // corners, and then one wave per force component.  Bound by its chain of dependent operations (the
 // longest task's ~190 and a component's ~90, against ~1,650 when one lane takes a vertex), the launch
-// and the two memory round trips: 5.1 us a step up to 128 x 128 vertices, where a lane per vertex took
-// 12.3 (and takes 9.0 now).
+// and the two memory round trips: 4.8 us a step on 64 x 64 vertices, 5.1 on 128 x 128, where a lane per
+// vertex took 12.3 (and takes 8.7 now).
 template <int MODE>
 __global__ void __launch_bounds__(768) grid_tiled_kernel_small(StepArgs A, const ClothView* __restrict__ cloths,
                                                                const TileRange* __restrict__ tiles) {

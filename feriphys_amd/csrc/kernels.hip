@@ -189,11 +189,11 @@ __device__ __forceinline__ void corner_group(f3 p, const PatchCorner* ce, const 
 // computed.  The groups that every lane of a wavefront has (all but a few vertices', on a regular
 // surface) run without masks, two abreast; what a slice's larger vertices have beyond is masked.
 //
-// Bound by the lanes' arithmetic (1,877 vector instructions a vertex in exact arithmetic, 684 of them
+// Bound by the lanes' arithmetic (1,879 vector instructions a wavefront in exact arithmetic, 684 of them
 // the 12 struts', 606 the six corners') with five workgroups at most on a CU, and on one mesh alone by
-// one wavefront's chain.  281,000 vertices in eight meshes, exact: 20.7 us a step, 24.3 when the strut
-// and corner entries (8 bytes each then) were looked up per vertex and waited for; fast 17.4 and 19.2.
-// 40,962 vertices: 9.6 and 12.4, fast 7.9 and 9.8.  Tried: four or six struts abreast or all entries
+// one wavefront's chain.  281,000 vertices in eight meshes, exact: 19.7 us a step, 24.3 when the strut
+// and corner entries (8 bytes each then) were looked up per vertex and waited for; fast 16.7 and 19.2.
+// 40,962 vertices: 9.2 and 12.4, fast 7.7 and 9.8.  Tried: four or six struts abreast or all entries
 // loaded up front 21.3 to 24, four lanes a vertex 34.7 (9.1 against 9.6 on 642 vertices), patches of 128
 // vertices 24.1.
 template <class M>
@@ -235,20 +235,31 @@ __global__ void __launch_bounds__(kBlock) patch_kernel(StepArgs A, CsrView T, co
   const uint32_t i = begin + (t < np ? t : np - 1);
   const float m = P.uniform_mass ? P.mass : A.mass[i];
   const bool pin = pinned(A.pins, i);
+  // (the tables while the states are on their way: 9.6 -> 9.2 us on 40,962 vertices)
+  const uint32_t u = kBlock - 1 - t;
+  const bool scan = !A.obs.use_grid && A.obs.n_faces <= kScanFaces;
+  float2 cls = make_float2(0.0f, 0.0f);
+  float4 obs = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (u < kPatchClasses) cls = T.p_cls[mesh * kPatchClasses + u];
+  if (scan && u < 4 * A.obs.n_faces) obs = reinterpret_cast<const float4*>(A.obs.faces)[u];
+  float4 sp[kRounds];
+  float2 sw[kRounds];
+#pragma unroll
+  for (uint32_t r = 0; r < kRounds; ++r) {
+    sp[r] = make_float4(S.x[g[r]], S.y[g[r]], S.z[g[r]], S.vx[g[r]]);
+    sw[r] = make_float2(S.vy[g[r]], S.vz[g[r]]);
+  }
+  if (M::kExact && t < kFdlEntries) fdl_entry(t, s_atan[t]);
+  if (u < kPatchClasses) s_cls[u] = cls;
+  if (scan && u < 4 * A.obs.n_faces) s_obs[u] = obs;
 #pragma unroll
   for (uint32_t r = 0; r < kRounds; ++r) {
     const uint32_t e = t + r * kBlock;
-    const float4 a = make_float4(S.x[g[r]], S.y[g[r]], S.z[g[r]], S.vx[g[r]]);
-    const float2 b = make_float2(S.vy[g[r]], S.vz[g[r]]);
     if (e < nl) {
-      s_p[e] = a;
-      s_w[e] = b;
+      s_p[e] = sp[r];
+      s_w[e] = sw[r];
     }
   }
-  if (t < kPatchClasses) s_cls[t] = T.p_cls[mesh * kPatchClasses + t];
-  const bool scan = !A.obs.use_grid && A.obs.n_faces <= kScanFaces;
-  if (scan && t < 4 * A.obs.n_faces) s_obs[t] = reinterpret_cast<const float4*>(A.obs.faces)[t];
-  if (M::kExact && t < kFdlEntries) fdl_entry(t, s_atan[t]);
   __syncthreads();
   auto Pl = [&](uint32_t l) { const float4 a = s_p[l]; return f3{a.x, a.y, a.z}; };
   auto Vl = [&](uint32_t l) { const float4 a = s_p[l]; const float2 b = s_w[l]; return f3{a.w, b.x, b.y}; };

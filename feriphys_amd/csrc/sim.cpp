@@ -210,8 +210,9 @@ uint64_t tile_count(const fp::ClothDesc& d, int shape) {
 }
 // Most 8x8 tiles that the exact kernel takes in place of the requested shapes: three to a CU.  Up to
 // there a step is one tile's chain of dependent work and the twelve-wave form is the faster (5.1 us
-// against 9.0 up to 128 x 128 vertices, 256 tiles; 8.1 against 9.4 at 192 x 192, 576 tiles); at 256 x
-// 256, 1,024 tiles, both take 9.6, and beyond it the larger tiles' fewer operations win.
+// against 8.7 up to 128 x 128 vertices, 256 tiles; 7.8 against 8.8 at 192 x 192, 576 tiles); at 224 x
+// 224, 784 tiles, both take 9.0, and beyond it the larger tiles' fewer operations win (256 x 256: 9.1
+// against 9.7).
 constexpr uint64_t kSmallTiles = 768;
 // Tiles resident at once: six workgroups on each of 256 CUs.
 constexpr uint64_t kResidentTiles = 1536;
