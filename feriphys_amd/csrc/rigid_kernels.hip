@@ -88,17 +88,20 @@ __device__ __forceinline__ f3 axpy(f3 a, float s, f3 b) { return f3{a.x + b.x * 
 __device__ __forceinline__ Q axpy(Q a, float s, Q b) { return Q{a.s + b.s * s, axpy(a.v, s, b.v)}; }
 
 // The world offsets of the cube's corners, R c with c = (+-1/2, +-1/2, +-1/2): with a = R / 2 (exact),
-// row by row (+-a0 +- a1) +- a2, where negation is exact: corner k is +-(s or d) +- a2 with s = a0 + a1
-// and d = a0 - a1.
+// row by row (+-a0 +- a1) +- a2, where negation is exact but for a zero's sign: corner k is +-(s or d) +- a2
+// with s = a0 + a1 and d = a0 - a1.
 struct Corners {
   f3 s, d, a;
 };
+// An offset that cancels to zero is +0 in the reference and may be -0 here, which a position of -0 would
+// let through into the corner, and from there into the side of a plane: corners are formed at x + 0.
+__device__ __forceinline__ f3 at_plus_zero(f3 x) { return add(x, f3{0.0f, 0.0f, 0.0f}); }
 __device__ __forceinline__ Corners corners_of(const M3& R) {
   const f3 a0 = smul(0.5f, R.c[0]), a1 = smul(0.5f, R.c[1]);
   return Corners{add(a0, a1), sub(a0, a1), smul(0.5f, R.c[2])};
 }
-// Corner k of kCubeCorner's order at body position x: the offsets are -(s - a), d + a, s + a, -(d - a),
-// -(s + a), d - a, s - a, -(d + a).
+// Corner k of kCubeCorner's order at body position x (of at_plus_zero): the offsets are -(s - a), d + a,
+// s + a, -(d - a), -(s + a), d - a, s - a, -(d + a).
 __device__ __forceinline__ f3 corner_at(const Corners& C, f3 x, int k) {
   const f3 b = k % 2 == 0 ? C.s : C.d;
   const bool minus = k == 0 || k == 3 || k == 5 || k == 6, negative = k == 0 || k == 3 || k == 4 || k == 7;
@@ -136,6 +139,7 @@ __device__ __forceinline__ ObsFace uniform_face(const ObsView& O, uint32_t f) {
 static_assert(kScanFaces * 8 <= 64, "a bit for each face and corner");
 __device__ __forceinline__ uint64_t corner_sides(const ObsView& O, const Corners& C, f3 x) {
   uint64_t sides = 0;
+  x = at_plus_zero(x);
   for (uint32_t f = 0; f < O.n_faces; f += 2) {  // two at a time, so that each corner is formed half as often
     // (of an odd number the last one twice)
     const ObsFace F = uniform_face(O, f), G = uniform_face(O, f + 1 < O.n_faces ? f + 1 : f);
@@ -326,7 +330,7 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
       }
       if (near != 0) {
         const Corners Co = keep.get_corners(was), Cn = keep.get_corners(is);
-        const f3 x_new = T.x;
+        const f3 x_old = at_plus_zero(S.x), x_new = at_plus_zero(T.x);
         // what the response needs of the old pose: once for the few-face scenes, whose marked corners mostly
         // hit, and per hit with the grids, where the search needs the registers
         M3 I_old;
@@ -338,7 +342,7 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
         while (near != 0) {
           const uint32_t k = (uint32_t)__builtin_ctz(near);
           near &= near - 1u;
-          const f3 op = corner_of_lane(Co, S.x, k), np = corner_of_lane(Cn, x_new, k);
+          const f3 op = corner_of_lane(Co, x_old, k), np = corner_of_lane(Cn, x_new, k);
           f3 nrm, v0;
           if (!hit_face<GRID>(O, op, np, P.dt_d, nrm, v0)) continue;
           if (GRID) keep.get_pose(I_old, w, vel);
