@@ -66,8 +66,9 @@ FP_HD float sqrt_f(float x) {
 }
 // The correctly rounded square root of x >= 2^-96 (sqrt_in_range of exact_ops.hpp): the hardware
 // reciprocal root r, g = x r and one Newton step with the exact residual x - g g, four operations where
-// choosing among the hardware root and its two neighbours took eight.  Zero (whose strut or face has no
-// direction anyway) gives NaN, tinier inputs a root within an ulp or two.
+// choosing among the hardware root and its two neighbours took eight.  Below 2^-96 it may be an ulp or two
+// off; zero, subnormal and infinite x give NaN (as did the forces of such struts with the hardware square
+// root, which takes a subnormal for zero).
 FP_HD float sqrt_cr(float x) {
 #ifdef __HIP_DEVICE_COMPILE__
   const float r = __builtin_amdgcn_rsqf(x), g = x * r;

@@ -3,6 +3,8 @@
 // training kernels are in surrogate_train.hip).
 #include "surrogate_device.hpp"
 
+#include <type_traits>
+
 #pragma clang fp contract(fast)
 
 namespace fp {
@@ -16,23 +18,30 @@ __device__ __forceinline__ void store_state(const SoA& o, uint32_t i, f3 x, f3 v
 
 // The 6 features of one slot: strain_scale * strain * d/|d| and (v_nbr - v) * H / L, from the
 // neighbour's position q and velocity w; zeros when `has` is false.  Branch-free, so that a caller
-// can issue every load of a pass before the first feature is computed.
-__device__ __forceinline__ void slot_feat_from(f3 p, f3 v, f3 q, f3 w, float rest, bool has, FeatParams fp, float* f) {
+// can issue every load of a pass before the first feature is computed.  The short root (exact but for
+// d2 < 2^-96, where it may be an ulp off) has no value for a subnormal d2, |d| < 1.1e-19: returns whether
+// that is so, and the features must then be formed again with GENERAL.
+template <bool GENERAL>
+__device__ __forceinline__ bool slot_feat_from(f3 p, f3 v, f3 q, f3 w, float rest, bool has, FeatParams fp, float* f) {
+  constexpr int kPositiveSubnormal = 0x080;
   const f3 d = sub(q, p);
   const float d2 = d.x * d.x + d.y * d.y + d.z * d.z;
-  const float len = sqrt_in_range(d2);  // (exact but for d2 < 2^-96, where it may be an ulp off)
+  const float len = GENERAL ? sqrt_rn(d2) : sqrt_in_range(d2);
   const float il = __builtin_amdgcn_rcpf(rest);
   const float st = (has && d2 > 0.0f) ? fp.strain_scale * ((len - rest) * il) * __builtin_amdgcn_rcpf(len) : 0.0f;
   const float hv = has ? fp.H * il : 0.0f;
   f[0] = st * d.x; f[1] = st * d.y; f[2] = st * d.z;
   f[3] = (w.x - v.x) * hv; f[4] = (w.y - v.y) * hv; f[5] = (w.z - v.z) * hv;
+  return !GENERAL && __builtin_amdgcn_classf(d2, kPositiveSubnormal);
 }
 
-__device__ __forceinline__ void slot_feat(const SoA& S, f3 p, f3 v, uint32_t self, SlotEnt e, FeatParams fp,
+template <bool GENERAL = true>
+__device__ __forceinline__ bool slot_feat(const SoA& S, f3 p, f3 v, uint32_t self, SlotEnt e, FeatParams fp,
                                           float* f) {
   const bool has = e.nbr != kNoSlot;
   const uint32_t nb = has ? e.nbr : self;
-  slot_feat_from(p, v, ld3(S.x, S.y, S.z, nb), ld3(S.vx, S.vy, S.vz, nb), has ? e.rest : 1.0f, has, fp, f);
+  return slot_feat_from<GENERAL>(p, v, ld3(S.x, S.y, S.z, nb), ld3(S.vx, S.vy, S.vz, nb), has ? e.rest : 1.0f, has, fp,
+                                 f);
 }
 
 __device__ __forceinline__ float unit_open(uint64_t h) { return ((float)(h >> 40) + 0.5f) * (1.0f / 16777216.0f); }
@@ -107,40 +116,49 @@ __global__ void __launch_bounds__(2048 / NT) sur_mlp_kernel(SoA S, const SlotEnt
     // features: lane group g computes slots 3g..3g+2 of its vertex (18 values, then 6 zeros), which
     // are its 8-element K slices of the three 32-wide K blocks of layer 1.  Every load is
     // unconditional (past-the-end columns read vertex n-1, empty slots the vertex itself; both are
-    // zeroed), so a pass's loads can all be in flight together.
+    // zeroed), so a pass's loads can all be in flight together.  A wavefront that meets a strut with a
+    // subnormal squared length forms all its features once more with the general root.
     bf16x8 B1[3][NT];
-    SlotEnt se[NT][3];
-    f3 p[NT], v[NT];
+    const auto features = [&](auto general) {
+      SlotEnt se[NT][3];
+      f3 p[NT], v[NT];
+      uint32_t first = v0 + col;
+      // (the rare second pass loads again what the first one had)
+      if constexpr (decltype(general)::value) asm volatile("" : "+v"(first));
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const uint32_t iv = v0 + nt * 16 + col;
-      const uint32_t i = iv < n ? iv : n - 1;
-      const SlotEnt* at = slots + slot_at(i, 3 * g);
-      p[nt] = ld3(S.x, S.y, S.z, i);
-      v[nt] = ld3(S.vx, S.vy, S.vz, i);
+      for (int nt = 0; nt < NT; ++nt) {
+        const uint32_t iv = first + nt * 16;
+        const uint32_t i = iv < n ? iv : n - 1;
+        const SlotEnt* at = slots + slot_at(i, 3 * g);
+        p[nt] = ld3(S.x, S.y, S.z, i);
+        v[nt] = ld3(S.vx, S.vy, S.vz, i);
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        se[nt][j] = at[64 * j];
-        se[nt][j].nbr = iv < n ? se[nt][j].nbr : kNoSlot;
+        for (int j = 0; j < 3; ++j) {
+          se[nt][j] = at[64 * j];
+          se[nt][j].nbr = iv < n ? se[nt][j].nbr : kNoSlot;
+        }
       }
-    }
+      bool again = false;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const uint32_t iv = v0 + nt * 16 + col;
-      const uint32_t i = iv < n ? iv : n - 1;
-      float f[24];
+      for (int nt = 0; nt < NT; ++nt) {
+        const uint32_t iv = first + nt * 16;
+        const uint32_t i = iv < n ? iv : n - 1;
+        float f[24];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        slot_feat(S, p[nt], v[nt], i, se[nt][j], fp, f + 6 * j);
-        __builtin_amdgcn_sched_barrier(0x20);  // loads may pass, arithmetic not: slots interleaved spill
+        for (int j = 0; j < 3; ++j) {
+          again = slot_feat<decltype(general)::value>(S, p[nt], v[nt], i, se[nt][j], fp, f + 6 * j) || again;
+          __builtin_amdgcn_sched_barrier(0x20);  // loads may pass, arithmetic not: slots interleaved spill
+        }
+#pragma unroll
+        for (int k = 18; k < 24; ++k) f[k] = 0.0f;
+#pragma unroll
+        for (int kb = 0; kb < 3; ++kb)
+#pragma unroll
+          for (int s = 0; s < 8; ++s) B1[kb][nt][s] = (__bf16)f[kb * 8 + s];
       }
-#pragma unroll
-      for (int k = 18; k < 24; ++k) f[k] = 0.0f;
-#pragma unroll
-      for (int kb = 0; kb < 3; ++kb)
-#pragma unroll
-        for (int s = 0; s < 8; ++s) B1[kb][nt][s] = (__bf16)f[kb * 8 + s];
-    }
+      return again;
+    };
+    if (__any(features(std::false_type{}))) features(std::true_type{});
     bf16x8 Bh[4][NT], Bg[4][NT];
     mfma_act_layer<3, kLd1, NT>(W1, Bias, B1, Bh, col, g);
     mfma_act_layer<4, kLd, NT>(W2, Bias + kHid, Bh, Bg, col, g);
