@@ -1,9 +1,9 @@
 // LDS-tiled step kernels for meshes built by Cloth::new (springy/cloth.rs:20-113) in the reference's
 // summation order, one workgroup per tile: a twelve-wave form for 64-vertex tiles, where a step is one
 // tile's chain of dependent work, and a lane per vertex for larger tiles, where it is vector issue
-// (the host's rule: build_block_lists in sim.cpp).  The per-vertex operations and their order are those of grid_kernel, so the EXACT form returns the
-// same bits as the reference.  HBM traffic: the state read once (plus halo rows that the L2 serves)
-// and written once.
+// (the host's rule: tile_rule.hpp).  The per-vertex operations and their order are those of grid_kernel,
+// so the EXACT form returns the same bits as the reference.  HBM traffic: the state read once (plus halo
+// rows that the L2 serves) and written once.
 #include "grid_tile_core.hpp"
 
 namespace fp {

@@ -136,7 +136,7 @@ struct TileRange {
 // TR x TC tile touches (TR+1) x (TC+1) quads; 15x15 and 7x31 make that exactly 256, one quad (two
 // faces) per thread in the face phase.
 // TILE_8x8 is not a caller's choice: the exact kernel takes it for simulations of few tiles (see
-// build_block_lists).
+// tile_rule.hpp).
 enum TileShape { TILE_15x15 = 0, TILE_7x31 = 1, TILE_16x16 = 2, N_TILE_SHAPES = 3, TILE_8x8 = 3, N_LAUNCH_SHAPES = 4 };
 constexpr int kTileRows[N_LAUNCH_SHAPES] = {15, 7, 16, 8};
 constexpr int kTileCols[N_LAUNCH_SHAPES] = {15, 31, 16, 8};

@@ -26,6 +26,7 @@
 
 #include "grid_fast.hpp"
 #include "sim_internal.hpp"
+#include "tile_rule.hpp"
 
 
 using namespace fpsim;
@@ -204,19 +205,6 @@ void cloth_tiles(uint32_t mesh, const fp::ClothDesc& d, int shape, std::vector<f
     for (uint32_t c = 0; c < d.cols; c += tc) out.push_back(fp::TileRange{mesh, r, c, (uint32_t)shape});
 }
 
-uint64_t tile_count(const fp::ClothDesc& d, int shape) {
-  const uint64_t tr = (uint64_t)fp::kTileRows[shape], tc = (uint64_t)fp::kTileCols[shape];
-  return ((d.rows + tr - 1) / tr) * ((d.cols + tc - 1) / tc);
-}
-// Most 8x8 tiles that the exact kernel takes in place of the requested shapes: three to a CU.  Up to
-// there a step is one tile's chain of dependent work and the twelve-wave form is the faster (5.1 us
-// against 8.7 up to 128 x 128 vertices, 256 tiles; 7.8 against 8.8 at 192 x 192, 576 tiles); at 224 x
-// 224, 784 tiles, both take 9.0, and beyond it the larger tiles' fewer operations win (256 x 256: 9.1
-// against 9.7).
-constexpr uint64_t kSmallTiles = 768;
-// Tiles resident at once: six workgroups on each of 256 CUs.
-constexpr uint64_t kResidentTiles = 1536;
-
 // Runs of the tile list per XCD (see xcd_order).
 constexpr size_t kTilePieces = 8;
 
@@ -245,37 +233,22 @@ std::vector<T> xcd_order(const std::vector<T>& t, size_t pieces = 1) {
 
 int build_block_lists(fp_sim* s) {
   // the lists depend on the kernel selection and, per mesh, on whether its masses are uniform and on
-  // its tile shape (topology, blocks and patches are fixed when the simulation is built)
+  // its tile shape and who chose it (topology, blocks and patches are fixed when the simulation is built)
   std::vector<int32_t> sig{s->kernel, s->math};
   for (const auto& m : s->meshes) {
     sig.push_back(m.uniform_mass ? 1 : 0);
-    sig.push_back(m.tile_shape);
+    sig.push_back(m.tile_chosen ? -1 - m.tile_shape : m.tile_shape);
   }
   if (sig == s->lists_sig) return FP_OK;
   std::vector<fp::BlockRange> g, c, cf, sb, sf;
   std::vector<fp::PatchRange> pl;
   std::vector<fp::TileRange> by_shape[fp::N_LAUNCH_SHAPES], all_tiles;
-  uint64_t n_small = 0;  // 8x8 tiles of all the cloths
-  for (const auto& m : s->meshes)
-    if (m.host.cloth.valid && m.uniform_mass) n_small += tile_count(m.host.cloth, fp::TILE_8x8);
-  const bool small = s->math == FP_MATH_EXACT && n_small <= kSmallTiles;
-  // Meshes of different tile shapes cost a launch per shape and step.  While all their tiles together are
-  // resident at once, a launch is one tile's latency and a second one as long again, so every mesh takes
-  // the shape that most tiles have.
-  const auto launched = [&](int shape) {
-    return s->math == FP_MATH_FAST && shape == fp::TILE_16x16 ? (int)fp::TILE_15x15 : shape;
-  };
-  uint64_t per_shape[fp::N_LAUNCH_SHAPES] = {};
+  std::vector<ClothTiles> cloths;
   for (const auto& m : s->meshes)
     if (m.host.cloth.valid && m.uniform_mass)
-      per_shape[launched(m.tile_shape)] += tile_count(m.host.cloth, launched(m.tile_shape));
-  int common = 0;
-  for (int sh = 1; sh < fp::N_TILE_SHAPES; ++sh)
-    if (per_shape[sh] > per_shape[common]) common = sh;
-  uint64_t n_common = 0;
-  for (const auto& m : s->meshes)
-    if (m.host.cloth.valid && m.uniform_mass) n_common += tile_count(m.host.cloth, common);
-  const bool one_shape = n_common <= kResidentTiles;
+      cloths.push_back(ClothTiles{m.host.cloth.rows, m.host.cloth.cols, m.tile_shape, m.tile_chosen});
+  const std::vector<int> shapes = launch_shapes(cloths, s->math == FP_MATH_FAST);
+  size_t cloth = 0;
   for (uint32_t mi = 0; mi < s->meshes.size(); ++mi) {
     MeshSlot& ms = s->meshes[mi];
     const bool grid_ok = ms.host.cloth.valid && ms.uniform_mass;
@@ -284,9 +257,8 @@ int build_block_lists(fp_sim* s) {
                                                        : MK_GRID_TILED;
     ms.tile_begin = ms.tile_end = (uint32_t)all_tiles.size();
     ms.on_patch = false;
+    if (grid_ok) ms.launch_shape = shapes[cloth++];
     if (ms.kernel == MK_GRID_TILED) {
-      // (the fast kernel has one quad per thread: 15x15 and 7x31 tiles; 16x16 becomes 15x15)
-      ms.launch_shape = small ? (int)fp::TILE_8x8 : one_shape ? common : launched(ms.tile_shape);
       std::vector<fp::TileRange> mt;
       cloth_tiles(mi, ms.host.cloth, ms.launch_shape, mt);
       by_shape[ms.launch_shape].insert(by_shape[ms.launch_shape].end(), mt.begin(), mt.end());
@@ -1096,10 +1068,19 @@ int fp_sim_autotune(fp_sim* s, uint32_t steps, int32_t* chosen_out) {
       if (m.kernel == MK_GRID_TILED && size_class(m.host.cloth) == cls) members.push_back(&m);
     if (members.empty()) continue;
     float best_ms = INFINITY;
-    int best = members[0]->tile_shape;
-    for (int shape = 0; shape < fp::N_TILE_SHAPES; ++shape) {
-      for (auto* m : members) m->tile_shape = shape;
-      if (int e = build_block_lists(s)) return e;
+    int best = 0;
+    const auto choose = [&](int shape) {  // -1: as if never chosen
+      for (auto* m : members) {
+        m->tile_chosen = shape >= 0;
+        m->tile_shape = shape >= 0 ? shape : default_tile_shape(m->host.cloth.rows, m->host.cloth.cols);
+      }
+      return build_block_lists(s);
+    };
+    // the library's own choice is a trial of its own where it is 8x8 tiles, which no caller can ask for
+    if (int e = choose(-1)) return e;
+    const bool own = members[0]->launch_shape == fp::TILE_8x8;
+    for (int shape = own ? -1 : 0; shape < fp::N_TILE_SHAPES; ++shape) {
+      if (int e = choose(shape)) return e;
       if (int e = restore()) return e;
       if (int e = run_steps(s, 2)) return e;  // warm-up
       float ms = 0.0f;
@@ -1110,10 +1091,9 @@ int fp_sim_autotune(fp_sim* s, uint32_t steps, int32_t* chosen_out) {
       HIP_TRY(hipEventElapsedTime(&ms, s->ev0, s->ev1));
       if (ms < best_ms) { best_ms = ms; best = shape; }
     }
-    for (auto* m : members) m->tile_shape = best;
-    chosen[cls] = best;
+    if (int e = choose(best)) return e;
+    chosen[cls] = members[0]->tile_shape;
   }
-  if (int e = build_block_lists(s)) return e;
   if (int e = restore()) return e;
   HIP_TRY(hipDeviceSynchronize());
   if (chosen_out)
@@ -1355,6 +1335,7 @@ int fp_sim_set_tile_shape(fp_sim* s, uint64_t mesh, int32_t shape) {
   if (shape < 0 || shape >= fp::N_TILE_SHAPES) return fail(FP_EINVAL, "unknown tile shape");
   HIP_TRY(hipStreamSynchronize(s->stream));
   s->meshes[mesh].tile_shape = shape;
+  s->meshes[mesh].tile_chosen = true;
   return build_block_lists(s);
 }
 

@@ -31,6 +31,7 @@ struct MeshSlot {
   bool uniform_mass = true;
   int kernel = MK_CSR;
   int tile_shape = fp::TILE_16x16;
+  bool tile_chosen = false;           // tile_shape was asked for, not the default
   int launch_shape = fp::TILE_16x16;  // the shape its tiles are built with under the current math form
   uint32_t blk_begin = 0, blk_end = 0;
   uint32_t fblk_begin = 0, fblk_end = 0;  // face blocks (range in fp_sim::h_face_blocks)

@@ -237,7 +237,12 @@ int fp_sim_set_torsion(fp_sim* sim, int32_t enabled);
 #define FP_MATH_FAST 1
 int fp_sim_set_kernel(fp_sim* sim, int32_t kernel, int32_t math);
 /* Tile shape of the LDS-tiled grid kernel for one cloth mesh (rows x columns per workgroup):
- * FP_TILE_15x15, FP_TILE_7x31 or FP_TILE_16x16.  The default is chosen from the cloth's size. */
+ * FP_TILE_15x15, FP_TILE_7x31 or FP_TILE_16x16.  The default is chosen from the cloth's size.  A shape
+ * that was set is the one that runs (FAST: 16x16 runs as 15x15).  Meshes left to the default may run
+ * in another: 8x8 tiles in small EXACT simulations, and one shape for all in simulations whose tiles
+ * are all resident at once.  EXACT results do not depend on the shape; FAST forces do in the last bits
+ * (the order of a vertex's sums at tile borders), also through which other meshes a simulation holds.
+ * fp_sim_get_tile_shape returns the set shape, or the default for the cloth's size. */
 #define FP_TILE_15x15 0
 #define FP_TILE_7x31 1
 #define FP_TILE_16x16 2
@@ -255,8 +260,11 @@ int fp_sim_get_tile_shape(const fp_sim* sim, uint64_t mesh, int32_t* shape);
 int fp_sim_get_mesh_kernel(const fp_sim* sim, uint64_t mesh, int32_t* kernel);
 /* Autotuner: meshes on the tiled grid kernel are grouped by size class (longer side < 16, < 32,
  * < 64, >= 64 vertices); for each class every tile shape is timed over `steps_per_trial` steps
- * (HIP events on the simulation's stream, state restored afterwards) and the fastest is kept.
- * chosen_out[4] (may be NULL) receives the shape per class (-1: no mesh in the class). */
+ * (HIP events on the simulation's stream, state restored afterwards) and the fastest is kept, as if
+ * set with fp_sim_set_tile_shape; where the library would run 8x8 tiles, those are timed as well, and
+ * if they are the fastest the class goes back to the default.  chosen_out[4] (may be NULL) receives the
+ * shape per class, as fp_sim_get_tile_shape returns it for the class's first mesh (-1: no mesh in the
+ * class). */
 int fp_sim_autotune(fp_sim* sim, uint32_t steps_per_trial, int32_t* chosen_out);
 /* n_steps of Simulation::step replayed from HIP graphs that capture `chunk` steps each (the
  * launch sequence of one chunk, captured once per state-buffer parity and reused until the
