@@ -213,19 +213,23 @@ grid_tiled_kernel(StepArgs A, const ClothView* __restrict__ cloths, const TileRa
   else gather_vertex<M, TR, TC, MODE, true>(L, A, P, C, r, c, lr, lc);
 }
 
+template <class M, int TR, int TC, int MODE>
+hipError_t launch_lanes(const StepArgs& a, const ClothView* cloths, const TileRange* tiles, uint32_t n, hipStream_t s) {
+  grid_tiled_kernel<M, TR, TC, MODE><<<dim3(n), dim3(kBlock), 0, s>>>(a, cloths, tiles);
+  return hipGetLastError();
+}
+
 template <int TR, int TC>
 hipError_t launch_shape(const StepArgs& a, const ClothView* cloths, const TileRange* tiles, uint32_t n, int mode,
                         hipStream_t s) {
-  const dim3 g(n), b(kBlock);
-  if (mode == MODE_STEP) grid_tiled_kernel<ExactMath, TR, TC, MODE_STEP><<<g, b, 0, s>>>(a, cloths, tiles);
-  else if (mode == MODE_FORCES) grid_tiled_kernel<ExactMath, TR, TC, MODE_FORCES><<<g, b, 0, s>>>(a, cloths, tiles);
-  else grid_tiled_kernel<FastMath, TR, TC, MODE_SURROGATE><<<g, b, 0, s>>>(a, cloths, tiles);
-  return hipGetLastError();
+  if (mode == MODE_STEP) return launch_lanes<ExactMath, TR, TC, MODE_STEP>(a, cloths, tiles, n, s);
+  if (mode == MODE_FORCES) return launch_lanes<ExactMath, TR, TC, MODE_FORCES>(a, cloths, tiles, n, s);
+  return launch_lanes<FastMath, TR, TC, MODE_SURROGATE>(a, cloths, tiles, n, s);
 }
 
 hipError_t launch_small(const StepArgs& a, const ClothView* cloths, const TileRange* tiles, uint32_t n, int mode,
                         hipStream_t s) {
-  if (mode == MODE_SURROGATE) return launch_shape<8, 8>(a, cloths, tiles, n, mode, s);
+  if (mode == MODE_SURROGATE) return launch_lanes<FastMath, 8, 8, MODE_SURROGATE>(a, cloths, tiles, n, s);
   if (mode == MODE_STEP) grid_tiled_kernel_small<MODE_STEP><<<dim3(n), dim3(768), 0, s>>>(a, cloths, tiles);
   else grid_tiled_kernel_small<MODE_FORCES><<<dim3(n), dim3(768), 0, s>>>(a, cloths, tiles);
   return hipGetLastError();
