@@ -629,11 +629,12 @@ hipError_t launch_csr(const StepArgs& a, const CsrView& t, const BlockRange* blo
 }
 
 // Every finite f32 x (grid-stride over all bit patterns): the exact kernels' shortened forms
-// against the operations they stand for, bad[0] rcp_rn(x) vs 1 / x and div_rn with x as divisor and
-// as dividend, bad[1] div_pi_rn(x) vs x / PI, bad[2] div3_rn(x) vs x / 3, bad[3] the branch-free
-// atan2 vs fdlibm's control flow at y = 1 and y = -1.7, and the corner weight's in-range form vs
-// the same, bad[4] sqrt_rn(x) and sqrt_rcp_rn(x) vs the compiler's correctly rounded sqrt and the
-// division (NaN payloads aside).
+// against the operations they stand for, bad[0] rcp_rn(x) vs 1 / x and div_rn and div3 with x as divisor
+// and as dividend, the other operand a constant or drawn by a hash of x over [2^-64, 2^64), bad[1]
+// div_pi_rn(x) vs x / PI, bad[2] div3_rn(x) vs x / 3, bad[3] the branch-free atan2 vs fdlibm's control
+// flow at y = 1 and y = -1.7, and the corner weight's in-range form vs the same, also with both operands
+// drawn, bad[4] sqrt_rn(x) and sqrt_rcp_rn(x) vs the compiler's correctly rounded sqrt and the division
+// (NaN payloads aside).
 __global__ void __launch_bounds__(kBlock) selftest_kernel(unsigned long long* __restrict__ bad) {
   unsigned long long b[5] = {0, 0, 0, 0, 0};
   auto bits = [](float f) { return __float_as_uint(f); };
@@ -647,6 +648,17 @@ __global__ void __launch_bounds__(kBlock) selftest_kernel(unsigned long long* __
     if (!__builtin_isfinite(x)) continue;
     b[0] += bits(rcp_rn(x)) != bits(1.0f / x);
     b[0] += differ(div_rn(1.7f, x), 1.7f / x) || differ(div_rn(x, -0.3f), x / -0.3f);
+    // two operands drawn over 128 octaves, significands and signs by other bits of the hash
+    uint64_t h = k * 0x9e3779b97f4a7c15ull;
+    h = (h ^ (h >> 32)) * 0xd6e8feb86659fd93ull;
+    h ^= h >> 32;
+    const auto draw = [](uint32_t r, uint32_t octave) {
+      return __uint_as_float((r & 0x807fffffu) | (octave % 128u + 63u) << 23);
+    };
+    const float u = draw((uint32_t)h, (uint32_t)k >> 9), v = draw((uint32_t)(h >> 32), (uint32_t)k >> 16);
+    b[0] += differ(div_rn(x, u), x / u) || differ(div_rn(u, x), u / x) || differ(div_rn(u, v), u / v);
+    const f3 q3 = ExactMath::div3(f3{u, v, x}, u * v);
+    b[0] += differ(q3.x, u / (u * v)) || differ(q3.y, v / (u * v)) || differ(q3.z, x / (u * v));
     b[1] += bits(div_pi_rn(x)) != bits(x / pi);
     b[2] += bits(div3_rn(x)) != bits(x / 3.0f);
     const float ys[2] = {1.0f, -1.7f};
@@ -654,6 +666,9 @@ __global__ void __launch_bounds__(kBlock) selftest_kernel(unsigned long long* __
     float w;
     if (ExactMath::corner_in_range<true>(1.0f, x, w, tab)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
     if (ExactMath::corner_in_range<false>(1.0f, x, w, nullptr)) b[3] += differ(w, fdlibm_atan2f_ref(1.0f, x) / pi);
+    const float n2 = __builtin_fabsf(u * v);
+    if (ExactMath::corner_in_range<true>(n2, u, w, tab)) b[3] += differ(w, fdlibm_atan2f_ref(__builtin_sqrtf(n2), u) / pi);
+    if (ExactMath::corner_in_range<true>(n2, x, w, tab)) b[3] += differ(w, fdlibm_atan2f_ref(__builtin_sqrtf(n2), x) / pi);
     if (x >= 0.0f && ExactMath::corner_in_range<false>(x, -0.37f, w, nullptr))
       b[3] += differ(w, fdlibm_atan2f_ref(__builtin_sqrtf(x), -0.37f) / pi);
     const float sr = __builtin_sqrtf(x);

@@ -63,8 +63,11 @@ struct ExactMath {
   }
   FP_HD static float atan2_(float y, float x) { return fdlibm_atan2f(y, x); }
   FP_HD static float div_pi(float x) { return div_pi_rn(x); }
-  // atan2(sqrt(n2), d) / PI where every quotient on the way is within div_by_rcp's range (returns
-  // true): the same roundings as div_pi(atan2_(sqrt_(n2), d)) in a quarter fewer operations.  With
+  // atan2(sqrt(n2), d) / PI where every quotient on the way is within div_by_rcp's reach (returns
+  // true): the same roundings as div_pi(atan2_(sqrt_(n2), d)) in a quarter fewer operations.  The root is
+  // within [2^-45, 2^45] and t within [2^-29, 2^25), so |d| is within 2^-71 and 2^75 and the first
+  // quotient's residual at least 2^-93; the second has a numerator t A - B that is +0 (its quotient then +0
+  // as well) or at least 2^-29 in magnitude and a denominator within [1, 2^26].  With
   // TAB, `tab` the kFdlEntries entries of fdl_entry, one wide LDS read stands for the selects that pick
   // the reduction interval (13 of a corner's 112 operations).
   template <bool TAB>

@@ -77,10 +77,10 @@ const char* fp_last_error(void);
 const char* fp_version(void);
 /* No counterpart in the reference.  Checks on the current GPU, over every finite f32 x, that the
  * exact kernels' shortened forms equal the operations they stand for: mismatches[0] the
- * reciprocal and the quotient with x as divisor and dividend, [1] x / PI, [2] x / 3, [3] the
- * branch-free atan2 and the corner weight made from it vs fdlibm's control flow, [4] the square
- * root and its reciprocal vs the compiler's correctly rounded sequences.  All five are 0 on a GPU
- * whose results the exact kernels reproduce. */
+ * reciprocal and the quotient with x as divisor and dividend (the other operand fixed or drawn),
+ * [1] x / PI, [2] x / 3, [3] the branch-free atan2 and the corner weight made from it vs fdlibm's
+ * control flow, [4] the square root and its reciprocal vs the compiler's correctly rounded
+ * sequences.  All five are 0 on a GPU whose results the exact kernels reproduce. */
 int fp_selftest_exact_math(uint64_t mismatches[5]);
 /* Config::default() (springy/config.rs:20-33): RK4, dt = Duration::from_millis(1), gravity
  * (0,-10,0), no wind, lift 1, drag 1, restitution 0.95, friction 0.3. */
