@@ -22,6 +22,7 @@
 #include <memory>
 #include <numeric>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "grid_fast.hpp"
@@ -189,10 +190,12 @@ bool refresh_mass(MeshSlot& ms, float m0, bool uniform) {
 int upload_params(fp_sim* s) {
   std::vector<fp::StepParams> p;
   for (auto& m : s->meshes) p.push_back(m.params);
-  if (s->params.p != nullptr && p.size() == s->h_params_last.size() &&
+  if (!s->stale && s->params.p != nullptr && p.size() == s->h_params_last.size() &&
       std::memcmp(p.data(), s->h_params_last.data(), p.size() * sizeof(fp::StepParams)) == 0)
     return FP_OK;  // the device copy already holds these values
+  const bool was = std::exchange(s->stale, true);
   HIP_TRY(s->params.assign(p.data(), p.size()));
+  s->stale = was;
   s->h_params_last = p;
   ++s->epoch;
   return FP_OK;
@@ -239,7 +242,8 @@ int build_block_lists(fp_sim* s) {
     sig.push_back(m.uniform_mass ? 1 : 0);
     sig.push_back(m.tile_chosen ? -1 - m.tile_shape : m.tile_shape);
   }
-  if (sig == s->lists_sig) return FP_OK;
+  if (!s->stale && sig == s->lists_sig) return FP_OK;
+  const bool was = std::exchange(s->stale, true);  // an upload that fails leaves one list empty and others old
   std::vector<fp::BlockRange> g, c, cf, sb, sf;
   std::vector<fp::PatchRange> pl;
   std::vector<fp::TileRange> by_shape[fp::N_LAUNCH_SHAPES], all_tiles;
@@ -307,8 +311,18 @@ int build_block_lists(fp_sim* s) {
     HIP_TRY(s->tiles[sh].upload(o.data(), o.size()));
   }
   HIP_TRY(s->mesh_tiles.upload(all_tiles.data(), all_tiles.size()));
+  s->stale = was;
   s->lists_sig = sig;
   ++s->epoch;
+  return FP_OK;
+}
+
+// What the launches read, built again after a call that could not upload all of it.
+int ensure_lists(fp_sim* s) {
+  if (!s->stale) return FP_OK;
+  if (int e = upload_params(s)) return e;
+  if (int e = build_block_lists(s)) return e;
+  s->stale = false;
   return FP_OK;
 }
 
@@ -352,6 +366,7 @@ hipError_t tiled_launch(fp_sim* s, const fp::StepArgs& a, const fp::TileRange* t
 }
 
 int run_steps(fp_sim* s, uint64_t n) {
+  if (int e = ensure_lists(s)) return e;
   for (uint64_t k = 0; k < n; ++k) {
     fp::StepArgs a = s->args(s->forces_dirty);
     bool exact = s->math == FP_MATH_EXACT;
@@ -372,6 +387,7 @@ int run_steps(fp_sim* s, uint64_t n) {
 // Enqueues n steps, replaying captured `chunk`-step graphs where possible.  A step that starts from
 // non-zero force records runs eagerly first (the captured launches assume clear forces).
 int run_steps_graph(fp_sim* s, uint64_t n, uint32_t chunk) {
+  if (int e = ensure_lists(s)) return e;  // not within a capture
   if (chunk == 0) return run_steps(s, n);
   if (s->forces_dirty && n > 0) {
     if (int e = run_steps(s, 1)) return e;
@@ -1204,7 +1220,7 @@ int fp_sim_set_points(fp_sim* s, uint64_t mesh, const float* rec, uint64_t n) {
                                     cur, s->mass.p, s->force[0].p, s->force[1].p, s->force[2].p, scan, s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   s->forces_dirty = s->forces_dirty || scan->force != 0;
-  if (!refresh_mass(m, rec[0], scan->mass == 0)) return FP_OK;
+  if (!refresh_mass(m, rec[0], scan->mass == 0)) return ensure_lists(s);
   if (int e = upload_params(s)) return e;
   return build_block_lists(s);
 }
@@ -1241,6 +1257,7 @@ int fp_host_free(void* ptr) {
 
 int fp_sim_accumulate_forces(fp_sim* s, uint64_t mesh) {
   if (int e = check_sim_mesh(s, mesh)) return e;
+  if (int e = ensure_lists(s)) return e;
   const MeshSlot& m = s->meshes[mesh];
   fp::StepArgs a = s->args(true);
   const fp::BlockRange* blk = s->all_blocks.p + m.blk_begin;

@@ -109,6 +109,7 @@ struct fp_sim {
   // would upload the same lists again does nothing (so a checkpoint restore keeps the graphs)
   std::vector<fp::StepParams> h_params_last;
   std::vector<int32_t> lists_sig;
+  bool stale = false;  // one of the two failed on the way: ensure_lists builds them again before a launch
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   uint64_t graph_epoch[2] = {0, 0};
   uint32_t graph_chunk[2] = {0, 0};
@@ -183,5 +184,6 @@ namespace fpsim {
 fp::StepParams make_params(const fp_config& c, float mass, bool uniform);
 int check_sim_mesh(const fp_sim* s, uint64_t mesh);
 int run_steps(fp_sim* s, uint64_t n);
+int ensure_lists(fp_sim* s);
 
 }  // namespace fpsim

@@ -111,6 +111,7 @@ fp::FeatParams feat_params(const fp_surrogate_config& c) {
 
 // One big step of every mesh, with the per-mesh fallback.
 int sur_big_step(fp_sim* s, fp_surrogate_stats& st, float* mlp_ms) {
+  if (int e = ensure_lists(s)) return e;
   auto& S = s->sur;
   const uint32_t nblk = (uint32_t)s->h_blocks.size();
   const size_t M = s->meshes.size();
