@@ -68,10 +68,11 @@ int build_slots(fp_sim* s) {
     mesh_slots.push_back(r);
   }
   HIP_TRY(S.mesh_slots.upload(mesh_slots.data(), mesh_slots.size()));
-  HIP_TRY(S.slots.upload(S.h_slots.data(), S.h_slots.size()));
   HIP_TRY(S.slot_k.upload(sk.data(), sk.size()));
   HIP_TRY(S.mesh_of.upload(mesh_of.data(), mesh_of.size()));
   HIP_TRY(S.ids.upload(ids.data(), ids.size()));
+  // last: where the slots are on the device, all of these are
+  HIP_TRY(S.slots.upload(S.h_slots.data(), S.h_slots.size()));
   return FP_OK;
 }
 

@@ -1,7 +1,8 @@
 """A device allocation that fails while a simulation's launch lists are rebuilt (records whose masses send a
-cloth from the tiled kernel to the general one).  The call reports it; afterwards nothing is launched over
-half-built lists: the same records set again, other records, or a step build them anew.  The failure is
-injected on the host (tests/native/failing_malloc.cpp), in a process of its own; no memory is exhausted."""
+cloth from the tiled kernel to the general one), or while the surrogate's slots are laid out.  The call reports
+it; afterwards nothing is launched over half-built lists: the same records set again, other records, or a step
+build them anew, and so does the surrogate set again.  The failure is injected on the host
+(tests/native/failing_malloc.cpp), in a process of its own; no memory is exhausted."""
 import os
 import subprocess
 import sys
@@ -27,6 +28,8 @@ sc = wl.config0(steps=1, seed=1, rows=20, cols=20)
 ref = wl.build_gpu(sc)
 assert shim.failing_malloc_calls() > 0  # the library's allocations pass through
 rec = ref.get_points(0)
+"""
+LISTS = r"""
 heavy = rec.copy()
 heavy[::3, 0] *= 2.0
 
@@ -73,10 +76,42 @@ print("ok", flush=True)
 """
 
 
-def test_lists_are_built_again_after_a_failed_allocation(tmp_path):
+SLOTS = r"""
+net = fa.Surrogate(fa.SurrogateConfig(strain_limit=1e30, energy_limit=1e30), seed=3)
+before = shim.failing_malloc_calls()
+ref.set_surrogate(net)
+made = shim.failing_malloc_calls() - before
+print("allocations of the surrogate:", made, flush=True)
+assert made >= 5
+ref.step_surrogate(2)
+want = ref.get_points(0)
+for nth in range(made):
+    sim = wl.build_gpu(sc)
+    shim.failing_malloc_in(nth)
+    try:
+        sim.set_surrogate(net)
+        raise SystemExit("no failure")
+    except fa.FpError as e:
+        assert "out of memory" in str(e), e
+    shim.failing_malloc_in(-1)
+    print("allocation", nth, "failed", flush=True)
+    try:  # not set: refused, not launched
+        sim.step_surrogate(1)
+        raise SystemExit("stepped without a network")
+    except fa.FpError:
+        pass
+    sim.set_surrogate(net)
+    sim.step_surrogate(2)
+    assert (bits(sim.get_points(0)) == bits(want)).all(), nth
+print("ok", flush=True)
+"""
+
+
+@pytest.mark.parametrize("body", [LISTS, SLOTS], ids=["lists", "slots"])
+def test_lists_are_built_again_after_a_failed_allocation(tmp_path, body):
     shim = str(tmp_path / "failing_malloc.so")
     subprocess.run(["g++", "-O1", "-shared", "-fPIC", os.path.join(ROOT, "tests", "native", "failing_malloc.cpp"), "-o",
                     shim], check=True)
-    p = subprocess.run([sys.executable, "-u", "-c", CHILD, shim, ROOT], capture_output=True, text=True, timeout=100)
+    p = subprocess.run([sys.executable, "-u", "-c", CHILD + body, shim, ROOT], capture_output=True, text=True, timeout=100)
     print(p.stdout[-3000:], p.stderr[-3000:], flush=True)
     assert p.returncode == 0 and p.stdout.rstrip().endswith("ok")
