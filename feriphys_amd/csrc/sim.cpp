@@ -338,16 +338,24 @@ int check_sim_mesh(const fp_sim* s, uint64_t mesh) {
   return FP_OK;
 }
 
+// Room in fp_sim::direct: one allocation for a simulation's life, always of the same size (each takes 20 to
+// 40 us, as long as a small mesh's records both ways; one of a size that the process has not had before, up to
+// a millisecond).
+constexpr size_t kDirectHead = 64;
+static_assert(sizeof(fp::RecordScan) <= kDirectHead, "the scan's place");
+hipError_t reserve_direct(fp_sim* s) { return s->direct.reserve(kDirectHead + fph::kDirectBytes); }
+float* direct_records(fp_sim* s) { return s->direct.floats() + kDirectHead / sizeof(float); }
+
 // `count` floats that `pack` writes on the device, into the caller's `dst`: straight into page-locked
 // memory and from there when they are few, otherwise through device memory and one copy.
 template <class Pack>
 int read_back(fp_sim* s, float* dst, uint64_t count, Pack pack) {
   const size_t bytes = count * sizeof(float);
   if (bytes <= fph::kDirectBytes) {
-    HIP_TRY(s->host_rec.reserve(fph::kDirectBytes));
-    HIP_TRY(pack(s->host_rec.floats()));
+    HIP_TRY(reserve_direct(s));
+    HIP_TRY(pack(direct_records(s)));
     HIP_TRY(hipStreamSynchronize(s->stream));
-    std::memcpy(dst, s->host_rec.p, bytes);
+    std::memcpy(dst, direct_records(s), bytes);
     return FP_OK;
   }
   HIP_TRY(s->rec_stage.reserve(count));
@@ -1202,13 +1210,12 @@ int fp_sim_set_points(fp_sim* s, uint64_t mesh, const float* rec, uint64_t n) {
   // scattered into the device order, and scanned for forces and unequal masses, by the device
   const size_t bytes = 10 * n * sizeof(float);
   const float* src;
-  HIP_TRY(s->scan.reserve(sizeof(fp::RecordScan)));
-  auto* scan = static_cast<fp::RecordScan*>(s->scan.p);
+  HIP_TRY(reserve_direct(s));
+  auto* scan = static_cast<fp::RecordScan*>(s->direct.p);
   *scan = fp::RecordScan{0, 0};
   if (bytes <= fph::kDirectBytes) {
-    HIP_TRY(s->host_rec.reserve(fph::kDirectBytes));
-    std::memcpy(s->host_rec.p, rec, bytes);
-    src = s->host_rec.floats();
+    std::memcpy(direct_records(s), rec, bytes);
+    src = direct_records(s);
   } else {
     HIP_TRY(s->rec_stage.reserve(10 * n));
     HIP_TRY(hipMemcpyAsync(s->rec_stage.p, rec, bytes, hipMemcpyHostToDevice, s->stream));

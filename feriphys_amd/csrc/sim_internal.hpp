@@ -65,8 +65,9 @@ struct fp_sim {
   // per general mesh, for every reference vertex its device-local slot (MeshSlot::pos), at vbase
   fph::DBuf<uint32_t> d_pos;
   fph::DBuf<float> rec_stage;  // 10-float records packed on the device for one readback
-  fph::HostBuf host_rec;       // small meshes' records, packed and unpacked by the kernels directly
-  fph::HostBuf scan;           // fp::RecordScan of the last records set
+  // the fp::RecordScan of the last records set and, from kDirectHead on, small meshes' records, packed and
+  // unpacked by the kernels directly
+  fph::HostBuf direct;
   fph::DBuf<uint32_t> pins;
   fph::DBuf<uint32_t> s_first, s_cnt, f_first, f_cnt, f_v, f_slot;
   fph::DBuf<fp::StrutEnt> s_ent;

@@ -20,6 +20,8 @@ sys.path.insert(0, sys.argv[2])
 hip = C.CDLL("libamdhip64.so.7")
 shim.failing_malloc_real.argtypes = [C.c_void_p]
 shim.failing_malloc_real(C.cast(hip.hipMalloc, C.c_void_p))
+shim.failing_host_malloc_real.argtypes = [C.c_void_p]
+shim.failing_host_malloc_real(C.cast(hip.hipHostMalloc, C.c_void_p))
 import feriphys_amd as fa
 from feriphys_amd import workloads as wl
 
@@ -107,7 +109,30 @@ print("ok", flush=True)
 """
 
 
-@pytest.mark.parametrize("body", [LISTS, SLOTS], ids=["lists", "slots"])
+# records in and out: one page-locked allocation for a simulation's life, reported when it fails
+RECORDS = r"""
+for size in (20, 120):
+    sim = wl.build_gpu(wl.config0(steps=1, seed=1, rows=size, cols=size))
+    before = shim.failing_host_malloc_calls()
+    shim.failing_host_malloc_in(0)
+    try:
+        sim.set_points(0, np.ones((size * size, 10), np.float32))
+        raise SystemExit("no failure")
+    except fa.FpError as e:
+        assert "out of memory" in str(e), e
+    made = []
+    r = rec if size == 20 else sim.get_points(0)
+    for _ in range(2):
+        sim.set_points(0, r)
+        assert (bits(sim.get_points(0)) == bits(r)).all()
+        made.append(shim.failing_host_malloc_calls() - before)
+    print("page-locked allocations, the failed one among them:", made, flush=True)
+    assert made == [2, 2]
+print("ok", flush=True)
+"""
+
+
+@pytest.mark.parametrize("body", [LISTS, SLOTS, RECORDS], ids=["lists", "slots", "records"])
 def test_lists_are_built_again_after_a_failed_allocation(tmp_path, body):
     shim = str(tmp_path / "failing_malloc.so")
     subprocess.run(["g++", "-O1", "-shared", "-fPIC", os.path.join(ROOT, "tests", "native", "failing_malloc.cpp"), "-o",
