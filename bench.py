@@ -42,10 +42,12 @@ COMMON = ["step_device.hpp", "vec.hpp", "exact_ops.hpp", "fdlibm_atan2f.hpp", "k
 # the source files each measured kernel is built from; a counter reading below is reported only
 # while these files still hash to the value it was measured on
 KERNEL_SOURCES = {
-    # sim.cpp deals the tiles to the XCDs, which sets how often halo rows are fetched twice;
-    # obstacles.cpp builds the broad-phase grids the collision search walks
-    "grid_tiled_kernel<ExactMath,16,16>": ["grid_tiled.hip", "grid_tile_core.hpp", "obstacles.cpp", "sim.cpp"] + COMMON,
-    "grid_fast_kernel<15,15>": ["grid_fast.hip", "grid_fast_core.hpp", "grid_fast.hpp", "obstacles.cpp", "sim.cpp"] + COMMON,
+    # sim.cpp deals the tiles to the XCDs, which sets how often halo rows are fetched twice, and
+    # tile_rule.hpp chooses their shape; obstacles.cpp builds the broad-phase grids the collision search walks
+    "grid_tiled_kernel<ExactMath,16,16>": ["grid_tiled.hip", "grid_tile_core.hpp", "tile_rule.hpp", "obstacles.cpp",
+                                           "sim.cpp"] + COMMON,
+    "grid_fast_kernel<15,15>": ["grid_fast.hip", "grid_fast_core.hpp", "grid_fast.hpp", "tile_rule.hpp", "obstacles.cpp",
+                                "sim.cpp"] + COMMON,
     "patch_kernel<ExactMath>": ["kernels.hip"] + COMMON,
 }
 # rocprofv3 readings per dispatch on the 1024 x 1024 cloth (first steps) and the 64 icospheres:
@@ -54,15 +56,15 @@ KERNEL_SOURCES = {
 # GRBM_GUI_ACTIVE summed over the 8 XCDs (the commands are in the profiles named)
 MEASURED = {
     ("grid_tiled_kernel<ExactMath,16,16>", "cloth1024"): {
-        "src_sha": "44c6e11c38609e71", "fetch_kib": 16043, "write_kib": 24577,
-        "valu_insts": 2.6651e7, "waves": 16384, "grbm_gui_active": 8.8612e5,
+        "src_sha": "819e8a97c9777cc5", "fetch_kib": 16056, "write_kib": 24577,
+        "valu_insts": 2.6651e7, "waves": 16384, "grbm_gui_active": 8.8886e5,
         "profiles": ["profiles/grid_tiled_exact_cloth1024.md", "profiles/grid_tiled_cloth1024_pmc.md"]},
     ("grid_fast_kernel<15,15>", "cloth1024"): {
-        "src_sha": "6cd356afb506531a", "fetch_kib": 16218, "write_kib": 24734,
-        "valu_insts": 1.1358e7, "waves": 19044, "grbm_gui_active": 5.2546e5,
+        "src_sha": "61935174bf7a799a", "fetch_kib": 16218, "write_kib": 24734,
+        "valu_insts": 1.1358e7, "waves": 19044, "grbm_gui_active": 5.3113e5,
         "profiles": ["profiles/grid_fast_cloth1024.md"]},
     ("patch_kernel<ExactMath>", "icospheres64"): {
-        "src_sha": "2906e54087b1bb00", "fetch_kib": 165096, "write_kib": 50329,
+        "src_sha": "bfd7735186ffa7f8", "fetch_kib": 165066, "write_kib": 50329,
         "profiles": ["profiles/batched_and_surfaces.md"]},
 }
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0
@@ -692,7 +694,7 @@ def rigid_scene(np, n, seed=0):
 
 
 RIGID_BODIES = 1 << 20
-RIGID_BYTES_PER_BODY = 2 * 29 * 4  # the 29-float record read and written once per launch
+RIGID_BYTES_PER_BODY = (29 + 13) * 4  # per launch: the 29-float record read, the 13 fields that change stored
 RIGID_STEPS_PER_LAUNCH = 64        # kRigidChunk of rigid.cpp: the record stays in registers between them
 
 
@@ -762,8 +764,9 @@ def bench_rigid(args, np, fa, wl):
         "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": rates["workload"], "bodies": n},
         "body_steps_per_s": rates["body_steps_per_s"],
-        "roofline": {"bound": "valu", "achieved": rates["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": rates["hbm_frac"], "traffic": None, "kernel_avg_us": rates["kernel_avg_us"],
+        # against HBM; what limits the kernel is vector issue (profiles/rigid_cubes1m.md)
+        "roofline": {"bound": "hbm", "achieved": rates["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": rates["hbm_frac"], "traffic": None, "limited_by": "valu", "kernel_avg_us": rates["kernel_avg_us"],
                      "bytes_per_launch": rates["bytes_per_launch"]},
         "cpu_baseline": cpu,
     }

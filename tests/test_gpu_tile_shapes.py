@@ -93,3 +93,29 @@ def test_autotune_reports_shapes_that_can_be_set(math):
     announce(f"autotune, math {math}: {chosen}")
     for k, shape in enumerate(chosen):
         assert shape in SHAPES and sim.get_tile_shape(k) == shape
+
+
+def test_fast_shapes_side_by_side_equal_each_alone():
+    """Fast steps of cloths with set shapes, a launch per shape, and of default ones beside them (more tiles
+    than are resident, so that they keep their own): each cloth's records are the bits of the cloth alone
+    with the shape it runs in."""
+    sizes = [(33, 34), (29, 65), (48, 17), (12, 200), (620, 640)]
+    shapes = [fa.FP_TILE_15x15, fa.FP_TILE_7x31, fa.FP_TILE_16x16, None, None]
+    alone = [fa.FP_TILE_15x15, fa.FP_TILE_7x31, fa.FP_TILE_15x15, fa.FP_TILE_7x31, fa.FP_TILE_15x15]
+    sim = wl.build_gpu(scene(sizes, obstacle=True))
+    sim.set_kernel(fa.FP_KERNEL_GRID, fa.FP_MATH_FAST)
+    for k, shape in enumerate(shapes):
+        if shape is not None:
+            sim.set_tile_shape(k, shape)
+    start = [sim.get_points(k) for k in range(len(sizes))]
+    announce("fast, three launches a step")
+    sim.step(7)
+    sim.step_graph(10, 5)
+    for k, size in enumerate(sizes):
+        one = wl.build_gpu(scene([size], obstacle=True))
+        one.set_kernel(fa.FP_KERNEL_GRID, fa.FP_MATH_FAST)
+        one.set_tile_shape(0, alone[k])
+        one.set_points(0, start[k])
+        one.step(17)
+        a, b = sim.get_points(k), one.get_points(0)
+        assert np.isfinite(b).all() and (bits(a) == bits(b)).all(), size
