@@ -18,12 +18,11 @@ __device__ __forceinline__ void store_state(const SoA& o, uint32_t i, f3 x, f3 v
 
 // The 6 features of one slot: strain_scale * strain * d/|d| and (v_nbr - v) * H / L, from the
 // neighbour's position q and velocity w; zeros when `has` is false.  Branch-free, so that a caller
-// can issue every load of a pass before the first feature is computed.  The short root (exact but for
-// d2 < 2^-96, where it may be an ulp off) has no value for a subnormal d2, |d| < 1.1e-19: returns whether
-// that is so, and the features must then be formed again with GENERAL.
+// can issue every load of a pass before the first feature is computed.  The short root is exact but for
+// d2 < 2^-96, where it may be an ulp off, and for a subnormal d2, |d| < 1.1e-19, where it gives NaN: a caller
+// without GENERAL looks for that in its results.
 template <bool GENERAL>
-__device__ __forceinline__ bool slot_feat_from(f3 p, f3 v, f3 q, f3 w, float rest, bool has, FeatParams fp, float* f) {
-  constexpr int kPositiveSubnormal = 0x080;
+__device__ __forceinline__ void slot_feat_from(f3 p, f3 v, f3 q, f3 w, float rest, bool has, FeatParams fp, float* f) {
   const f3 d = sub(q, p);
   const float d2 = d.x * d.x + d.y * d.y + d.z * d.z;
   const float len = GENERAL ? sqrt_rn(d2) : sqrt_in_range(d2);
@@ -32,16 +31,14 @@ __device__ __forceinline__ bool slot_feat_from(f3 p, f3 v, f3 q, f3 w, float res
   const float hv = has ? fp.H * il : 0.0f;
   f[0] = st * d.x; f[1] = st * d.y; f[2] = st * d.z;
   f[3] = (w.x - v.x) * hv; f[4] = (w.y - v.y) * hv; f[5] = (w.z - v.z) * hv;
-  return !GENERAL && __builtin_amdgcn_classf(d2, kPositiveSubnormal);
 }
 
 template <bool GENERAL = true>
-__device__ __forceinline__ bool slot_feat(const SoA& S, f3 p, f3 v, uint32_t self, SlotEnt e, FeatParams fp,
+__device__ __forceinline__ void slot_feat(const SoA& S, f3 p, f3 v, uint32_t self, SlotEnt e, FeatParams fp,
                                           float* f) {
   const bool has = e.nbr != kNoSlot;
   const uint32_t nb = has ? e.nbr : self;
-  return slot_feat_from<GENERAL>(p, v, ld3(S.x, S.y, S.z, nb), ld3(S.vx, S.vy, S.vz, nb), has ? e.rest : 1.0f, has, fp,
-                                 f);
+  slot_feat_from<GENERAL>(p, v, ld3(S.x, S.y, S.z, nb), ld3(S.vx, S.vy, S.vz, nb), has ? e.rest : 1.0f, has, fp, f);
 }
 
 __device__ __forceinline__ float unit_open(uint64_t h) { return ((float)(h >> 40) + 0.5f) * (1.0f / 16777216.0f); }
@@ -113,21 +110,19 @@ __global__ void __launch_bounds__(2048 / NT) sur_mlp_kernel(SoA S, const SlotEnt
   for (uint32_t r0 = u0; r0 < u1; r0 += kThreads / 64) {
     if (r0 + wave >= u1) continue;
     const uint32_t v0 = (r0 + wave) * 16 * NT;
-    // features: lane group g computes slots 3g..3g+2 of its vertex (18 values, then 6 zeros), which
-    // are its 8-element K slices of the three 32-wide K blocks of layer 1.  Every load is
-    // unconditional (past-the-end columns read vertex n-1, empty slots the vertex itself; both are
-    // zeroed), so a pass's loads can all be in flight together.  A wavefront that meets a strut with a
-    // subnormal squared length forms all its features once more with the general root.
-    bf16x8 B1[3][NT];
-    const auto features = [&](auto general) {
+    // One unit; false where its outputs are not all numbers and were not stored.
+    const auto unit = [&](auto general) {
+      constexpr bool kGeneral = decltype(general)::value;
+      // features: lane group g computes slots 3g..3g+2 of its vertex (18 values, then 6 zeros), which
+      // are its 8-element K slices of the three 32-wide K blocks of layer 1.  Every load is
+      // unconditional (past-the-end columns read vertex n-1, empty slots the vertex itself; both are
+      // zeroed), so a pass's loads can all be in flight together.
+      bf16x8 B1[3][NT];
       SlotEnt se[NT][3];
       f3 p[NT], v[NT];
-      uint32_t first = v0 + col;
-      // (the rare second pass loads again what the first one had)
-      if constexpr (decltype(general)::value) asm volatile("" : "+v"(first));
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        const uint32_t iv = first + nt * 16;
+        const uint32_t iv = v0 + nt * 16 + col;
         const uint32_t i = iv < n ? iv : n - 1;
         const SlotEnt* at = slots + slot_at(i, 3 * g);
         p[nt] = ld3(S.x, S.y, S.z, i);
@@ -138,15 +133,14 @@ __global__ void __launch_bounds__(2048 / NT) sur_mlp_kernel(SoA S, const SlotEnt
           se[nt][j].nbr = iv < n ? se[nt][j].nbr : kNoSlot;
         }
       }
-      bool again = false;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        const uint32_t iv = first + nt * 16;
+        const uint32_t iv = v0 + nt * 16 + col;
         const uint32_t i = iv < n ? iv : n - 1;
         float f[24];
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-          again = slot_feat<decltype(general)::value>(S, p[nt], v[nt], i, se[nt][j], fp, f + 6 * j) || again;
+          slot_feat<kGeneral>(S, p[nt], v[nt], i, se[nt][j], fp, f + 6 * j);
           __builtin_amdgcn_sched_barrier(0x20);  // loads may pass, arithmetic not: slots interleaved spill
         }
 #pragma unroll
@@ -156,34 +150,43 @@ __global__ void __launch_bounds__(2048 / NT) sur_mlp_kernel(SoA S, const SlotEnt
 #pragma unroll
           for (int s = 0; s < 8; ++s) B1[kb][nt][s] = (__bf16)f[kb * 8 + s];
       }
-      return again;
-    };
-    if (__any(features(std::false_type{}))) features(std::true_type{});
-    bf16x8 Bh[4][NT], Bg[4][NT];
-    mfma_act_layer<3, kLd1, NT>(W1, Bias, B1, Bh, col, g);
-    mfma_act_layer<4, kLd, NT>(W2, Bias + kHid, Bh, Bg, col, g);
-    mfma_act_layer<4, kLd, NT>(W3, Bias + 2 * kHid, Bg, Bh, col, g);
-    f32x4 o[NT];
+      bf16x8 Bh[4][NT], Bg[4][NT];
+      mfma_act_layer<3, kLd1, NT>(W1, Bias, B1, Bh, col, g);
+      mfma_act_layer<4, kLd, NT>(W2, Bias + kHid, Bh, Bg, col, g);
+      mfma_act_layer<4, kLd, NT>(W3, Bias + 2 * kHid, Bg, Bh, col, g);
+      f32x4 o[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) o[nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int nt = 0; nt < NT; ++nt) o[nt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(W4 + col * kLd + kb * 32 + g * 8);
+      for (int kb = 0; kb < 4; ++kb) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(W4 + col * kLd + kb * 32 + g * 8);
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) o[nt] = mfma(a, Bh[kb][nt], o[nt]);
-    }
-    if (g == 0) {
-      const float b0 = Bias[3 * kHid], b1 = Bias[3 * kHid + 1], b2 = Bias[3 * kHid + 2];
+        for (int nt = 0; nt < NT; ++nt) o[nt] = mfma(a, Bh[kb][nt], o[nt]);
+      }
+      if constexpr (!kGeneral) {
+        bool number = true;
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const uint32_t i = v0 + nt * 16 + col;
-        if (i < n) {
-          da[3 * (size_t)i] = out_scale * (o[nt][0] + b0);
-          da[3 * (size_t)i + 1] = out_scale * (o[nt][1] + b1);
-          da[3 * (size_t)i + 2] = out_scale * (o[nt][2] + b2);
+        for (int nt = 0; nt < NT; ++nt) number = number && o[nt][0] == o[nt][0];
+        if (!__all(number)) return false;
+      }
+      if (g == 0) {
+        const float b0 = Bias[3 * kHid], b1 = Bias[3 * kHid + 1], b2 = Bias[3 * kHid + 2];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          const uint32_t i = v0 + nt * 16 + col;
+          if (i < n) {
+            da[3 * (size_t)i] = out_scale * (o[nt][0] + b0);
+            da[3 * (size_t)i + 1] = out_scale * (o[nt][1] + b1);
+            da[3 * (size_t)i + 2] = out_scale * (o[nt][2] + b2);
+          }
         }
       }
-    }
+      return true;
+    };
+    // A strut with a subnormal squared length has NaN for features with the short root, and one NaN
+    // feature makes every output of its vertex NaN: only such units (and those whose states are not
+    // numbers) are evaluated again, with the general root, and the others pay a compare a tile.
+    if (!unit(std::false_type{})) unit(std::true_type{});
   }
 }
 
