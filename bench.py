@@ -56,15 +56,15 @@ KERNEL_SOURCES = {
 # GRBM_GUI_ACTIVE summed over the 8 XCDs (the commands are in the profiles named)
 MEASURED = {
     ("grid_tiled_kernel<ExactMath,16,16>", "cloth1024"): {
-        "src_sha": "819e8a97c9777cc5", "fetch_kib": 16056, "write_kib": 24577,
-        "valu_insts": 2.6651e7, "waves": 16384, "grbm_gui_active": 8.8886e5,
+        "src_sha": "abf8c787b479a322", "fetch_kib": 16052, "write_kib": 24576,
+        "valu_insts": 2.6651e7, "waves": 16384, "grbm_gui_active": 8.8616e5,
         "profiles": ["profiles/grid_tiled_exact_cloth1024.md", "profiles/grid_tiled_cloth1024_pmc.md"]},
     ("grid_fast_kernel<15,15>", "cloth1024"): {
-        "src_sha": "61935174bf7a799a", "fetch_kib": 16218, "write_kib": 24734,
-        "valu_insts": 1.1358e7, "waves": 19044, "grbm_gui_active": 5.3113e5,
+        "src_sha": "397a2874a3099c2c", "fetch_kib": 16218, "write_kib": 24734,
+        "valu_insts": 1.1358e7, "waves": 19044, "grbm_gui_active": 5.2830e5,
         "profiles": ["profiles/grid_fast_cloth1024.md"]},
     ("patch_kernel<ExactMath>", "icospheres64"): {
-        "src_sha": "bfd7735186ffa7f8", "fetch_kib": 165066, "write_kib": 50329,
+        "src_sha": "bfd7735186ffa7f8", "fetch_kib": 165056, "write_kib": 50349,
         "profiles": ["profiles/batched_and_surfaces.md"]},
 }
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0

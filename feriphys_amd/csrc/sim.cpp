@@ -470,6 +470,7 @@ int build_incidence(fp_sim* s) {
   std::vector<uint16_t> scls(n_sent + 1, 0);
   std::vector<float2> cls_tab(s->meshes.size() * fp::kPatchClasses, float2{0.0f, 0.0f});
   std::vector<uint8_t> cls_ok(s->meshes.size(), 1);
+  std::vector<uint8_t> odd_len(N, 0);  // a strut whose length or its inverse is not a normal number
   for (size_t mi = 0; mi < s->meshes.size(); ++mi) {
     auto& ms_ = s->meshes[mi];
     const auto& h = ms_.host;
@@ -479,6 +480,7 @@ int build_incidence(fp_sim* s) {
       const uint32_t ea = sfirst[a] + fp::kSlice * sfill[a]++, eb = sfirst[b] + fp::kSlice * sfill[b]++;
       sent[ea] = fp::StrutEnt{b, h.s_len[k], h.s_k[k], h.s_c[k]};
       sent[eb] = fp::StrutEnt{a, h.s_len[k], h.s_k[k], h.s_c[k]};
+      if (!(std::fabs(h.s_len[k]) >= 0x1p-126f && std::fabs(h.s_len[k]) <= 0x1p126f)) odd_len[a] = odd_len[b] = 1;
       if (!cls_ok[mi]) continue;
       const float kn = h.s_kn[k], cn = h.s_cn[k], inv = 1.0f / h.s_len[k];
       if (!same_bits(inv * kn, h.s_k[k]) || !same_bits(inv * cn, h.s_c[k])) { cls_ok[mi] = 0; continue; }
@@ -591,11 +593,7 @@ int build_incidence(fp_sim* s) {
           pr.s_max[w] = *std::max_element(scnt.begin() + v0, scnt.begin() + v1);
           pr.f_min[w] = *std::min_element(fcnt.begin() + v0, fcnt.begin() + v1);
           pr.f_max[w] = *std::max_element(fcnt.begin() + v0, fcnt.begin() + v1);
-          for (uint32_t i = v0; i < v1; ++i)
-            for (uint32_t j = 0; j < scnt[i]; ++j) {
-              const float len = std::fabs(sent[sfirst[i] + fp::kSlice * j].len);
-              if (!(len >= 0x1p-126f && len <= 0x1p126f)) pr.s_min[w] = 0;
-            }
+          if (std::find(odd_len.begin() + v0, odd_len.begin() + v1, 1) != odd_len.begin() + v1) pr.s_min[w] = 0;
         }
       }
       s->h_patches.push_back(pr);
@@ -606,11 +604,20 @@ int build_incidence(fp_sim* s) {
   HIP_TRY(s->p_corner.upload(pcorner.data(), pcorner.size()));
   {
     std::vector<fp::PatchStrut> pent(n_sent + fp::kSlice, fp::PatchStrut{1.0f, 0, 0});
-    for (uint64_t i = 0; i < N; ++i)
-      for (uint32_t j = 0; j < scnt[i]; ++j) {
-        const uint32_t e = sfirst[i] + fp::kSlice * j;
-        pent[e] = fp::PatchStrut{sent[e].len, sloc[e], (uint16_t)(scls[e] | 0x8000u)};
-      }
+    for (const auto& ms_ : s->meshes) {  // in the entries' own order: slice by slice, a slice's j-th entries together
+      if (!ms_.patch_ok) continue;       // a cloth's, or those of a mesh on the CSR kernel, are never read
+      for (size_t b = 0; b + 1 < ms_.bstart.size(); ++b)
+        for (uint64_t v0 = ms_.vbase + ms_.bstart[b], v1 = ms_.vbase + ms_.bstart[b + 1]; v0 < v1; v0 += fp::kSlice) {
+          const uint64_t end = std::min<uint64_t>(v1, v0 + fp::kSlice);
+          const uint32_t most = *std::max_element(scnt.begin() + v0, scnt.begin() + end);
+          for (uint32_t j = 0; j < most; ++j)
+            for (uint64_t i = v0; i < end; ++i) {
+              if (j >= scnt[i]) continue;
+              const uint32_t e = sfirst[i] + fp::kSlice * j;
+              pent[e] = fp::PatchStrut{sent[e].len, sloc[e], (uint16_t)(scls[e] | 0x8000u)};
+            }
+        }
+    }
     HIP_TRY(s->p_ent.upload(pent.data(), pent.size()));
     HIP_TRY(s->p_cls.upload(cls_tab.data(), cls_tab.size()));
   }

@@ -28,7 +28,11 @@ int build_slots(fp_sim* s) {
   std::vector<float> sk(fp::slot_count(N), 0.0f);
   std::vector<uint32_t> mesh_of(N), ids;
   std::vector<uint8_t> used(N, 0);
-  static const int offs[10][2] = {{0, 1}, {0, -1}, {1, 0}, {-1, 0}, {-1, 1}, {1, -1}, {0, 2}, {0, -2}, {2, 0}, {-2, 0}};
+  // slot of the grid offset (dr, dc) at [dr + 2][dc + 2]: (0,+1) (0,-1) (+1,0) (-1,0) (-1,+1) (+1,-1) and the
+  // same two away along the axes
+  static const int8_t slot_of[5][5] = {
+      {-1, -1, 9, -1, -1}, {-1, -1, 3, 4, -1}, {7, 1, -1, 0, 6}, {-1, 5, 2, -1, -1}, {-1, -1, 8, -1, -1}};
+  std::vector<fp::MeshSlots> mesh_slots;
   for (uint32_t mi = 0; mi < s->meshes.size(); ++mi) {
     const MeshSlot& ms = s->meshes[mi];
     const fp::HostMesh& h = ms.host;
@@ -39,33 +43,31 @@ int build_slots(fp_sim* s) {
       if (!pin[ms.ref(i)]) ids.push_back((uint32_t)(ms.vbase + i));
     }
     const bool grid = h.cloth.valid;
-    const int64_t C = h.cloth.cols;
+    const uint32_t C = h.cloth.cols;
+    uint32_t seen = 0;  // slots in use, a bit each
+    const auto put = [&](uint64_t gi, int slot, uint32_t other, uint64_t k) {
+      const size_t at = fp::slot_at((uint32_t)gi, slot);
+      S.h_slots[at] = fp::SlotEnt{(uint32_t)ms.dev(other), h.s_len[k]};
+      sk[at] = h.s_k[k];
+      seen |= 1u << slot;
+    };
     for (uint64_t k = 0; k < h.n_struts(); ++k) {
       if (!(h.s_len[k] > 0.0f)) continue;
-      for (int side = 0; side < 2; ++side) {
-        const uint32_t self = side ? h.s_v1[k] : h.s_v0[k], other = side ? h.s_v0[k] : h.s_v1[k];
-        const uint64_t gi = ms.dev(self);
-        int slot = -1;
-        if (grid) {
-          const int64_t dr = (int64_t)(other / C) - (int64_t)(self / C), dc = (int64_t)(other % C) - (int64_t)(self % C);
-          for (int j = 0; j < 10; ++j)
-            if (offs[j][0] == dr && offs[j][1] == dc) slot = j;
-        } else if (used[gi] < fp::kSlots) {
-          slot = used[gi]++;
+      const uint32_t a = h.s_v0[k], b = h.s_v1[k];
+      if (grid) {
+        const int64_t dr = (int64_t)(b / C) - (int64_t)(a / C), dc = (int64_t)(b % C) - (int64_t)(a % C);
+        if (dr < -2 || dr > 2 || dc < -2 || dc > 2) continue;
+        const int s0 = slot_of[2 + dr][2 + dc], s1 = slot_of[2 - dr][2 - dc];
+        if (s0 >= 0) put(ms.dev(a), s0, b, k);
+        if (s1 >= 0) put(ms.dev(b), s1, a, k);
+      } else {
+        for (int side = 0; side < 2; ++side) {
+          const uint64_t gi = ms.dev(side ? b : a);
+          if (used[gi] < fp::kSlots) put(gi, used[gi]++, side ? a : b, k);
         }
-        if (slot < 0) continue;
-        S.h_slots[fp::slot_at((uint32_t)gi, slot)] = fp::SlotEnt{(uint32_t)ms.dev(other), h.s_len[k]};
-        sk[fp::slot_at((uint32_t)gi, slot)] = h.s_k[k];
       }
     }
-  }
-  std::vector<fp::MeshSlots> mesh_slots;
-  for (const auto& ms : s->meshes) {
-    fp::MeshSlots r{ms.blk_begin, ms.blk_end, 0u, 0u};
-    for (uint64_t i = ms.vbase; i < ms.vbase + ms.host.n; ++i)
-      for (uint32_t j = r.n_slots; j < (uint32_t)fp::kSlots; ++j)
-        if (S.h_slots[fp::slot_at((uint32_t)i, (int)j)].nbr != fp::kNoSlot) r.n_slots = j + 1;
-    mesh_slots.push_back(r);
+    mesh_slots.push_back(fp::MeshSlots{ms.blk_begin, ms.blk_end, seen ? 32u - (uint32_t)__builtin_clz(seen) : 0u, 0u});
   }
   HIP_TRY(S.mesh_slots.upload(mesh_slots.data(), mesh_slots.size()));
   HIP_TRY(S.slot_k.upload(sk.data(), sk.size()));
