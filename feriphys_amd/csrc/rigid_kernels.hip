@@ -118,6 +118,17 @@ __device__ __forceinline__ f3 corner_of_lane(const Corners& C, f3 x, uint32_t k)
   return f3{one(C.s.x, C.d.x, C.a.x, x.x), one(C.s.y, C.d.y, C.a.y, x.y), one(C.s.z, C.d.z, C.a.z, x.z)};
 }
 
+// The same as the reference writes it, (r0 c0 + r1 c1) + r2 c2 per row and then + x: for a pose that is not a
+// number, where the sign of a NaN decides on which side of a plane the corner is, and the flips above would
+// turn it.  Opaque, so that nothing of it is shared with the usual form (171 registers, two waves a SIMD).
+__device__ __forceinline__ f3 corner_as_written(Q q, f3 x, uint32_t k) {
+  f3 c = f3{0x66u >> k & 1u ? 0.5f : -0.5f, 0xccu >> k & 1u ? 0.5f : -0.5f, k < 4u ? 0.5f : -0.5f};
+  settle(q);
+  settle(c);
+  const M3 R = from_quat(q);
+  return add(mv(R, c), x);
+}
+
 // Obstacle face f (the same for the whole wave): never written while a kernel runs, so read through the
 // constant address space, which puts it in scalar registers.
 __device__ __forceinline__ ObsFace uniform_face(const ObsView& O, uint32_t f) {
@@ -302,10 +313,14 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
       T = Body{add(S.x, ax), Q{S.q.s + aq.s, add(S.q.v, aq.v)}, add(S.p, ap), add(S.l, al)};
       settle(T);
     }
-    // normalize_rotation: q * (1 / sqrt(s s + v . v))
+    // normalize_rotation: q * (1 / sqrt(s s + v . v)).  A step is odd where that is out of the short forms'
+    // range (the test is theirs): every step whose new rotation is NaN is, and so every one whose old was.
+    bool odd;
     {
+      const float n2 = T.q.s * T.q.s + dot(T.q.v, T.q.v);
+      odd = !(n2 >= 0x1p-96f && n2 <= 0x1p96f);
       float root, inv;
-      sqrt_rcp_rn(T.q.s * T.q.s + dot(T.q.v, T.q.v), root, inv);
+      sqrt_rcp_rn(n2, root, inv);
       T.q = Q{T.q.s * inv, f3{T.q.v.x * inv, T.q.v.y * inv, T.q.v.z * inv}};
     }
     // update_state: the cube's vertices against the obstacles
@@ -328,9 +343,10 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
           near = (near | near >> 8) & 0xffu;
         }
       }
+      if (odd) near = 0xffu;  // the sides of a NaN's corners say nothing
       if (near != 0) {
         const Corners Co = keep.get_corners(was), Cn = keep.get_corners(is);
-        const f3 x_old = at_plus_zero(S.x), x_new = at_plus_zero(T.x);
+        const f3 x_new = T.x;
         // what the response needs of the old pose: once for the few-face scenes, whose marked corners mostly
         // hit, and per hit with the grids, where the search needs the registers
         M3 I_old;
@@ -342,7 +358,14 @@ __global__ void __launch_bounds__(kBlock) rigid_step_kernel(float* __restrict__ 
         while (near != 0) {
           const uint32_t k = (uint32_t)__builtin_ctz(near);
           near &= near - 1u;
-          const f3 op = corner_of_lane(Co, x_old, k), np = corner_of_lane(Cn, x_new, k);
+          f3 op, np;
+          if (__builtin_expect(odd, 0)) {
+            op = corner_as_written(S.q, S.x, k);
+            np = corner_as_written(T.q, x_new, k);
+          } else {
+            op = corner_of_lane(Co, at_plus_zero(S.x), k);
+            np = corner_of_lane(Cn, at_plus_zero(x_new), k);
+          }
           f3 nrm, v0;
           if (!hit_face<GRID>(O, op, np, P.dt_d, nrm, v0)) continue;
           if (GRID) keep.get_pose(I_old, w, vel);
